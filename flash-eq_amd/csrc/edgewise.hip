@@ -455,6 +455,8 @@ extern "C" int feq_edgewise_fwd(const feq_layout* L, const feq_binning* b, int32
         const int rc = ew_split_fwd(*L, *b, rank, E, x, nullptr, 0, P, Q, dist, C, F, y, ws,
                                     ws_bytes, false, stream_of(stream));
         if (rc != -1) return rc;
+        const int rw = ew_wave_fwd(*L, *b, rank, E, x, P, Q, dist, C, F, y, stream_of(stream));
+        if (rw != -1) return rw;
     }
     const size_t clds = c_lds(*L, rank, fwd_lds(*L, rank)), lds = fwd_lds(*L, rank) + clds;
     const int nt = pick_threads(lds);
@@ -499,15 +501,20 @@ extern "C" int feq_edgewise_bwd(const feq_layout* L, const feq_binning* b, int32
     const int kw = rank * L->wdim;
     if (!ew_tail_supported(*b, kw))
         return fail(FEQ_ERR_UNSUPPORTED, "empty radial-function rows");
+    const bool wave = path == kPathSplit && !gP && !gQ && gx && ew_wave_supported(*L, rank);
     const size_t clds = c_lds(*L, rank, bwd_lds(*L, rank)), lds = bwd_lds(*L, rank) + clds;
     const int nt = pick_threads(lds);
     auto kern = clds ? (nt == 256 ? k_ew_bwd<256, true> : nt == 512 ? k_ew_bwd<512, true> : k_ew_bwd<1024, true>)
                      : (nt == 256 ? k_ew_bwd<256, false> : nt == 512 ? k_ew_bwd<512, false> : k_ew_bwd<1024, false>);
-    if (int rc = ensure_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
+    if (int rc = wave ? FEQ_OK : ensure_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
     const int G = groups_for(E);
     float* part = static_cast<float*>(ws);
     float* dFe = part + align_up(static_cast<size_t>(G) * ncc, 64);
     float* tail = dFe + align_up(static_cast<size_t>(E) * kw, 64);
+    if (wave) {
+        if (int rc = ew_wave_bwd(*L, *b, rank, E, gy, x, P, Q, dist, C, F, gx, dFe, part, s)) return rc;
+        return ew_tail(*L, *b, rank, E, dist, F, dFe, part, ew_wave_groups(*L, E), ncc, gC, gF, gdist, tail, s);
+    }
     EwDims D{rank, b->num_bins};
     FEQ_LAUNCH("k_ew_bwd", kern, dim3(G), dim3(nt), lds, s, *L, *b, D, E, gy, x, P, Q, dist,
                        C, F, gx, dFe, gdist, gP, gQ, part);

@@ -201,8 +201,19 @@ int ew0_bwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, cons
             float* gdist, const NodeScatter* ns, void* ws, size_t ws_bytes, hipStream_t s,
             const float* ym = nullptr, float* gP = nullptr, float* gQ = nullptr);
 
+// Wave-per-edge family on the float32 matrix cores (edgewise_wave.hip): layouts
+// without split kernels; -1 when it does not cover the shape.  The backward
+// writes dF_e and ew_wave_groups(L, E) partials of dC for ew_tail.
+bool ew_wave_supported(const feq_layout& L, int rank);
+int ew_wave_groups(const feq_layout& L, int64_t E);
+int ew_wave_fwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, const float* x, const float* P,
+                const float* Q, const float* dist, const float* C, const float* F, float* y, hipStream_t s);
+int ew_wave_bwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, const float* gy, const float* x,
+                const float* P, const float* Q, const float* dist, const float* C, const float* F, float* gx,
+                float* dFe, float* dC_part, hipStream_t s);
+
 // Kernel family of the fused edgewise layer.  The default tries the split-fp16
-// kernels, then the shape-generic ones; FEQ_EW_PATH=generic (or
+// kernels, then the wave-per-edge ones, then the shape-generic ones; FEQ_EW_PATH=generic (or
 // FEQ_FORCE_GENERIC=1) uses only the generic ones, so tests can check the
 // implementations against each other.
 enum { kPathSplit = 0, kPathGeneric = 2 };
