@@ -16,6 +16,8 @@
 // Distance gradient: one workgroup per edge, a fixed-order workgroup sum.
 #include "feq_internal.h"
 
+#include <type_traits>
+
 namespace feq {
 namespace {
 
@@ -387,12 +389,32 @@ size_t table_lds(const feq_layout& L, int ob, int ib) {
 
 size_t bin_ws_bytes(const feq_binning& b, int64_t E) {
     return align_up(sizeof(int64_t) * E, 256) + align_up(sizeof(int32_t) * E, 256) +
-           align_up(sizeof(int32_t) * (b.num_bins + 1), 256) + feq_csr_workspace(E, b.num_bins) + 256;
+           align_up(sizeof(int32_t) * (b.num_bins + 1), 256) + align_up(feq_csr_workspace(E, b.num_bins), 256) + 256;
+}
+
+// The edges grouped by lower bin (bin_ws_bytes of workspace).
+template <class T>
+int bin_csr(const feq_binning& b, int64_t E, const T* dist, Carver& cv, int32_t** perm, int32_t** offsets,
+            feq_stream_t stream) {
+    int64_t* lo = cv.take<int64_t>(E);
+    *perm = cv.take<int32_t>(E);
+    *offsets = cv.take<int32_t>(b.num_bins + 1);
+    void* csr_ws = cv.take<char>(feq_csr_workspace(E, b.num_bins));
+    auto kb = k_bd_bins<T>;
+    FEQ_LAUNCH("k_bd_bins", kb, dim3(ceil_div(E, 256)), dim3(256), 0, stream_of(stream), b, E, dist, lo);
+    return feq_csr_by_dst(lo, E, b.num_bins, *perm, *offsets, csr_ws, feq_csr_workspace(E, b.num_bins), stream);
+}
+
+// Whether the matrix-product form (float32) runs: its sizes and the workspace.
+template <class T>
+bool use_bdm(const feq_layout& L, const feq_binning& b, int64_t E, const void* ws, size_t ws_bytes) {
+    return std::is_same_v<T, float> && ws && bdm_supported(L, b, E) &&
+           ws_bytes >= bin_ws_bytes(b, E) + bdm_workspace(L, b, E);
 }
 
 template <class T>
 int blockdiag_fwd(const feq_layout* L, const feq_binning* b, int64_t E, const T* x, const T* table,
-                  const T* dist, T* y, feq_stream_t stream) {
+                  const T* dist, T* y, void* ws, size_t ws_bytes, feq_stream_t stream) {
     if (int rc = check_layout(L)) return rc;
     if (int rc = check_binning(b)) return rc;
     if (E < 0) return fail(FEQ_ERR_INVALID, "negative edge count");
@@ -401,6 +423,15 @@ int blockdiag_fwd(const feq_layout* L, const feq_binning* b, int64_t E, const T*
     if (E > 0x7fffffffLL) return fail(FEQ_ERR_UNSUPPORTED, "more than 2^31-1 edges");
     const size_t lds = sizeof(T) * L->cin * L->din;
     if (lds > 64 * 1024) return fail(FEQ_ERR_UNSUPPORTED, "Cin*Din too large for this kernel");
+    if constexpr (std::is_same_v<T, float>) {
+        if (use_bdm<T>(*L, *b, E, ws, ws_bytes)) {
+            Carver cv(ws);
+            int32_t *perm, *offsets;
+            if (int rc = bin_csr<T>(*b, E, dist, cv, &perm, &offsets, stream)) return rc;
+            return bdm_fwd(*L, *b, E, x, table, dist, perm, y, static_cast<char*>(ws) + bin_ws_bytes(*b, E),
+                           stream_of(stream));
+        }
+    }
     auto k = k_bd_fwd<T>;
     FEQ_LAUNCH("k_bd_fwd", k, dim3(E), dim3(kThreads), lds, stream_of(stream), *L, *b, x, table,
                dist, y);
@@ -434,24 +465,26 @@ int blockdiag_bwd(const feq_layout* L, const feq_binning* b, int64_t E, const T*
     table_slices(*L, sizeof(T), ob, ib);
     const size_t lds_t = table_lds<T>(*L, ob, ib);
     if (lds_t > 64 * 1024) return fail(FEQ_ERR_UNSUPPORTED, "representation too large for this kernel");
-    // the edges grouped by lower bin
     Carver cv(ws);
-    int64_t* lo = cv.take<int64_t>(E);
-    int32_t* perm = cv.take<int32_t>(E);
-    int32_t* offsets = cv.take<int32_t>(b->num_bins + 1);
-    void* csr_ws = cv.take<char>(feq_csr_workspace(E, b->num_bins));
-    auto kb = k_bd_bins<T>;
-    FEQ_LAUNCH("k_bd_bins", kb, dim3(ceil_div(E, 256)), dim3(256), 0, s, *b, E, dist, lo);
-    if (int rc = feq_csr_by_dst(lo, E, b->num_bins, perm, offsets, csr_ws,
-                                feq_csr_workspace(E, b->num_bins), stream))
-        return rc;
+    int32_t *perm, *offsets;
+    if (int rc = bin_csr<T>(*b, E, dist, cv, &perm, &offsets, stream)) return rc;
+    bool mm = false, dr_done = false;
+    if constexpr (std::is_same_v<T, float>) {
+        mm = use_bdm<T>(*L, *b, E, ws, ws_bytes);
+        if (mm)
+            if (int rc = bdm_bwd(*L, *b, E, gy, x, table, dist, perm, offsets, gx, gtable, gdist, &dr_done,
+                                 static_cast<char*>(ws) + bin_ws_bytes(*b, E), s))
+                return rc;
+    }
+    if (!mm) {
     auto kx = k_bd_bwd_x<T>;
     FEQ_LAUNCH("k_bd_bwd_x", kx, dim3(E), dim3(kThreads), lds_x, s, *L, *b, gy, table, dist, gx);
     const int nslices = static_cast<int>(ceil_div(L->cout, ob) * ceil_div(L->cin, ib));
     auto kt = k_bd_bwd_table<T>;
     FEQ_LAUNCH("k_bd_bwd_table", kt, dim3(b->num_bins + 1, nslices), dim3(kThreads), lds_t, s, *L,
                *b, E, gy, x, dist, perm, offsets, ob, ib, gtable);
-    if (gdist) {
+    }
+    if (gdist && !dr_done) {
         auto kr = k_bd_bwd_r<T>;
         FEQ_LAUNCH("k_bd_bwd_r", kr, dim3(E), dim3(kThreads), lds_r, s, *L, *b, gy, x, table, dist,
                    gdist);
@@ -480,13 +513,13 @@ using namespace feq;
 
 extern "C" size_t feq_blockdiag_workspace(const feq_layout* L, const feq_binning* b, int64_t E) {
     if (!L || !b || E <= 0) return 0;
-    return bin_ws_bytes(*b, E);
+    return bin_ws_bytes(*b, E) + (bdm_supported(*L, *b, E) ? bdm_workspace(*L, *b, E) : 0);
 }
 
 extern "C" int feq_blockdiag_fwd(const feq_layout* L, const feq_binning* b, int64_t E,
                                  const float* x, const float* table, const float* dist, float* y,
-                                 void*, size_t, feq_stream_t stream) {
-    return blockdiag_fwd<float>(L, b, E, x, table, dist, y, stream);
+                                 void* ws, size_t ws_bytes, feq_stream_t stream) {
+    return blockdiag_fwd<float>(L, b, E, x, table, dist, y, ws, ws_bytes, stream);
 }
 
 extern "C" int feq_blockdiag_bwd(const feq_layout* L, const feq_binning* b, int64_t E,
@@ -499,7 +532,7 @@ extern "C" int feq_blockdiag_bwd(const feq_layout* L, const feq_binning* b, int6
 extern "C" int feq_blockdiag_fwd_f64(const feq_layout* L, const feq_binning* b, int64_t E,
                                      const double* x, const double* table, const double* dist,
                                      double* y, feq_stream_t stream) {
-    return blockdiag_fwd<double>(L, b, E, x, table, dist, y, stream);
+    return blockdiag_fwd<double>(L, b, E, x, table, dist, y, nullptr, 0, stream);
 }
 
 extern "C" int feq_blockdiag_bwd_f64(const feq_layout* L, const feq_binning* b, int64_t E,

@@ -1,0 +1,619 @@
+// The generic block-diagonal op in float32 as matrix products
+// (v_mfma_f32_16x16x4_f32) over edges grouped by their lower bin.
+//
+// blockdiag.hip's per-edge kernels read both table rows of the bin for every
+// edge (2 Cout Cin Wdim values: 156 KB at lvals 0..2 x 32), so the L2 bounds
+// them.  Here a workgroup takes 16 edges in the order of their bins (the stable
+// CSR by bin), one 16-channel tile of outputs, and reads each table row once for
+// the 16:
+//   forward   Y[co, e] (o)  += T_w[co, ci] X[ci, e] (i) + D_w[co, ci] (t_e X[ci, e] (i))
+//   gradient  GX[ci, e] (i) += T_w[co, ci]^T G[co, e] (o) + t_e D_w^T G
+//   table     dT_w[co, ci]  += sum over e of G[co, e] (o) X[ci, e] (i)
+// with X = s^l x, G = s^l gy, T the bin's row and D the next row's difference to
+// it: T + t D is the well-conditioned form where linear bins extrapolate
+// (|t| >> 1), as in the per-edge kernels.  The table is first packed into operand
+// order (k_bdm_pack), T and D side by side, zero-padded to 16 channels.
+//
+// Lane l = (c = l % 16, g = l / 16); a reduction step r takes the indices
+// 4 r + g: the staged rows [slot][channel][edge] (257 floats from slot to slot)
+// are then read as 64 consecutive floats.  The four waves of a workgroup share
+// the staged rows and split the (m, output) pairs.  Sums run in a fixed order.
+//
+// Lvals 0..2 x 32, 20 000 edges, 65 table rows, the per-edge kernels and these:
+// forward 1163 us, now 94 + 15 (pack) + 35 (sort by bin); input and distance
+// gradients 816 + 1724, now 154 + 17 (pack); table gradient 2256, now 232 + 10.
+// The matrix steps alone would take 20 to 40 us each: the staging of 16 edges'
+// rows, one memory latency per 16 channels, bounds these.
+#include "feq_internal.h"
+
+namespace feq {
+namespace {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+constexpr int kThreads = 256;
+constexpr int kSS = 257;        // floats from slot to slot of the staged rows
+constexpr int kMaxSlots = 63;   // staged slots (64 KB of LDS)
+constexpr int kMaxPairs = 64;
+constexpr int kMaxUnits = 160;
+
+// A pair: the z components of one index of an m-block, and the block's other side.
+struct Pair {
+    int8_t slot;     // first slot of the produced side
+    int8_t other;    // first slot of the summed side
+    int8_t n;        // indices summed over
+    int8_t z;        // 1 or 2 components
+    int16_t w;       // weight of the first summed index
+    int16_t step;    // weights from one summed index to the next
+};
+struct Pairs {
+    int32_t n;
+    Pair p[kMaxPairs];
+};
+// A unit of the table gradient: the z weights of one (o, i) of an m-block.
+struct Unit {
+    int8_t o, i, z, pad;
+    int16_t w;
+};
+struct Units {
+    int32_t n;
+    Unit u[kMaxUnits];
+};
+
+__device__ __forceinline__ v4f mfma4(float a, float b, v4f c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Edge of a sorted position, with its bin state.
+struct EdgeRow {
+    int64_t e;
+    int lo;
+    float t, s, dtdr, r;
+};
+__device__ __forceinline__ EdgeRow edge_row(const feq_binning& B, const int32_t* __restrict__ perm,
+                                            const float* __restrict__ dist, int64_t pos, int64_t E) {
+    EdgeRow R;
+    R.e = perm[pos < E ? pos : E - 1];
+    R.r = dist[R.e];
+    const EdgeBin eb = edge_bin(R.r, B);
+    R.lo = eb.lo;
+    R.t = eb.t;
+    R.dtdr = eb.dtdr;
+    R.s = R.r / (R.r + B.sh_scale);
+    return R;
+}
+
+// Rows c0 .. c0 + 15 of (E, nch, dim) of the 16 edges at e[], times scale[edge][l],
+// and weight[edge], to st[slot][channel][edge] (EDGE_MINOR) or st[slot][edge][channel]; zeros for
+// channels outside and for edges from n on.
+template <bool EDGE_MINOR>
+__device__ __forceinline__ void stage_rows(const float* __restrict__ x, int nch, int c0, int dim, const int64_t* e,
+                                           const float* scale, int sstride, const int8_t* deg, int n, float* st,
+                                           const float* weight = nullptr) {
+    const int per = 16 * dim;
+    for (int q0 = threadIdx.x; q0 < 16 * per; q0 += 4 * kThreads) {
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int q = q0 + u * kThreads, ed = q / per, rest = q - ed * per, ch = rest / dim;
+            const bool ok = q < 16 * per && ed < n && c0 + ch < nch;
+            v[u] = x[ok ? (e[ed & 15] * nch + c0) * dim + rest : 0];
+            v[u] = ok ? v[u] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int q = q0 + u * kThreads, ed = q / per, rest = q - ed * per, ch = rest / dim, d = rest - ch * dim;
+            if (q < 16 * per) {
+                float sc = scale[ed * sstride + deg[d]];
+                if (weight) sc *= weight[ed];
+                st[d * kSS + (EDGE_MINOR ? ch * 16 + ed : ed * 16 + ch)] = v[u] * sc;
+            }
+        }
+    }
+}
+
+constexpr int kPow = 32;        // powers of s kept per edge (+ 1: no bank conflicts)
+
+// Operand order of the table: fragment (b, w, row tile, reduction tile) holds for
+// lane (c, g) the four values r of T, then of D: T[co, ci] with, forward, co = 16
+// row + c and ci = 16 red + 4 r + g, and transposed (TR) with ci = 16 row + c and
+// co = 16 red + 4 r + g.  A workgroup packs the 16 x 16 channels of one bin.
+template <bool TR>
+__global__ void __launch_bounds__(kThreads)
+k_bdm_pack(const float* __restrict__ table, int cout, int cin, int wd, int wchunk, float* __restrict__ frag) {
+    extern __shared__ float sm[];   // [2][16 * 16][wchunk + 1]
+    const int64_t b = blockIdx.x;
+    const int nci = (cin + 15) / 16, nco = (cout + 15) / 16;
+    const int cot = blockIdx.y / nci, cit = blockIdx.y % nci;
+    const int row = TR ? cit : cot, red = TR ? cot : cit, nrow = TR ? nci : nco, nred = TR ? nco : nci;
+    const int64_t ts = static_cast<int64_t>(cout) * cin * wd;
+    for (int w0 = 0; w0 < wd; w0 += wchunk) {
+        const int nw = wd - w0 < wchunk ? wd - w0 : wchunk, ls = wchunk + 1;
+        __syncthreads();
+        for (int q = threadIdx.x; q < 256 * nw; q += kThreads) {
+            const int ch = q / nw, w = q - ch * nw, co = 16 * cot + ch / 16, ci = 16 * cit + ch % 16;
+            const bool ok = co < cout && ci < cin;
+            const int64_t at = ok ? b * ts + (static_cast<int64_t>(co) * cin + ci) * wd + w0 + w : 0;
+            const float lo = table[at], hi = table[ok ? at + ts : 0];
+            sm[ch * ls + w] = ok ? lo : 0.0f;
+            sm[(256 + ch) * ls + w] = ok ? hi - lo : 0.0f;
+        }
+        __syncthreads();
+        for (int q = threadIdx.x; q < 512 * nw; q += kThreads) {
+            const int w = q / 512, k = q - w * 512, d = k >> 8, l = (k & 255) >> 2, r = k & 3;
+            const int a = l & 15, z = 4 * r + (l >> 4);       // row and reduction channel
+            const int ch = TR ? z * 16 + a : a * 16 + z;
+            frag[((((b * wd + w0 + w) * nrow + row) * nred + red) * 2 + d) * 256 + l * 4 + r] = sm[(256 * d + ch) * ls + w];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// A tile's product for up to MAXP pairs per wave: acc[p] += T S + D (t S), or with
+// GD acc[p] += T S, accD[p] += D S, accS[p] += T (l S) + D (t l S) (S: the staged
+// rows, l: the degree of the summed slot; the distance gradient's three sums).
+template <int MAXP, bool GD>
+struct TileAcc {
+    v4f a[MAXP][2];
+    v4f d[GD ? MAXP : 1][2];
+    v4f s[GD ? MAXP : 1][2];
+};
+
+// SIGN: +1 forward (re += a re + b im, im += a im - b re), -1 transposed
+// (re += a re - b im, im += a im + b re).
+template <int MAXP, bool GD, int SIGN>
+__device__ __forceinline__ void tile_product(const Pairs& PT, int wave, const float* __restrict__ frag, int64_t bin, int wd,
+                                             int nrow, int row, int nred, int red, const float* st, float mask, float t,
+                                             const int8_t* deg, TileAcc<MAXP, GD>& A) {
+    const int lane = threadIdx.x & 63;
+    const int64_t wstride = static_cast<int64_t>(nrow) * nred * 512;
+    const float* f0 = frag + ((bin * wd * nrow + row) * nred + red) * 512;
+#pragma unroll
+    for (int p = 0; p < MAXP; ++p) {
+        if (wave + 4 * p >= PT.n) break;
+        const Pair P = PT.p[wave + 4 * p];
+        for (int k = 0; k < P.n; ++k) {
+            const float* fa = f0 + (P.w + k * P.step) * wstride;
+            const float* sr = st + (P.other + P.z * k) * kSS;
+            v4f T[2], D[2], S[2];
+            T[0] = *reinterpret_cast<const v4f*>(fa + 4 * lane);
+            D[0] = *reinterpret_cast<const v4f*>(fa + 256 + 4 * lane);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[0][r] = sr[64 * r + lane] * mask;
+            const float l = GD ? static_cast<float>(deg[P.other + P.z * k]) : 0.0f;
+            if (P.z == 2) {
+                T[1] = *reinterpret_cast<const v4f*>(fa + wstride + 4 * lane);
+                D[1] = *reinterpret_cast<const v4f*>(fa + wstride + 256 + 4 * lane);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) S[1][r] = sr[kSS + 64 * r + lane] * mask;
+            }
+            // component c of the products with the (a, b) fragments Q and the rows R
+            auto add = [&](const v4f (&Q)[2], const v4f (&R)[2], v4f (&acc)[2]) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[0] = mfma4(Q[0][r], R[0][r], acc[0]);
+                if (P.z == 2) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        acc[1] = mfma4(Q[0][r], R[1][r], acc[1]);
+                        acc[0] = mfma4(Q[1][r], SIGN > 0 ? R[1][r] : -R[1][r], acc[0]);
+                        acc[1] = mfma4(Q[1][r], SIGN > 0 ? -R[0][r] : R[0][r], acc[1]);
+                    }
+                }
+            };
+            auto times = [&](float q) {
+                struct { v4f v[2]; } R;
+#pragma unroll
+                for (int z = 0; z < 2; ++z)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) R.v[z][r] = S[z][r] * q;
+                return R;
+            };
+            add(T, S, A.a[p]);
+            if constexpr (GD) {
+                add(D, S, A.d[p]);
+                if (l != 0.0f) {
+                    const auto L0 = times(l), L1 = times(l * t);
+                    add(T, L0.v, A.s[p]);
+                    add(D, L1.v, A.s[p]);
+                }
+            } else {
+                const auto S1 = times(t);
+                add(D, S1.v, A.a[p]);
+            }
+        }
+    }
+}
+
+template <int MAXP, bool GD>
+__device__ __forceinline__ void clear(TileAcc<MAXP, GD>& A) {
+#pragma unroll
+    for (int p = 0; p < MAXP; ++p)
+#pragma unroll
+        for (int z = 0; z < 2; ++z) A.a[p][z] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (GD)
+#pragma unroll
+        for (int p = 0; p < MAXP; ++p)
+#pragma unroll
+            for (int z = 0; z < 2; ++z) A.d[p][z] = A.s[p][z] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+}
+
+// Workgroup (tile of 16 sorted positions, 16-channel tile of outputs); x: the
+// summed side (E, nch, din) scaled by s^l, y: the produced side (E, noch, dout).
+// GD: the distance gradient's share of this channel tile to gpart[tile of
+// channels][position's edge], from xo, the features on the produced side.
+template <int MAXP, bool GD, int SIGN>
+__global__ void __launch_bounds__(kThreads, 2)
+k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __restrict__ perm,
+            const float* __restrict__ dist, const float* __restrict__ x, int nch, int din, int noch, int dout, int wd,
+            const float* __restrict__ frag, const float* __restrict__ xo, float* __restrict__ y,
+            float* __restrict__ gpart) {
+    extern __shared__ float st[];
+    __shared__ float sPow[16 * (kPow + 1)];
+    __shared__ int64_t sE[16];
+    __shared__ int sLo[16];
+    __shared__ float sRed[4 * 64];
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t p0 = static_cast<int64_t>(blockIdx.x) * 16;
+    const int n = static_cast<int>(E - p0 < 16 ? E - p0 : 16);
+    const int8_t* din_deg = SIGN > 0 ? L.lslot_in : L.lslot_out;
+    const int8_t* dout_deg = SIGN > 0 ? L.lslot_out : L.lslot_in;
+    const EdgeRow R = edge_row(B, perm, dist, p0 + (c < n ? c : n - 1), E);
+    if (threadIdx.x < 16) {
+        sE[c] = R.e;
+        sLo[c] = R.lo;
+        float p = 1.0f;
+        for (int l = 0; l < kPow; ++l) {
+            sPow[c * (kPow + 1) + l] = p;
+            p *= R.s;
+        }
+    }
+    __syncthreads();
+    const int row = blockIdx.y, nrow = gridDim.y, nred = (nch + 15) / 16;
+    TileAcc<MAXP, GD> A;
+    clear(A);
+    for (int red = 0; red < nred; ++red) {
+        __syncthreads();
+        stage_rows<true>(x, nch, 16 * red, din, sE, sPow, kPow + 1, din_deg, n, st);
+        __syncthreads();
+        for (int p = 0; p < n;) {       // the tile's bins, in order
+            const int bin = sLo[p];
+            tile_product<MAXP, GD, SIGN>(PT, wave, frag, bin, wd, nrow, row, nred, red, st,
+                                         R.lo == bin ? 1.0f : 0.0f, R.t, din_deg, A);
+            while (p < n && sLo[p] == bin) ++p;
+        }
+    }
+    if constexpr (GD) {
+        // x on the produced side: sum of x accD, and of l x (accT + t accD) + x accS
+        __syncthreads();
+        stage_rows<true>(xo, noch, 16 * row, dout, sE, sPow, kPow + 1, dout_deg, n, st);
+        __syncthreads();
+        float at = 0.0f, as = 0.0f;
+#pragma unroll
+        for (int p = 0; p < MAXP; ++p) {
+            if (wave + 4 * p >= PT.n) break;
+            const Pair P = PT.p[wave + 4 * p];
+            const float l = static_cast<float>(dout_deg[P.slot]);
+            for (int z = 0; z < P.z; ++z) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float q = st[(P.slot + z) * kSS + (4 * g + r) * 16 + c];
+                    const v4f a = z ? A.a[p][1] : A.a[p][0], d = z ? A.d[p][1] : A.d[p][0], s = z ? A.s[p][1] : A.s[p][0];
+                    at += q * d[r];
+                    as += q * (l * (a[r] + R.t * d[r]) + s[r]);
+                }
+            }
+        }
+        float v = at * R.dtdr;
+        if (L.has_lpos) v += as * (B.sh_scale / (R.r * (R.r + B.sh_scale)));
+        sRed[threadIdx.x] = v;
+        __syncthreads();
+        if (threadIdx.x < n) {
+            float sum = 0.0f;
+            for (int k = 0; k < 16; ++k) sum += sRed[16 * k + threadIdx.x];
+            gpart[static_cast<int64_t>(row) * E + sE[threadIdx.x]] = sum;
+        }
+    }
+    // the produced rows through LDS, so that they leave in whole runs
+    __syncthreads();
+    for (int q = threadIdx.x; q < dout * kSS; q += kThreads) st[q] = 0.0f;    // slots that no weight reaches
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < MAXP; ++p) {
+        if (wave + 4 * p >= PT.n) break;
+        const Pair P = PT.p[wave + 4 * p];
+        const float sc = sPow[c * (kPow + 1) + dout_deg[P.slot]];
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+            if (z < P.z) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float v = A.a[p][z][r];
+                    if constexpr (GD) v += R.t * A.d[p][z][r];
+                    st[(P.slot + z) * kSS + (4 * g + r) * 16 + c] = v * sc;
+                }
+            }
+    }
+    __syncthreads();
+    const int per = 16 * dout;
+    for (int q = threadIdx.x; q < n * per; q += kThreads) {
+        const int ed = q / per, rest = q - ed * per, ch = rest / dout, d = rest - ch * dout;
+        if (16 * row + ch < noch) y[(sE[ed] * noch + 16 * row) * dout + rest] = st[d * kSS + ch * 16 + ed];
+    }
+}
+
+// gdist[e] = the channel tiles' shares in order.
+__global__ void k_bdm_dr(const float* __restrict__ part, int n, int64_t E, float* __restrict__ gdist) {
+    const int64_t e = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+    if (e >= E) return;
+    float v = part[e];
+    for (int k = 1; k < n; ++k) v += part[k * E + e];
+    gdist[e] = v;
+}
+
+// ---------------------------------------------------------------------------
+// Workgroup (table row b, co and ci tile, chunk of 4 kMaxU units and a split of the
+// row's edges): the edges of bin b (weight 1 - t) and of bin b - 1 (weight t) in
+// sorted order, 16 at a time, their indices, bins and powers 64 at a time (one
+// memory latency for four tiles).  Few table rows leave the chip idle (65 rows
+// and 4 tiles: 260 workgroups, 577 us, 232 with eight splits), so the edges
+// are then split and the splits' sums added in order (k_bdm_sum).
+constexpr int kMaxU = 8;
+constexpr int kHead = 64;
+
+__global__ void __launch_bounds__(kThreads, 2)
+k_bdm_table(feq_layout L, Units UT, feq_binning B, int64_t E, const int32_t* __restrict__ perm,
+            const int32_t* __restrict__ offsets, const float* __restrict__ dist, const float* __restrict__ gy,
+            const float* __restrict__ x, int splits, float* __restrict__ gtable) {
+    extern __shared__ float st[];       // gy rows, then x rows
+    __shared__ float sPow[kHead * (kPow + 1)];
+    __shared__ int64_t sE[kHead];
+    __shared__ float sW[kHead];
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cin = L.cin, cout = L.cout, din = L.din, dout = L.dout, wd = L.wdim, nb = B.num_bins;
+    const int b = blockIdx.x, nci = (cin + 15) / 16, cot = blockIdx.y / nci, cit = blockIdx.y % nci;
+    const int split = blockIdx.z % splits;
+    const int u0 = (blockIdx.z / splits) * 4 * kMaxU + wave;
+    float* sg = st;
+    float* sx = st + dout * kSS;
+    v4f acc[kMaxU][2];
+#pragma unroll
+    for (int u = 0; u < kMaxU; ++u) acc[u][0] = acc[u][1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    const int a0 = b < nb ? offsets[b] : 0, n_lo = b < nb ? offsets[b + 1] - a0 : 0;
+    const int h0 = b > 0 ? offsets[b - 1] : 0, n_all = n_lo + (b > 0 ? offsets[b] - h0 : 0);
+    const int per = ((n_all + splits - 1) / splits + 15) / 16 * 16;
+    const int end = per * (split + 1) < n_all ? per * (split + 1) : n_all;
+    for (int base = per * split, head = 0; base < end; base += 16, head = (head + 16) % kHead) {
+        const int n = end - base < 16 ? end - base : 16;
+        __syncthreads();
+        if (head == 0) {
+            if (threadIdx.x < kHead) {
+                const int pos = base + lane < end ? base + lane : end - 1;
+                const EdgeRow R = edge_row(B, perm, dist, pos < n_lo ? a0 + pos : h0 + pos - n_lo, E);
+                sE[lane] = R.e;
+                sW[lane] = pos < n_lo ? 1.0f - R.t : R.t;
+                float p = 1.0f;
+                for (int l = 0; l < kPow; ++l) {
+                    sPow[lane * (kPow + 1) + l] = p;
+                    p *= R.s;
+                }
+            }
+            __syncthreads();
+        }
+        stage_rows<false>(gy, cout, 16 * cot, dout, sE + head, sPow + head * (kPow + 1), kPow + 1, L.lslot_out, n, sg,
+                          sW + head);
+        stage_rows<false>(x, cin, 16 * cit, din, sE + head, sPow + head * (kPow + 1), kPow + 1, L.lslot_in, n, sx);
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < kMaxU; ++u) {
+            if (u0 + 4 * u >= UT.n) break;
+            const Unit U = UT.u[u0 + 4 * u];
+            const float* ga = sg + U.o * kSS;
+            const float* xa = sx + U.i * kSS;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float gr = ga[64 * r + lane], fr = xa[64 * r + lane];
+                acc[u][0] = mfma4(gr, fr, acc[u][0]);
+                if (U.z == 2) {     // a: fr gr + fi gi, b: fi gr - fr gi
+                    const float gi = ga[kSS + 64 * r + lane], fi = xa[kSS + 64 * r + lane];
+                    acc[u][0] = mfma4(gi, fi, acc[u][0]);
+                    acc[u][1] = mfma4(gr, fi, acc[u][1]);
+                    acc[u][1] = mfma4(gi, -fr, acc[u][1]);
+                }
+            }
+        }
+    }
+    const int ci = 16 * cit + c;
+#pragma unroll
+    for (int u = 0; u < kMaxU; ++u) {
+        if (u0 + 4 * u >= UT.n) break;
+        const Unit U = UT.u[u0 + 4 * u];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int co = 16 * cot + 4 * g + r;
+            if (co < cout && ci < cin) {
+                float* o = gtable + (((static_cast<int64_t>(split) * (nb + 1) + b) * cout + co) * cin + ci) * wd + U.w;
+                o[0] = acc[u][0][r];
+                if (U.z == 2) o[1] = acc[u][1][r];
+            }
+        }
+    }
+}
+
+// out[q] = the splits' sums in order.
+__global__ void __launch_bounds__(kThreads)
+k_bdm_sum(const float* __restrict__ part, int splits, int64_t n, float* __restrict__ out) {
+    const int64_t q = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x;
+    if (q >= n) return;
+    float v = part[q];
+    for (int k = 1; k < splits; ++k) v += part[k * n + q];
+    out[q] = v;
+}
+
+// ---------------------------------------------------------------------------
+// The pairs of the produced side, the costliest first so that the waves' shares
+// are even; false when there are more than kMaxPairs.
+bool build_pairs(const feq_layout& L, bool transposed, Pairs& T) {
+    T.n = 0;
+    for (int k = 0; k < L.nblocks; ++k) {
+        const int z = L.blk[k][0] ? 2 : 1, ni = L.blk[k][1], no = L.blk[k][2];
+        for (int a = 0; a < (transposed ? ni : no); ++a) {
+            if (T.n == kMaxPairs) return false;
+            Pair& p = T.p[T.n++];
+            p.z = static_cast<int8_t>(z);
+            p.n = static_cast<int8_t>(transposed ? no : ni);
+            p.slot = static_cast<int8_t>((transposed ? L.blk[k][3] : L.blk[k][4]) + z * a);
+            p.other = static_cast<int8_t>(transposed ? L.blk[k][4] : L.blk[k][3]);
+            p.w = static_cast<int16_t>(L.blk[k][5] + z * (transposed ? a : a * ni));
+            p.step = static_cast<int16_t>(transposed ? z * ni : z);
+        }
+    }
+    auto cost = [](const Pair& p) { return p.n * p.z * p.z; };
+    for (int a = 1; a < T.n; ++a)
+        for (int b = a; b > 0 && cost(T.p[b]) > cost(T.p[b - 1]); --b) {
+            const Pair t = T.p[b];
+            T.p[b] = T.p[b - 1], T.p[b - 1] = t;
+        }
+    return true;
+}
+
+bool build_units(const feq_layout& L, Units& T) {
+    T.n = 0;
+    for (int z = 2; z >= 1; --z)        // the two-weight units first, dealt evenly
+        for (int k = 0; k < L.nblocks; ++k) {
+            if ((L.blk[k][0] ? 2 : 1) != z) continue;
+            for (int o = 0; o < L.blk[k][2]; ++o)
+                for (int i = 0; i < L.blk[k][1]; ++i) {
+                    if (T.n == kMaxUnits) return false;
+                    T.u[T.n++] = Unit{static_cast<int8_t>(L.blk[k][4] + z * o), static_cast<int8_t>(L.blk[k][3] + z * i),
+                                      static_cast<int8_t>(z), 0,
+                                      static_cast<int16_t>(L.blk[k][5] + z * (o * L.blk[k][1] + i))};
+                }
+        }
+    return true;
+}
+
+int tiles16(int n) { return (n + 15) / 16; }
+constexpr int kPackLds = 48 * 1024;
+int pack_chunk(int wd) {
+    const int most = kPackLds / (512 * 4) - 1;
+    return wd < most ? wd : most;
+}
+size_t frag_floats(const feq_layout& L, const feq_binning& B) {
+    return static_cast<size_t>(B.num_bins) * L.wdim * tiles16(L.cin) * tiles16(L.cout) * 512;
+}
+constexpr int kMaxP = 8;        // pairs per wave; 4 with the distance gradient's sums
+
+template <bool TR>
+int pack(const feq_layout& L, const feq_binning& B, const float* table, float* frag, hipStream_t s) {
+    auto k = k_bdm_pack<TR>;
+    const int chunk = pack_chunk(L.wdim);
+    FEQ_LAUNCH("k_bdm_pack", k, dim3(B.num_bins, tiles16(L.cin) * tiles16(L.cout)), dim3(kThreads),
+               sizeof(float) * 512 * (chunk + 1), s, table, L.cout, L.cin, L.wdim, chunk, frag);
+    return FEQ_OK;
+}
+
+}  // namespace
+
+// Work (edges times table weights) from which on the products run.
+constexpr double kBdmMinWork = 2.5e7;
+
+// Where the products beat the per-edge kernels: their fixed cost (the sort by
+// bin and the packed table, about 80 us) against the per-edge kernels' 3 ps per
+// edge and table weight forward.
+bool bdm_supported(const feq_layout& L, const feq_binning& B, int64_t E) {
+    Pairs P;
+    Units U;
+    if (L.din > kMaxSlots || L.dout > kMaxSlots || L.wdim < 1 || B.num_bins < 1) return false;
+    for (int q = 0; q < L.din; ++q)
+        if (L.lslot_in[q] >= kPow) return false;
+    for (int q = 0; q < L.dout; ++q)
+        if (L.lslot_out[q] >= kPow) return false;
+    if (sizeof(float) * kSS * static_cast<size_t>(L.din + L.dout) > 128 * 1024) return false;
+    if (!build_pairs(L, false, P) || P.n > 4 * kMaxP || !build_pairs(L, true, P) || P.n > 4 * kMaxP) return false;
+    if (!build_units(L, U)) return false;
+    return static_cast<double>(E) * L.cin * L.cout * L.wdim >= kBdmMinWork;
+}
+
+namespace {
+size_t table_floats(const feq_layout& L, const feq_binning& B) {
+    return static_cast<size_t>(B.num_bins + 1) * L.cout * L.cin * L.wdim;
+}
+// Splits of a table row's edges: enough workgroups for eight per CU, at least 32
+// edges (of the 2 E / rows that a row has on average) each, at most eight.
+int table_splits(const feq_layout& L, const feq_binning& B, int64_t E, int units) {
+    const int64_t wgs = static_cast<int64_t>(B.num_bins + 1) * tiles16(L.cin) * tiles16(L.cout) * ceil_div(units, 4 * kMaxU);
+    int64_t n = ceil_div(2048, wgs);
+    const int64_t most = 2 * E / (B.num_bins + 1) / 32;
+    n = n < most ? n : most;
+    return static_cast<int>(n < 1 ? 1 : n > 8 ? 8 : n);
+}
+}  // namespace
+
+size_t bdm_workspace(const feq_layout& L, const feq_binning& B, int64_t E) {
+    Units U;
+    build_units(L, U);
+    const int splits = table_splits(L, B, E, U.n);
+    return sizeof(float) * (frag_floats(L, B) + 64 + static_cast<size_t>(E) * tiles16(L.cin) + 64 +
+                            (splits > 1 ? splits * table_floats(L, B) : 0));
+}
+
+static int bdm_lds(const void* fn, size_t bytes) {
+    if (bytes > 64 * 1024)
+        FEQ_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
+    return FEQ_OK;
+}
+
+int bdm_fwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* x, const float* table, const float* dist,
+            const int32_t* perm, float* y, void* ws, hipStream_t s) {
+    Pairs P;
+    build_pairs(L, false, P);
+    float* frag = static_cast<float*>(ws);
+    if (int rc = pack<false>(L, B, table, frag, s)) return rc;
+    auto k = P.n <= 16 ? k_bdm_apply<4, false, 1> : k_bdm_apply<kMaxP, false, 1>;
+    const size_t lds = sizeof(float) * kSS * (L.din > L.dout ? L.din : L.dout);
+    if (int rc = bdm_lds(reinterpret_cast<const void*>(k), lds)) return rc;
+    FEQ_LAUNCH("k_bdm_fwd", k, dim3(static_cast<unsigned>(ceil_div(E, 16)), tiles16(L.cout)), dim3(kThreads), lds, s, L,
+               P, B, E, perm, dist, x, L.cin, L.din, L.cout, L.dout, L.wdim, frag, static_cast<const float*>(nullptr), y,
+               static_cast<float*>(nullptr));
+    return FEQ_OK;
+}
+
+int bdm_bwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* gy, const float* x, const float* table,
+            const float* dist, const int32_t* perm, const int32_t* offsets, float* gx, float* gtable, float* gdist,
+            bool* dr_done, void* ws, hipStream_t s) {
+    Pairs P;
+    Units U;
+    build_pairs(L, true, P);
+    build_units(L, U);
+    float* frag = static_cast<float*>(ws);
+    float* gpart = frag + align_up(frag_floats(L, B), 64);
+    if (int rc = pack<true>(L, B, table, frag, s)) return rc;
+    // the distance gradient rides along where its sums fit the registers
+    const bool gd = gdist && P.n <= 16;
+    auto k = gd ? k_bdm_apply<4, true, -1> : P.n <= 16 ? k_bdm_apply<4, false, -1> : k_bdm_apply<kMaxP, false, -1>;
+    const size_t lds = sizeof(float) * kSS * (L.din > L.dout ? L.din : L.dout);
+    if (int rc = bdm_lds(reinterpret_cast<const void*>(k), lds)) return rc;
+    const int nt = tiles16(L.cin);
+    FEQ_LAUNCH("k_bdm_bwd_x", k, dim3(static_cast<unsigned>(ceil_div(E, 16)), nt), dim3(kThreads), lds, s, L, P, B, E,
+               perm, dist, gy, L.cout, L.dout, L.cin, L.din, L.wdim, frag, x, gx, gpart);
+    if (gd)
+        FEQ_LAUNCH("k_bdm_dr", k_bdm_dr, dim3(static_cast<unsigned>(ceil_div(E, 256))), dim3(256), 0, s, gpart, nt, E,
+                   gdist);
+    *dr_done = gd;
+    const size_t tlds = sizeof(float) * kSS * (L.din + L.dout);
+    if (int rc = bdm_lds(reinterpret_cast<const void*>(&k_bdm_table), tlds)) return rc;
+    const int splits = table_splits(L, B, E, U.n);
+    float* tpart = splits > 1 ? gpart + align_up(static_cast<size_t>(E) * nt, 64) : gtable;
+    FEQ_LAUNCH("k_bdm_table", k_bdm_table,
+               dim3(B.num_bins + 1, nt * tiles16(L.cout), static_cast<unsigned>(ceil_div(U.n, 4 * kMaxU) * splits)),
+               dim3(kThreads), tlds, s, L, U, B, E, perm, offsets, dist, gy, x, splits, tpart);
+    const int64_t nt_all = static_cast<int64_t>(table_floats(L, B));
+    if (splits > 1)
+        FEQ_LAUNCH("k_bdm_sum", k_bdm_sum, dim3(static_cast<unsigned>(ceil_div(nt_all, kThreads))), dim3(kThreads), 0, s,
+                   tpart, splits, nt_all, gtable);
+    return FEQ_OK;
+}
+
+}  // namespace feq

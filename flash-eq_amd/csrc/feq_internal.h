@@ -201,6 +201,17 @@ int ew0_bwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, cons
             float* gdist, const NodeScatter* ns, void* ws, size_t ws_bytes, hipStream_t s,
             const float* ym = nullptr, float* gP = nullptr, float* gQ = nullptr);
 
+// The generic block-diagonal op in float32 as matrix products over edges grouped
+// by bin (blockdiag_mm.hip); perm, offsets: the stable CSR by lower bin.
+// *dr_done: whether gdist was written.
+bool bdm_supported(const feq_layout& L, const feq_binning& B, int64_t E);
+size_t bdm_workspace(const feq_layout& L, const feq_binning& B, int64_t E);
+int bdm_fwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* x, const float* table, const float* dist,
+            const int32_t* perm, float* y, void* ws, hipStream_t s);
+int bdm_bwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* gy, const float* x, const float* table,
+            const float* dist, const int32_t* perm, const int32_t* offsets, float* gx, float* gtable, float* gdist,
+            bool* dr_done, void* ws, hipStream_t s);
+
 // Wave-per-edge family on the float32 matrix cores (edgewise_wave.hip): layouts
 // without split kernels; -1 when it does not cover the shape.  The backward
 // writes dF_e and ew_wave_groups(L, E) partials of dC for ew_tail.

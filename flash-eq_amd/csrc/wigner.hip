@@ -14,376 +14,186 @@
 //
 // Plan layout per irrep (lvals order), n = 2l+1 doubles blocks:
 //   V (n*n, row-major) | z (n): signed m coupling of each row | partner (n)
-#include "feq_internal.h"
-
-#include <cfloat>
-#include <cmath>
-#include <type_traits>
+#include "wigner_math.h"
 
 namespace feq {
 namespace {
 
-struct WignerArgs {
-    int32_t nirr;
-    int32_t dim;
-    int32_t lvals[FEQ_MAX_IRREPS];
-    int32_t off[FEQ_MAX_IRREPS];       // component offset of every irrep
-    int32_t plan_off[FEQ_MAX_IRREPS];  // offset of every irrep's plan block (doubles)
-};
+// ---- one lane per edge ------------------------------------------------------------
+// Degrees up to kLaneL.  A lane holds an edge; the workgroup's four waves take an
+// irrep's columns in turn, so every lane of a wave computes the same column of
+// the same degree and the constants V are wave-uniform (scalar loads).  Finished
+// (2l+1)^2 blocks go to LDS, an odd number of values from edge to edge (no bank
+// conflicts), and the matrices leave in rows of consecutive addresses, zeros
+// included.  FLAT: all blocks of the 64 edges fit kFlatLds and their matrices are
+// one run of memory; else block by block, whose rows are one run per edge (short
+// for small degrees: lvals 0..2, 640 000 edges, 121 us against 61).
+// With a thread per (edge, column) a wave met every degree in turn, one branch
+// after the other, and read V by lane.  Forward and backward in float32, that way
+// and this: lvals 0..6, 40 000 edges 366 and 1502 us, now 97 (384 MB written, 4.0
+// TB/s) and 207; lvals 0..4, 40 000 edges 74 and 259, now 36 and 63; lvals 0..2,
+// 640 000 edges 133 and 296, now 61 and 150.
+constexpr int kLaneEdges = 64;
 
-// nan_to_num(x, 0.0) in the output type: NaN -> 0, +-inf -> +-max
-template <class T>
-__device__ __forceinline__ T sanitize(double v) {
-    if (v != v) return T(0);
-    if constexpr (std::is_same_v<T, float>) {
-        if (v > static_cast<double>(FLT_MAX)) return FLT_MAX;
-        if (v < -static_cast<double>(FLT_MAX)) return -FLT_MAX;
-        return static_cast<float>(v);
-    } else {
-        if (v > DBL_MAX) return DBL_MAX;
-        if (v < -DBL_MAX) return -DBL_MAX;
-        return v;
-    }
-}
+constexpr size_t kFlatLds = 48 * 1024;   // three workgroups per CU
 
-// Column c of D for an irrep of degree L (n = 2L + 1) and edge angles (phi,
-// ang = theta rho): D = Z(phi) V Z(ang) V^T Z(-phi), where Z(x) rotates the
-// (r, 2L - r) pair by (L - r) x -- the structure of the m-diagonal generator,
-// which the host checks when it builds V.  All indices are compile-time, so
-// the vectors live in registers.
-template <int L>
-__device__ __forceinline__ void wigner_column(const double* __restrict__ V, int c, double phi,
-                                              double ang, double (&y)[2 * L + 1]) {
-    constexpr int n = 2 * L + 1;
-    double cp[L + 1], sp[L + 1], ca[L + 1], sa[L + 1];
-    cp[0] = 1.0;
-    sp[0] = 0.0;
-    ca[0] = 1.0;
-    sa[0] = 0.0;
-    double c1p, s1p, c1a, s1a;
-    sincos(phi, &s1p, &c1p);
-    sincos(ang, &s1a, &c1a);
-#pragma unroll
-    for (int q = 1; q <= L; ++q) {
-        cp[q] = cp[q - 1] * c1p - sp[q - 1] * s1p;
-        sp[q] = sp[q - 1] * c1p + cp[q - 1] * s1p;
-        ca[q] = ca[q - 1] * c1a - sa[q - 1] * s1a;
-        sa[q] = sa[q - 1] * c1a + ca[q - 1] * s1a;
-    }
-    // v1 = Z(-phi) e_c: entries at c (cos) and its partner n-1-c (sin of the
-    // partner's coupling), then w = V^T v1
-    const int pc = n - 1 - c;
-    const int mc = L - c;                         // coupling of row c
-    const int amc = mc < 0 ? -mc : mc;
-    double cphi = 1.0, sphi = 0.0;
-#pragma unroll
-    for (int q = 0; q <= L; ++q)
-        if (q == amc) {
-            cphi = cp[q];
-            sphi = sp[q];
+// FLAT: place of matrix element j in an edge's staged blocks, -1 outside them.
+__device__ __forceinline__ void flat_table(const WignerArgs& A, const int32_t* __restrict__ perm, int16_t* at) {
+    const int dim = A.dim;
+    for (int j = threadIdx.x; j < dim * dim; j += blockDim.x) {
+        const int r = j / dim, col = perm[j - r * dim];
+        int k = 0, off = 0;
+        while (k + 1 < A.nirr && r >= A.off[k + 1]) {
+            off += (2 * A.lvals[k] + 1) * (2 * A.lvals[k] + 1);
+            ++k;
         }
-    const double v_c = cphi;
-    const double v_p = pc != c ? (mc < 0 ? -sphi : sphi) : 0.0;
-    double w[n], u[n];
-#pragma unroll
-    for (int q = 0; q < n; ++q) w[q] = V[c * n + q] * v_c + V[pc * n + q] * v_p;
-    // u = Z(ang) w
-#pragma unroll
-    for (int r = 0; r < n; ++r) {
-        const int m = L - r, am = m < 0 ? -m : m;
-        u[r] = ca[am] * w[r] + (r != L ? (m < 0 ? -sa[am] : sa[am]) * w[n - 1 - r] : 0.0);
-    }
-    // x = V u, y = Z(phi) x
-    double xv[n];
-#pragma unroll
-    for (int r = 0; r < n; ++r) {
-        double acc = 0.0;
-#pragma unroll
-        for (int q = 0; q < n; ++q) acc += V[r * n + q] * u[q];
-        xv[r] = acc;
-    }
-#pragma unroll
-    for (int r = 0; r < n; ++r) {
-        const int m = L - r, am = m < 0 ? -m : m;
-        y[r] = cp[am] * xv[r] + (r != L ? (m < 0 ? -sp[am] : sp[am]) * xv[n - 1 - r] : 0.0);
+        const int n = 2 * A.lvals[k] + 1, c = col - A.off[k];
+        at[j] = static_cast<int16_t>(c >= 0 && c < n ? off + (r - A.off[k]) * n + c : -1);
     }
 }
 
-template <int L, class T>
-__device__ __forceinline__ void column_into(const double* V, int c, double phi, double ang,
-                                            bool ident, T* dst, int stride) {
-    constexpr int n = 2 * L + 1;
-    double y[n];
-    if (L == 0) {
-        y[0] = 1.0;
-    } else if (ident) {
-#pragma unroll
-        for (int r = 0; r < n; ++r) y[r] = r == c ? 1.0 : 0.0;
-    } else {
-        wigner_column<L>(V, c, phi, ang, y);
-    }
-#pragma unroll
-    for (int r = 0; r < n; ++r) dst[r * stride] = sanitize<T>(y[r]);
+// q / d for q < 2^20 and d < 2^13, inv = 1 / d.
+__device__ __forceinline__ int quotient(int q, float inv) {
+    return static_cast<int>((static_cast<float>(q) + 0.5f) * inv);
 }
 
-struct EdgeFrame {
-    double phi, ang;
-    int ident;   // axis of zero length: D = I
-};
-
-// Workgroup: a tile of EPB edges; thread t computes standard column c0 = t % dim
-// of edge t / dim into an LDS tile of the edges' M = D[:, perm] matrices, which
-// is then written with coalesced stores.
-// LMAX: the largest degree the launch handles (the register footprint of the
-// per-column vectors grows with it, so small representations get a small kernel).
-// T = float: the frame in float32, as the reference's float32 rot_to_ez (whose
-// clamp bounds +-(1 - eps) round to +-1); T = double: the frame in float64 with
-// the clamp as written (a float64 module runs rot_to_ez in float64).
-template <int LMAX, class T>
+template <int LMAX, class T, bool FLAT>
 __global__ void __launch_bounds__(256)
-k_wigner(WignerArgs A, int epb, const double* __restrict__ plan, const int32_t* __restrict__ perm,
-         int64_t E, const T* __restrict__ dirs, T* __restrict__ out) {
-    extern __shared__ __align__(16) char sMraw[];
-    T* sM = reinterpret_cast<T*>(sMraw);              // epb x dim x dim
-    __shared__ EdgeFrame sFr[256];
-    __shared__ int sInv[FEQ_MAX_SLOTS];
+k_wigner_lane(WignerArgs A, int stride, const double* __restrict__ plan, const int32_t* __restrict__ perm,
+              int64_t E, const T* __restrict__ dirs, T* __restrict__ out) {
+    extern __shared__ __align__(16) char sBraw[];
+    T* sB = reinterpret_cast<T*>(sBraw);              // kLaneEdges x (2l+1)^2
+    __shared__ int sPerm[FEQ_MAX_SLOTS];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int dim = A.dim, dd = dim * dim;
-    const int64_t e0 = static_cast<int64_t>(blockIdx.x) * epb;
-    const int ne = static_cast<int>(E - e0 < epb ? E - e0 : epb);
-    for (int q = threadIdx.x; q < epb * dd; q += blockDim.x) sM[q] = T(0);
-    for (int j = threadIdx.x; j < dim; j += blockDim.x) sInv[perm[j]] = j;
-    if (threadIdx.x < ne) {
-        // edge frame in float32 like rot_to_ez: d = v/(|v|+eps), axis = (-d_y, d_x, 0)/(|.|+eps),
-        // theta = acos(clamp(d_z, -1, 1)); a = rho (cos phi, sin phi)
-        const int64_t e = e0 + threadIdx.x;
-        const T eps = T(1e-8);
-        const T vx = dirs[3 * e], vy = dirs[3 * e + 1], vz = dirs[3 * e + 2];
-        const T nv = sqrt(vx * vx + vy * vy + vz * vz) + eps;
-        const T dx = vx / nv, dy = vy / nv, dz = vz / nv;
-        const T a0r = -dy, a1r = dx;
-        const T na = sqrt(a0r * a0r + a1r * a1r) + eps;
-        const T a0 = a0r / na, a1 = a1r / na;
-        const T theta = acos(fmin(fmax(dz, T(-1) + eps), T(1) - eps));
-        const double rho = sqrt(static_cast<double>(a0) * a0 + static_cast<double>(a1) * a1);
-        EdgeFrame f;
-        f.ident = rho == 0.0;
-        f.phi = f.ident ? 0.0 : atan2(static_cast<double>(a1), static_cast<double>(a0));
-        f.ang = static_cast<double>(theta) * rho;
-        sFr[threadIdx.x] = f;
-    }
-    __syncthreads();
-    const int el = threadIdx.x / dim;
-    if (el < ne) {
-        const int c0 = threadIdx.x % dim;
-        int k = 0;
-        while (k + 1 < A.nirr && c0 >= A.off[k + 1]) ++k;
-        const int l = A.lvals[k], base = A.off[k], c = c0 - base;
+    const int64_t e0 = static_cast<int64_t>(blockIdx.x) * kLaneEdges;
+    const int ne = static_cast<int>(E - e0 < kLaneEdges ? E - e0 : kLaneEdges);
+    for (int j = threadIdx.x; j < dim; j += blockDim.x) sPerm[j] = perm[j];
+    const EdgeFrame f = edge_frame(dirs + 3 * (e0 + (lane < ne ? lane : ne - 1)));
+    const Trig tr = trig_of(f.phi, f.ang);
+    int16_t* sAt = reinterpret_cast<int16_t*>(sB + kLaneEdges * stride);
+    if constexpr (FLAT) flat_table(A, perm, sAt);
+    int off = 0;
+    for (int k = 0; k < A.nirr; ++k) {
+        const int l = A.lvals[k], base = A.off[k], n = 2 * l + 1;
         const double* V = plan + A.plan_off[k];
-        const EdgeFrame f = sFr[el];
-        T* dst = sM + el * dd + base * dim + sInv[c0];   // rows base.., column j
+        T* mine = sB + (FLAT ? lane * stride + off : lane * n * n);
+        off += n * n;
+        if constexpr (!FLAT) __syncthreads();         // the previous block's copy (and sPerm)
         switch (l) {
-#define FEQ_WCASE(LL) \
-    case LL:                                                                             \
-        if constexpr (LL <= LMAX) column_into<LL>(V, c, f.phi, f.ang, f.ident, dst, dim); \
+#define FEQ_WCASE(LL)                                                                     \
+    case LL:                                                                              \
+        if constexpr (LL <= LMAX)                                                         \
+            for (int c = wave; c < n; c += 4)                                             \
+                column_into<LL>(V, c, tr, f.ident, mine + c, n);                          \
         break;
-            FEQ_WCASE(0) FEQ_WCASE(1) FEQ_WCASE(2) FEQ_WCASE(3) FEQ_WCASE(4) FEQ_WCASE(5)
-            FEQ_WCASE(6) FEQ_WCASE(7) FEQ_WCASE(8) FEQ_WCASE(9) FEQ_WCASE(10) FEQ_WCASE(11)
-            FEQ_WCASE(12) FEQ_WCASE(13) FEQ_WCASE(14) FEQ_WCASE(15) FEQ_WCASE(16)
+            FEQ_WCASE(0) FEQ_WCASE(1) FEQ_WCASE(2) FEQ_WCASE(3) FEQ_WCASE(4) FEQ_WCASE(5) FEQ_WCASE(6)
 #undef FEQ_WCASE
             default: break;
         }
+        if constexpr (FLAT) continue;
+        __syncthreads();
+        // the place in the block of each element of its rows that the lane
+        // writes (the same for every edge), -1 where D has no entry
+        const int row = n * dim;
+        for (int q0 = 0; q0 < row; q0 += 64 * 8) {
+            int at[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int q = q0 + 64 * i + lane, r = q / dim, j = q - r * dim;
+                const int c = q < row ? sPerm[j] - base : -1;
+                at[i] = c >= 0 && c < n ? r * n + c : -1;
+            }
+            for (int e = wave; e < ne; e += 4) {
+                T* o = out + (e0 + e) * dd + base * dim + q0;
+                const T* b = sB + e * n * n;
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (q0 + 64 * i + lane < row) o[64 * i + lane] = at[i] >= 0 ? b[at[i]] : T(0);
+            }
+        }
     }
-    __syncthreads();
-    T* o = out + e0 * dd;
-    for (int q = threadIdx.x; q < ne * dd; q += blockDim.x) o[q] = sM[q];
-}
-
-// ---- backward: gradient with respect to the edge directions --------------------------
-//
-// With X(phi) = cos(phi) G0 + sin(phi) G1 = Z(phi) V G2 V^T Z(-phi) and the
-// exponent theta (a0 G0 + a1 G1) = ang X(phi) (a = rho (cos phi, sin phi),
-// ang = theta rho), the derivatives of D = exp(ang X(phi)) are exact and cheap:
-//     dD/dang = X D,        dD/dphi = G2 D - D G2
-// (phi enters as a conjugation by the z-rotation Z(phi) = exp(phi G2)).  Each
-// thread takes one column c of an irrep block of D and adds, with G = dL/dD
-// (the columns of dL/dM moved back through perm):
-//     <G[:,c], X D[:,c]>                                 to dL/dang,
-//     <G[:,c], G2 D[:,c]> - z_c <G[:,pc], D[:,c]>        to dL/dphi
-// (z_c = L - c: G2's coupling of row c to its partner row pc = n-1-c).  At
-// rho = 0 (the forward's D = I) the exponent is theta (a0 G0 + a1 G1) at a = 0,
-// whose derivative is dD/da_k = theta G_k: the threads add <G[:,c], G_k e_c>.
-// One thread per edge then chains (phi, ang) -- or (a0, a1) -- back through
-// a = a_raw/(|a_raw|+eps), a_raw = (-d_y, d_x), theta = acos(d_z) and
-// d = v/(|v|+eps), the operations of rot_to_ez (wigner.py:220-238), with
-// torch's conventions (the norm's gradient is 0 at 0).
-
-// out = X(phi) y for one irrep: Z(phi) V G2 V^T Z(-phi) y, with cos(q phi),
-// sin(q phi) for q = 0..L in cpm, spm.
-template <int L>
-__device__ __forceinline__ void apply_axis_generator(const double* __restrict__ V,
-                                                     const double (&cpm)[L + 1],
-                                                     const double (&spm)[L + 1],
-                                                     const double (&y)[2 * L + 1],
-                                                     double (&out)[2 * L + 1]) {
-    constexpr int n = 2 * L + 1;
-    double u[n], w[n], x[n];
-    // u = Z(-phi) y
-#pragma unroll
-    for (int r = 0; r < n; ++r) {
-        const int m = L - r, am = m < 0 ? -m : m;
-        u[r] = cpm[am] * y[r] - (r != L ? (m < 0 ? -spm[am] : spm[am]) * y[n - 1 - r] : 0.0);
-    }
-    // w = V^T u
-#pragma unroll
-    for (int q = 0; q < n; ++q) {
-        double acc = 0.0;
-#pragma unroll
-        for (int r = 0; r < n; ++r) acc += V[r * n + q] * u[r];
-        w[q] = acc;
-    }
-    // w <- G2 w: (G2 w)[r] = (L - r) w[n-1-r]
-#pragma unroll
-    for (int r = 0; r < n; ++r) u[r] = static_cast<double>(L - r) * w[n - 1 - r];
-    // x = V u
-#pragma unroll
-    for (int r = 0; r < n; ++r) {
-        double acc = 0.0;
-#pragma unroll
-        for (int q = 0; q < n; ++q) acc += V[r * n + q] * u[q];
-        x[r] = acc;
-    }
-    // out = Z(phi) x
-#pragma unroll
-    for (int r = 0; r < n; ++r) {
-        const int m = L - r, am = m < 0 ? -m : m;
-        out[r] = cpm[am] * x[r] + (r != L ? (m < 0 ? -spm[am] : spm[am]) * x[n - 1 - r] : 0.0);
+    if constexpr (FLAT) {
+        __syncthreads();
+        const float inv = 1.0f / static_cast<float>(dd);
+        T* o = out + e0 * dd;
+#pragma unroll 4
+        for (int q = threadIdx.x; q < ne * dd; q += 256) {
+            const int e = quotient(q, inv), at = sAt[q - e * dd];
+            o[q] = at >= 0 ? sB[e * stride + at] : T(0);
+        }
     }
 }
 
-template <int L>
-__device__ __forceinline__ void multiples(double ang, double (&c)[L + 1], double (&s)[L + 1]) {
-    c[0] = 1.0;
-    s[0] = 0.0;
-    if (L == 0) return;
-    double s1, c1;
-    sincos(ang, &s1, &c1);
-#pragma unroll
-    for (int q = 1; q <= L; ++q) {
-        c[q] = c[q - 1] * c1 - s[q - 1] * s1;
-        s[q] = s[q - 1] * c1 + c[q - 1] * s1;
-    }
-}
-
-// Contributions of column c of one irrep block.  gcol / gpar: columns c and
-// n-1-c of dL/dD restricted to the block's rows.  t0/t1: (dL/dang, dL/dphi), or
-// at rho = 0 (ident) (dL/da0, dL/da1) without the factor theta.
-template <int L, class T>
-__device__ __forceinline__ void column_grad(const double* V, int c, double phi, double ang,
-                                            bool ident, const T* gcol, const T* gpar,
-                                            int stride, double& t0, double& t1) {
-    constexpr int n = 2 * L + 1;
-    t0 = 0.0;
-    t1 = 0.0;
-    if (L == 0) return;                       // D = 1 is constant
-    double g[n], gp[n], y[n], xy[n];
-#pragma unroll
-    for (int r = 0; r < n; ++r) {
-        g[r] = gcol[r * stride];
-        gp[r] = gpar[r * stride];
-    }
-    if (ident) {
-        double cz[L + 1], sz[L + 1], c9[L + 1], s9[L + 1];
-        multiples<L>(0.0, cz, sz);
-        multiples<L>(0.5 * M_PI, c9, s9);
-#pragma unroll
-        for (int r = 0; r < n; ++r) y[r] = r == c ? 1.0 : 0.0;
-        apply_axis_generator<L>(V, cz, sz, y, xy);      // G0 e_c
-#pragma unroll
-        for (int r = 0; r < n; ++r) t0 += g[r] * xy[r];
-        apply_axis_generator<L>(V, c9, s9, y, xy);      // G1 e_c
-#pragma unroll
-        for (int r = 0; r < n; ++r) t1 += g[r] * xy[r];
-        return;
-    }
-    wigner_column<L>(V, c, phi, ang, y);
-    double cp[L + 1], sp[L + 1];
-    multiples<L>(phi, cp, sp);
-    apply_axis_generator<L>(V, cp, sp, y, xy);
-#pragma unroll
-    for (int r = 0; r < n; ++r) {
-        t0 += g[r] * xy[r];
-        t1 += g[r] * static_cast<double>(L - r) * y[n - 1 - r] - static_cast<double>(L - c) * gp[r] * y[r];
-    }
-}
-
-template <int LMAX, class T>
+// One lane per edge (see k_wigner_lane): the block of dL/dM goes to LDS, every
+// wave adds its columns' terms, and the first wave sums the four in order.
+template <int LMAX, class T, bool FLAT>
 __global__ void __launch_bounds__(256)
-k_wigner_bwd(WignerArgs A, int epb, const double* __restrict__ plan, const int32_t* __restrict__ perm,
-             int64_t E, const T* __restrict__ dirs, const T* __restrict__ gM,
-             T* __restrict__ gdirs) {
-    extern __shared__ __align__(16) char sGraw[];
-    T* sG = reinterpret_cast<T*>(sGraw);              // epb x dim x dim (dL/dM tile)
-    __shared__ EdgeFrame sFr[256];
+k_wigner_lane_bwd(WignerArgs A, int stride, const double* __restrict__ plan, const int32_t* __restrict__ perm,
+                  int64_t E, const T* __restrict__ dirs, const T* __restrict__ gM, T* __restrict__ gdirs) {
+    extern __shared__ __align__(16) char sBraw[];
+    T* sB = reinterpret_cast<T*>(sBraw);              // kLaneEdges x (2l+1)^2
     __shared__ int sInv[FEQ_MAX_SLOTS];
     __shared__ double sT0[256], sT1[256];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int dim = A.dim, dd = dim * dim;
-    const int64_t e0 = static_cast<int64_t>(blockIdx.x) * epb;
-    const int ne = static_cast<int>(E - e0 < epb ? E - e0 : epb);
-    const T* gsrc = gM + e0 * dd;
-    for (int q = threadIdx.x; q < ne * dd; q += blockDim.x) sG[q] = gsrc[q];
+    const int64_t e0 = static_cast<int64_t>(blockIdx.x) * kLaneEdges;
+    const int ne = static_cast<int>(E - e0 < kLaneEdges ? E - e0 : kLaneEdges);
     for (int j = threadIdx.x; j < dim; j += blockDim.x) sInv[perm[j]] = j;
-    // The frame in double from the float32 directions: near the poles (|d_z| -> 1)
-    // d theta / d d_z = -1/sqrt(1 - d_z^2) amplifies the float32 rounding of d_z
-    // (1 - |d_z| = 3e-6 loses 2% to it), while the forward's matrices are
-    // insensitive to it; the gradient is therefore formed from an exact frame.
-    double dxv = 0.0, dyv = 0.0, dzv = 0.0, nvv = 0.0, nav = 0.0, a0v = 0.0, a1v = 0.0, thv = 0.0;
-    const double eps = 1e-8;
-    if (threadIdx.x < ne) {
-        const int64_t e = e0 + threadIdx.x;
-        const double vx = dirs[3 * e], vy = dirs[3 * e + 1], vz = dirs[3 * e + 2];
-        nvv = sqrt(vx * vx + vy * vy + vz * vz);
-        const double nv = nvv + eps;
-        dxv = vx / nv;
-        dyv = vy / nv;
-        dzv = vz / nv;
-        const double a0r = -dyv, a1r = dxv;
-        nav = sqrt(a0r * a0r + a1r * a1r);
-        const double na = nav + eps;
-        a0v = a0r / na;
-        a1v = a1r / na;
-        // the reference's clamp to [-1 + eps, 1 - eps] (wigner.py:235), which
-        // binds in float64 (within ~1.4e-4 rad of the poles; in float32 its
-        // bounds round to +-1, as the forward's float32 frame has them)
-        thv = acos(fmin(fmax(dzv, -1.0 + eps), 1.0 - eps));
-        const double rho = sqrt(a0v * a0v + a1v * a1v);
-        EdgeFrame f;
-        f.ident = rho == 0.0;
-        f.phi = f.ident ? 0.0 : atan2(a1v, a0v);
-        f.ang = thv * rho;
-        sFr[threadIdx.x] = f;
-    }
-    __syncthreads();
-    const int el = threadIdx.x / dim;
+    const int64_t el = e0 + (lane < ne ? lane : ne - 1);
+    const ExactFrame X = exact_frame(dirs + 3 * el);
+    const Trig tr = trig_of(X.f.phi, X.f.ang);
     double t0 = 0.0, t1 = 0.0;
-    if (el < ne) {
-        const int c0 = threadIdx.x % dim;
-        int k = 0;
-        while (k + 1 < A.nirr && c0 >= A.off[k + 1]) ++k;
-        const int l = A.lvals[k], base = A.off[k], c = c0 - base, n = 2 * l + 1;
+    if constexpr (FLAT) {
+        int16_t* sAt = reinterpret_cast<int16_t*>(sB + kLaneEdges * stride);
+        flat_table(A, perm, sAt);
+        __syncthreads();
+        const float inv = 1.0f / static_cast<float>(dd);
+        const T* src = gM + e0 * dd;
+#pragma unroll 8
+        for (int q = threadIdx.x; q < ne * dd; q += 256) {
+            const T v = src[q];
+            const int e = quotient(q, inv), at = sAt[q - e * dd];
+            if (at >= 0) sB[e * stride + at] = v;
+        }
+        __syncthreads();
+    }
+    int off = 0;
+    for (int k = 0; k < A.nirr; ++k) {
+        const int l = A.lvals[k], base = A.off[k], n = 2 * l + 1, nn = n * n, at = off;
+        off += nn;
+        if (l == 0) continue;                         // D = 1 is constant
         const double* V = plan + A.plan_off[k];
-        const EdgeFrame f = sFr[el];
-        // column c of dL/dD is column sInv[c] of dL/dM; rows base.. of the block
-        const T* gcol = sG + el * dd + base * dim + sInv[c0];
-        const T* gpar = sG + el * dd + base * dim + sInv[base + n - 1 - c];
+        if constexpr (!FLAT) {
+        __syncthreads();                              // the previous block's reads (and sInv)
+        for (int q0 = 0; q0 < nn; q0 += 64) {         // a lane's element is the same in every edge
+            const int q = q0 + lane, r = q / n;
+            const bool ok = q < nn;
+            const T* src = gM + e0 * dd + (ok ? (base + r) * dim + sInv[base + q - r * n] : 0);
+#pragma unroll 4
+            for (int e = wave; e < ne; e += 4) {
+                const T v = src[static_cast<int64_t>(e) * dd];
+                if (ok) sB[e * nn + q] = v;
+            }
+        }
+        __syncthreads();
+        }
+        const int le = lane < ne ? lane : ne - 1;
+        const T* b = sB + (FLAT ? le * stride + at : le * nn);
         switch (l) {
-#define FEQ_WCASE(LL)                                                                    \
-    case LL:                                                                             \
-        if constexpr (LL <= LMAX)                                                        \
-            column_grad<LL>(V, c, f.phi, f.ang, f.ident, gcol, gpar, dim, t0, t1);       \
+#define FEQ_WCASE(LL)                                                                     \
+    case LL:                                                                              \
+        if constexpr (LL <= LMAX)                                                         \
+            for (int c = wave; c < n; c += 4) {                                           \
+                double u0, u1;                                                            \
+                column_grad<LL>(V, c, tr, X.f.ident, b + c, b + n - 1 - c, n, u0, u1);    \
+                t0 += u0;                                                                 \
+                t1 += u1;                                                                 \
+            }                                                                             \
         break;
-            FEQ_WCASE(0) FEQ_WCASE(1) FEQ_WCASE(2) FEQ_WCASE(3) FEQ_WCASE(4) FEQ_WCASE(5)
-            FEQ_WCASE(6) FEQ_WCASE(7) FEQ_WCASE(8) FEQ_WCASE(9) FEQ_WCASE(10) FEQ_WCASE(11)
-            FEQ_WCASE(12) FEQ_WCASE(13) FEQ_WCASE(14) FEQ_WCASE(15) FEQ_WCASE(16)
+            FEQ_WCASE(1) FEQ_WCASE(2) FEQ_WCASE(3) FEQ_WCASE(4) FEQ_WCASE(5) FEQ_WCASE(6)
 #undef FEQ_WCASE
             default: break;
         }
@@ -391,70 +201,42 @@ k_wigner_bwd(WignerArgs A, int epb, const double* __restrict__ plan, const int32
     sT0[threadIdx.x] = t0;
     sT1[threadIdx.x] = t1;
     __syncthreads();
-    if (threadIdx.x >= ne) return;
-    // per edge: sum the columns in a fixed order, then the chain rule
+    if (wave || lane >= ne) return;
     double s0 = 0.0, s1 = 0.0;
-    for (int q = 0; q < dim; ++q) {
-        s0 += sT0[threadIdx.x * dim + q];
-        s1 += sT1[threadIdx.x * dim + q];
+    for (int w = 0; w < 4; ++w) {
+        s0 += sT0[64 * w + lane];
+        s1 += sT1[64 * w + lane];
     }
-    const EdgeFrame f = sFr[threadIdx.x];
-    const double th = thv, a0 = a0v, a1 = a1v;
-    double ga0, ga1, gth;
-    if (f.ident) {
-        ga0 = th * s0;
-        ga1 = th * s1;
-        gth = 0.0;                            // the exponent theta * (a . G) vanishes with a
-    } else {
-        const double rho = sqrt(a0 * a0 + a1 * a1);
-        const double cph = a0 / rho, sph = a1 / rho;
-        const double grho = th * s0;          // ang = theta rho
-        gth = rho * s0;
-        ga0 = cph * grho - sph / rho * s1;
-        ga1 = sph * grho + cph / rho * s1;
-    }
-    // a = a_raw / (|a_raw| + eps), a_raw = (-d_y, d_x)
-    const double ar0 = -dyv, ar1 = dxv, na = nav, ta = na + eps;
-    double gr0 = ga0 / ta, gr1 = ga1 / ta;
-    if (na > 0.0) {
-        const double dotp = (ga0 * ar0 + ga1 * ar1) / (na * ta * ta);
-        gr0 -= dotp * ar0;
-        gr1 -= dotp * ar1;
-    }
-    double gd0 = gr1, gd1 = -gr0, gd2 = 0.0;
-    // theta = acos(clamp(d_z, -1 + eps, 1 - eps)): -1/sqrt(1 - d_z^2) where the
-    // clamp passes d_z, 0 where it binds (torch's clamp gradient), so the
-    // directions along +-e_z get finite gradients, the float64 values of the
-    // reference's formula (its float32 autograd has 0 * -inf = NaN there)
-    const double dz = dzv;
-    if (gth != 0.0 && dz >= -1.0 + eps && dz <= 1.0 - eps) gd2 = -gth / sqrt(1.0 - dz * dz);
-    // d = v / (|v| + eps)
-    const int64_t e = e0 + threadIdx.x;
-    const double vx = dirs[3 * e], vy = dirs[3 * e + 1], vz = dirs[3 * e + 2];
-    const double nv = nvv, tv = nv + eps;
-    double gv0 = gd0 / tv, gv1 = gd1 / tv, gv2 = gd2 / tv;
-    if (nv > 0.0) {
-        const double dotv = (gd0 * vx + gd1 * vy + gd2 * vz) / (nv * tv * tv);
-        gv0 -= dotv * vx;
-        gv1 -= dotv * vy;
-        gv2 -= dotv * vz;
-    }
-    gdirs[3 * e] = static_cast<T>(gv0);
-    gdirs[3 * e + 1] = static_cast<T>(gv1);
-    gdirs[3 * e + 2] = static_cast<T>(gv2);
+    frame_grad(X, s0, s1, dirs + 3 * el, gdirs + 3 * el);
 }
 
 // Calls f with std::integral_constant<int, LMAX> for the smallest compiled LMAX
 // that covers every degree of A.
 template <class Fn>
-int with_lmax(const WignerArgs& A, Fn&& f) {
-    int lmax = 0;
-    for (int i = 0; i < A.nirr; ++i) lmax = A.lvals[i] > lmax ? A.lvals[i] : lmax;
+int with_lane_lmax(const WignerArgs& A, Fn&& f) {
+    const int lmax = max_degree(A);
     if (lmax <= 2) return f(std::integral_constant<int, 2>{});
     if (lmax <= 4) return f(std::integral_constant<int, 4>{});
-    if (lmax <= 6) return f(std::integral_constant<int, 6>{});
-    if (lmax <= 10) return f(std::integral_constant<int, 10>{});
-    return f(std::integral_constant<int, 16>{});
+    return f(std::integral_constant<int, kLaneL>{});
+}
+// Values from edge to edge of the FLAT form, 0 where its LDS would exceed
+// kFlatLds or, backward, where it would read the zeros of degrees over 2 for
+// nothing (lvals 0..3, 40 000 edges: 83 us against 41), and the LDS of the form that runs (else the widest block of the edges).
+template <class T>
+int lane_shape(const WignerArgs& A, bool backward, size_t* lds) {
+    size_t sum = 0;
+    for (int i = 0; i < A.nirr; ++i) sum += (2 * A.lvals[i] + 1) * (2 * A.lvals[i] + 1);
+    sum |= 1;
+    const size_t flat = sizeof(T) * kLaneEdges * sum + 2 * static_cast<size_t>(A.dim) * A.dim;
+    const size_t n = 2 * static_cast<size_t>(max_degree(A)) + 1;
+    const bool use = flat <= kFlatLds && (!backward || max_degree(A) <= 2);
+    *lds = use ? flat : sizeof(T) * kLaneEdges * n * n;
+    return use ? static_cast<int>(sum) : 0;
+}
+int set_lds(const void* fn, size_t lds) {
+    if (lds > 64 * 1024)
+        FEQ_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    return FEQ_OK;
 }
 
 }  // namespace
@@ -493,19 +275,6 @@ int wigner_args(const int32_t* lvals, int32_t n, WignerArgs& A) {
     return FEQ_OK;
 }
 
-// Edges per workgroup: one thread per (edge, column), the edges' matrices
-// (dim x dim values of T) staged in at most 64 KB of LDS.
-template <class T>
-int wigner_epb(int dim, int* epb, size_t* lds) {
-    int e = 256 / dim;
-    const int cap = static_cast<int>((64 * 1024) / (sizeof(T) * static_cast<size_t>(dim) * dim));
-    e = e < cap ? e : cap;
-    if (e < 1) return fail(FEQ_ERR_UNSUPPORTED, "representation dimension %d too large", dim);
-    *epb = e;
-    *lds = sizeof(T) * static_cast<size_t>(e) * dim * dim;
-    return FEQ_OK;
-}
-
 template <class T>
 int wigner_fwd(const int32_t* lvals, int32_t n, const double* plan, const int32_t* perm, int64_t E,
                const T* dirs, T* out, feq_stream_t stream) {
@@ -514,15 +283,17 @@ int wigner_fwd(const int32_t* lvals, int32_t n, const double* plan, const int32_
     if (E < 0) return fail(FEQ_ERR_INVALID, "negative edge count");
     if (E == 0) return FEQ_OK;
     if (!plan || !perm || !dirs || !out) return fail(FEQ_ERR_INVALID, "NULL pointer");
-    int epb;
     size_t lds;
-    if (int rc = wigner_epb<T>(A.dim, &epb, &lds)) return rc;
-    return with_lmax(A, [&](auto LL) -> int {
-        auto kern = k_wigner<decltype(LL)::value, T>;
-        FEQ_LAUNCH("k_wigner", kern, dim3(ceil_div(E, epb)), dim3(256), lds, stream_of(stream), A,
-                   epb, plan, perm, E, dirs, out);
-        return FEQ_OK;
-    });
+    if (max_degree(A) <= kLaneL)
+        return with_lane_lmax(A, [&](auto LL) -> int {
+            const int stride = lane_shape<T>(A, false, &lds);
+            auto kern = stride ? k_wigner_lane<decltype(LL)::value, T, true> : k_wigner_lane<decltype(LL)::value, T, false>;
+            if (int rc = set_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
+            FEQ_LAUNCH("k_wigner", kern, dim3(ceil_div(E, kLaneEdges)), dim3(256), lds, stream_of(stream),
+                       A, stride, plan, perm, E, dirs, out);
+            return FEQ_OK;
+        });
+    return wigner_high_fwd<T>(A, plan, perm, E, dirs, out, stream_of(stream));
 }
 
 template <class T>
@@ -533,15 +304,17 @@ int wigner_bwd(const int32_t* lvals, int32_t n, const double* plan, const int32_
     if (E < 0) return fail(FEQ_ERR_INVALID, "negative edge count");
     if (E == 0) return FEQ_OK;
     if (!plan || !perm || !dirs || !grad_out || !grad_dirs) return fail(FEQ_ERR_INVALID, "NULL pointer");
-    int epb;
     size_t lds;
-    if (int rc = wigner_epb<T>(A.dim, &epb, &lds)) return rc;
-    return with_lmax(A, [&](auto LL) -> int {
-        auto kern = k_wigner_bwd<decltype(LL)::value, T>;
-        FEQ_LAUNCH("k_wigner_bwd", kern, dim3(ceil_div(E, epb)), dim3(256), lds, stream_of(stream), A,
-                   epb, plan, perm, E, dirs, grad_out, grad_dirs);
-        return FEQ_OK;
-    });
+    if (max_degree(A) <= kLaneL)
+        return with_lane_lmax(A, [&](auto LL) -> int {
+            const int stride = lane_shape<T>(A, true, &lds);
+            auto kern = stride ? k_wigner_lane_bwd<decltype(LL)::value, T, true> : k_wigner_lane_bwd<decltype(LL)::value, T, false>;
+            if (int rc = set_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
+            FEQ_LAUNCH("k_wigner_bwd", kern, dim3(ceil_div(E, kLaneEdges)), dim3(256), lds, stream_of(stream),
+                       A, stride, plan, perm, E, dirs, grad_out, grad_dirs);
+            return FEQ_OK;
+        });
+    return wigner_high_bwd<T>(A, plan, perm, E, dirs, grad_out, grad_dirs, stream_of(stream));
 }
 }  // namespace
 

@@ -606,9 +606,11 @@ class BlockDiagonalFn(torch.autograd.Function):
                                                    N.ptr(xs), N.ptr(ts), N.ptr(rs), N.ptr(y),
                                                    N.stream_ptr(dev))
                 else:
+                    ws = N.workspace(lib.feq_blockdiag_workspace(N.ctypes.byref(layout),
+                                                                 N.ctypes.byref(binning), E), dev)
                     rc = lib.feq_blockdiag_fwd(N.ctypes.byref(layout), N.ctypes.byref(binning), E,
-                                               N.ptr(xs), N.ptr(ts), N.ptr(rs), N.ptr(y), None, 0,
-                                               N.stream_ptr(dev))
+                                               N.ptr(xs), N.ptr(ts), N.ptr(rs), N.ptr(y), N.ptr(ws),
+                                               ws.numel(), N.stream_ptr(dev))
             N.check(rc, "feq_blockdiag_fwd")
         ctx.save_for_backward(xs, ts, rs)
         ctx.meta = (layout, binning, features.dtype, table.dtype, dist.dtype)

@@ -118,8 +118,9 @@ int feq_bin_edges(const feq_binning* b, int64_t num_edges, const float* dist,
                   int32_t* lo, float* t, feq_stream_t stream);
 
 /* ---- generic block-diagonal op: table (num_bins+1, Cout, Cin, Wdim) ----------
- * The forward needs no workspace (pass NULL, 0).  The backward needs
- * feq_blockdiag_workspace bytes: it groups the edges by lower bin and sums the
+ * The forward needs no workspace (NULL, 0); given feq_blockdiag_workspace bytes
+ * it runs large calls as matrix products over edges grouped by bin.  The
+ * backward needs feq_blockdiag_workspace bytes: it groups the edges by lower bin and sums the
  * table gradient per bin in a fixed order (no atomics: the same bits on every
  * run).  grad_dist may be NULL (not needed).  grad_x, grad_table and
  * grad_dist are overwritten. */
