@@ -25,14 +25,15 @@
 // What bounds them: the float32 matrix cores (a step of 16x16x4 takes 32
 // cycles).  lvals 0..6 x 32 channels take 568 steps forward, 810 for the input
 // gradient and 624 for the pattern gradient per edge, against 30 KB of memory.
-// At 50 000 such edges: 0.73, 1.23 and 0.91 ms (51%, 44% and 46% of that
-// bound), where edgewise.hip's vector kernels (a workgroup per edge, every
+// At 50 000 such edges: 0.71, 1.21 and 0.91 ms (matrix cores busy 55%, 45% and 47%
+// of the time, the vector unit another 15 to 19%, which two waves per SIMD overlap
+// little), where edgewise.hip's vector kernels (a workgroup per edge, every
 // product through LDS) took 7.1 ms forward and 18.3 ms backward; at lvals 0..4 x
-// 32 and 20 000 edges 0.15, 0.25 and 0.19 ms against 1.24 and 3.29.  Two waves
-// per SIMD (launch bounds, and the LDS copies of the basis) cover each other's
-// memory latency; reading the operands from memory without the LDS copy of the
-// basis took 1.5, 2.9 and 1.6 ms: the requests of 4 rows x 16 scattered columns
-// bound it.
+// 32 and 20 000 edges 0.14, 0.23 and 0.18 ms against 1.24 and 3.29.  Reading the
+// operands from memory without the LDS copy of the basis took 1.5, 2.9 and 1.6 ms
+// (requests of 4 rows x 16 scattered columns); loads under lane conditions 1.0, 2.0
+// and 1.0; eight waves of the grid per resident wave, so that each read its tables
+// for two or three edges only, 0.73, 1.23 and 0.91.
 #include "feq_internal.h"
 
 namespace feq {
@@ -142,15 +143,17 @@ __device__ __forceinline__ float coef(const float* sFk, const int (&code)[2], in
 
 // A basis matrix (n = dim^2 contiguous floats, 4-byte aligned) to the wave's LDS
 // copy: requested by begin, written by end, so that other work stands between.
-constexpr int kStage = 10;      // 16-byte pieces per lane and round
+constexpr int kStage(int nb) { return nb == 1 ? 2 : nb == 2 ? 4 : nb == 3 ? 6 : 10; }   // 16-byte pieces per lane
+template <int NB>
 struct Staged {
-    v4f v[kStage];
+    v4f v[kStage(NB)];
     float tail;
 };
-__device__ __forceinline__ void stage_begin(const float* __restrict__ Bm, int n, Staged& st) {
+template <int NB>
+__device__ __forceinline__ void stage_begin(const float* __restrict__ Bm, int n, Staged<NB>& st) {
     const int lane = lane_id(), n4 = n >> 2;
 #pragma unroll
-    for (int u = 0; u < kStage; ++u)
+    for (int u = 0; u < kStage(NB); ++u)
         if (64 * u < n4) {
             const unsigned q = 64 * u + lane < n4 ? 64 * u + lane : n4 - 1;
             __builtin_memcpy(&st.v[u], Bm + 4 * q, 16);
@@ -158,18 +161,19 @@ __device__ __forceinline__ void stage_begin(const float* __restrict__ Bm, int n,
     const unsigned q = 4 * n4 + lane < n ? 4 * n4 + lane : n - 1;
     st.tail = Bm[q];
 }
-__device__ __forceinline__ void stage_end(const float* __restrict__ Bm, int n, const Staged& st, float* sB) {
+template <int NB>
+__device__ __forceinline__ void stage_end(const float* __restrict__ Bm, int n, const Staged<NB>& st, float* sB) {
     const int lane = lane_id(), n4 = n >> 2;
     wave_sync();    // earlier reads of the copy
 #pragma unroll
-    for (int u = 0; u < kStage; ++u)
+    for (int u = 0; u < kStage(NB); ++u)
         if (64 * u < n4) {
             const int q = 64 * u + lane;
             *reinterpret_cast<v4f*>(sB + 4 * (q < n4 ? q : n4 - 1)) = st.v[u];
         }
     const int q = 4 * n4 + lane;
     if (q < n) sB[q] = st.tail;
-    for (int p = 64 * kStage + lane; p < n4; p += 64) {     // dim over 50
+    for (int p = 64 * kStage(NB) + lane; p < n4; p += 64) {     // wider than the pieces
         v4f v;
         __builtin_memcpy(&v, Bm + 4 * p, 16);
         *reinterpret_cast<v4f*>(sB + 4 * p) = v;
@@ -185,14 +189,16 @@ __host__ __device__ constexpr int wave_floats(int wd, int din, int dout) {
     return basis_floats(din, dout) + (fe_floats(wd) + 3) / 4 * 4;
 }
 
-// Stages a basis with other work of the wave between request and use.
-template <class Fn>
+template <int NB, class Fn>
 __device__ __forceinline__ void stage_basis(const float* __restrict__ Bm, int dim, float* sB, Fn&& between) {
-    Staged st;
-    stage_begin(Bm, dim * dim, st);
+    Staged<NB> st;
+    stage_begin<NB>(Bm, dim * dim, st);
     between();
-    stage_end(Bm, dim * dim, st, sB);
+    stage_end<NB>(Bm, dim * dim, st, sB);
 }
+// Where its registers allow, a wave requests the next edge's basis while it works
+// on this one.
+constexpr bool ahead(int nb) { return nb <= 2; }
 
 // Elements 16 kb + 4 g + (0..3) of a row of dim floats; zeros past its end and
 // where !ok (the row is then a valid one).
@@ -341,14 +347,19 @@ __device__ __forceinline__ v4f load_c(const float* __restrict__ Ck, int co0, int
     return v;
 }
 
+// Workgroups per CU: what the registers allow without (much) spilling.  The grids
+// are one such set of workgroups, each wave taking every (grid * 4)-th edge: its
+// tables are read once.
+constexpr int fwd_groups(int ct, int nb) { return ct * nb < 8 ? 3 : 2; }
+constexpr int bwd_x_groups(int nb) { return nb == 1 ? 3 : 2; }
+
 // ---------------------------------------------------------------------------
 template <int CT, int NB>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, fwd_groups(CT, NB))
 k_ewg_fwd(GenTab T, feq_binning B, int64_t E, const float* __restrict__ x, const float* __restrict__ P,
           const float* __restrict__ Q, const float* __restrict__ dist, const float* __restrict__ C,
           const float* __restrict__ F, float* __restrict__ y) {
     extern __shared__ float sm[];
-    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int cin = T.cin, cout = T.cout, din = T.din, dout = T.dout, wd = T.wd, last = T.last;
     float* sB = sm + wave * wave_floats(wd, din, dout);
@@ -358,29 +369,45 @@ k_ewg_fwd(GenTab T, feq_binning B, int64_t E, const float* __restrict__ x, const
     load_slots<NB>(T.out_slot, out_col, out_red);
     load_deg(T, deg);
     load_codes<NB, false>(T, code);
-    for (int64_t e = static_cast<int64_t>(blockIdx.x) * 4 + wave; e < E; e += static_cast<int64_t>(gridDim.x) * 4) {
+    const int64_t step = static_cast<int64_t>(gridDim.x) * 4, first = static_cast<int64_t>(blockIdx.x) * 4 + wave;
+    Staged<ahead(NB) ? NB : 1> st;
+    if constexpr (ahead(NB))
+        if (first < E) stage_begin<NB>(P + first * din * din, din * din, st);
+    for (int64_t e = first; e < E; e += step) {
         v4f fs[CT][NB];
-        stage_basis(P + e * din * din, din, sB, [&] { edge_weights(T, B, dist[e], F, sFe, deg); });
+        if constexpr (ahead(NB)) {
+            edge_weights(T, B, dist[e], F, sFe, deg);
+            stage_end<NB>(P + e * din * din, din * din, st, sB);
+            stage_begin<NB>(P + (e + step < E ? e + step : e) * din * din, din * din, st);
+        } else {
+            stage_basis<NB>(P + e * din * din, din, sB, [&] { edge_weights(T, B, dist[e], F, sFe, deg); });
+        }
         rotate_in<CT, NB, false>(x + e * cin * din, 0, cin, sB, din, in_col, fs);
-        if (Q != P) stage_basis(Q + e * dout * dout, dout, sB, [] {});
+        if (Q != P) stage_basis<NB>(Q + e * dout * dout, dout, sB, [] {});
         for (int co0 = 0; co0 < cout; co0 += 16) {
             v4f m[NB];
 #pragma unroll
             for (int b = 0; b < NB; ++b) m[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            // the patterns one rank ahead: the products cover their latency
+            v4f cv[CT], cn[CT];
+#pragma unroll
+            for (int t = 0; t < CT; ++t) cv[t] = load_c<false>(C, co0, 16 * t, cout, cin);
 #pragma unroll 1
             for (int k = 0; k < kRank; ++k) {
-                const float* Ck = C + static_cast<int64_t>(k) * cout * cin;
+                const float* Cn = C + static_cast<int64_t>(k + 1 < kRank ? k + 1 : k) * cout * cin;
                 v4f G[NB];
+#pragma unroll
+                for (int t = 0; t < CT; ++t) cn[t] = load_c<false>(Cn, co0, 16 * t, cout, cin);
 #pragma unroll
                 for (int b = 0; b < NB; ++b) G[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int t = 0; t < CT; ++t) {
-                    const v4f cv = load_c<false>(Ck, co0, 16 * t, cout, cin);
+                for (int t = 0; t < CT; ++t)
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
 #pragma unroll
-                        for (int b = 0; b < NB; ++b) G[b] = mfma4(fs[t][b][r], cv[r], G[b]);
-                }
+                        for (int b = 0; b < NB; ++b) G[b] = mfma4(fs[t][b][r], cv[t][r], G[b]);
+#pragma unroll
+                for (int t = 0; t < CT; ++t) cv[t] = cn[t];
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -402,7 +429,7 @@ __host__ __device__ constexpr int bwd_x_floats(int wd, int din, int dout, int nb
 }
 
 template <int CT, int NB>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, bwd_x_groups(NB))
 k_ewg_bwd_x(GenTab T, feq_binning B, int64_t E, const float* __restrict__ gy, const float* __restrict__ x,
             const float* __restrict__ P, const float* __restrict__ Q, const float* __restrict__ dist,
             const float* __restrict__ C, const float* __restrict__ F, float* __restrict__ gx,
@@ -425,32 +452,47 @@ k_ewg_bwd_x(GenTab T, feq_binning B, int64_t E, const float* __restrict__ gy, co
     load_slots<NB>(T.out_slot, out_col, out_red);
     load_deg(T, deg);
     load_codes<NB, true>(T, code);
-    for (int64_t e = static_cast<int64_t>(blockIdx.x) * 4 + wave; e < E; e += static_cast<int64_t>(gridDim.x) * 4) {
+    const int64_t step = static_cast<int64_t>(gridDim.x) * 4, first = static_cast<int64_t>(blockIdx.x) * 4 + wave;
+    Staged<ahead(NB) ? NB : 1> st;
+    if constexpr (ahead(NB))
+        if (first < E) stage_begin<NB>(Q + first * dout * dout, dout * dout, st);
+    for (int64_t e = first; e < E; e += step) {
         v4f gd[CT][NB];
         float dF[kRank][kMaxW / 64] = {};   // of the weights lane + 64 j
-        stage_basis(Q + e * dout * dout, dout, sB, [&] { edge_weights(T, B, dist[e], F, sFe, deg); });
+        if constexpr (ahead(NB)) {
+            edge_weights(T, B, dist[e], F, sFe, deg);
+            stage_end<NB>(Q + e * dout * dout, dout * dout, st, sB);
+            stage_begin<NB>(Q + (e + step < E ? e + step : e) * dout * dout, dout * dout, st);
+        } else {
+            stage_basis<NB>(Q + e * dout * dout, dout, sB, [&] { edge_weights(T, B, dist[e], F, sFe, deg); });
+        }
         rotate_in<CT, NB, false>(gy + e * cout * dout, 0, cout, sB, dout, out_col, gd);
-        if (Q != P) stage_basis(P + e * din * din, din, sB, [] {});
+        if (Q != P) stage_basis<NB>(P + e * din * din, din, sB, [] {});
         for (int ci0 = 0; ci0 < cin; ci0 += 16) {
             v4f fs[1][NB], dfs[NB];
             rotate_in<1, NB, false>(x + e * cin * din, ci0, cin, sB, din, in_col, fs);
 #pragma unroll
             for (int b = 0; b < NB; ++b) dfs[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            v4f cv[CT], cn[CT];     // the patterns one rank ahead
+#pragma unroll
+            for (int t = 0; t < CT; ++t) cv[t] = load_c<true>(C, 16 * t, ci0, cout, cin);
 #pragma unroll
             for (int k = 0; k < kRank; ++k) {
-                const float* Ck = C + static_cast<int64_t>(k) * cout * cin;
+                const float* Cn = C + static_cast<int64_t>(k + 1 < kRank ? k + 1 : k) * cout * cin;
+#pragma unroll
+                for (int t = 0; t < CT; ++t) cn[t] = load_c<true>(Cn, 16 * t, ci0, cout, cin);
                 const float* sFk = sFe + k * (wd + 1);
                 v4f H[NB], Z[NB];
 #pragma unroll
                 for (int b = 0; b < NB; ++b) H[b] = Z[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int t = 0; t < CT; ++t) {
-                    const v4f cv = load_c<true>(Ck, 16 * t, ci0, cout, cin);
+                for (int t = 0; t < CT; ++t)
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
 #pragma unroll
-                        for (int b = 0; b < NB; ++b) H[b] = mfma4(gd[t][b][r], cv[r], H[b]);
-                }
+                        for (int b = 0; b < NB; ++b) H[b] = mfma4(gd[t][b][r], cv[t][r], H[b]);
+#pragma unroll
+                for (int t = 0; t < CT; ++t) cv[t] = cn[t];
                 const int ln = lane_id(), c = ln & 15, g = ln >> 4;
                 wave_sync();    // the previous rank's reads
 #pragma unroll
@@ -527,11 +569,21 @@ k_ewg_bwd_c(GenTab T, feq_binning B, int64_t E, int ncot, int subs, const float*
     for (int k = 0; k < kRank; ++k)
 #pragma unroll
         for (int t = 0; t < CT; ++t) dC[k][t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int64_t e = static_cast<int64_t>(blockIdx.x) * subs + sub; e < E; e += static_cast<int64_t>(gridDim.x) * subs) {
+    const int64_t step = static_cast<int64_t>(gridDim.x) * subs, first = static_cast<int64_t>(blockIdx.x) * subs + sub;
+    Staged<ahead(NB) ? NB : 1> st;
+    if constexpr (ahead(NB))
+        if (first < E) stage_begin<NB>(P + first * din * din, din * din, st);
+    for (int64_t e = first; e < E; e += step) {
         v4f fs[CT][NB], gd[1][NB];
-        stage_basis(P + e * din * din, din, sB, [&] { edge_weights(T, B, dist[e], F, sFe, deg); });
+        if constexpr (ahead(NB)) {
+            edge_weights(T, B, dist[e], F, sFe, deg);
+            stage_end<NB>(P + e * din * din, din * din, st, sB);
+            stage_begin<NB>(P + (e + step < E ? e + step : e) * din * din, din * din, st);
+        } else {
+            stage_basis<NB>(P + e * din * din, din, sB, [&] { edge_weights(T, B, dist[e], F, sFe, deg); });
+        }
         rotate_in<CT, NB, true>(x + e * cin * din, 0, cin, sB, din, in_col, fs);
-        if (Q != P) stage_basis(Q + e * dout * dout, dout, sB, [] {});
+        if (Q != P) stage_basis<NB>(Q + e * dout * dout, dout, sB, [] {});
         rotate_in<1, NB, true>(gy + e * cout * dout, 16 * cot, cout, sB, dout, out_col, gd);
 #pragma unroll
         for (int k = 0; k < kRank; ++k) {
@@ -693,8 +745,8 @@ int ew_wave_fwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, 
 #define FEQ_PICK(c, n) if (ct == c && nb == n) kern = k_ewg_fwd<c, n>;
     FEQ_EWG_SHAPES(FEQ_PICK)
 #undef FEQ_PICK
-    const int64_t wgs = ceil_div(E, 4);
-    const dim3 grid(static_cast<unsigned>(wgs < 2048 ? wgs : 2048));
+    const int64_t wgs = ceil_div(E, 4), most = 256 * fwd_groups(ct, nb);
+    const dim3 grid(static_cast<unsigned>(wgs < most ? wgs : most));
     const size_t lds = 4 * sizeof(float) * wave_floats(L.wdim, L.din, L.dout);
     if (int rc = set_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
     FEQ_LAUNCH("k_ewg_fwd", kern, grid, dim3(256), lds, s, T, B, E, x, P, Q, dist, C, F, y);
@@ -717,8 +769,8 @@ int ew_wave_bwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, 
     if (cti == c && nb == n) kc = k_ewg_bwd_c<c, n>;
     FEQ_EWG_SHAPES(FEQ_PICK)
 #undef FEQ_PICK
-    const int64_t wgs = ceil_div(E, 4);
-    const dim3 grid(static_cast<unsigned>(wgs < 2048 ? wgs : 2048));
+    const int64_t wgs = ceil_div(E, 4), most = 256 * bwd_x_groups(nb);
+    const dim3 grid(static_cast<unsigned>(wgs < most ? wgs : most));
     const size_t lds = 4 * sizeof(float) * bwd_x_floats(L.wdim, L.din, L.dout, nb);
     if (int rc = set_lds(reinterpret_cast<const void*>(kx), lds)) return rc;
     FEQ_LAUNCH("k_ewg_bwd_x", kx, grid, dim3(256), lds, s, T, B, E, gy, x, P, Q, dist, C, F, gx, dFe);
