@@ -20,8 +20,8 @@ namespace feq {
 namespace {
 
 // ---- one lane per edge ------------------------------------------------------------
-// Degrees up to kLaneL.  A lane holds an edge; the workgroup's four waves take an
-// irrep's columns in turn, so every lane of a wave computes the same column of
+// Degrees up to kLaneL.  A lane holds an edge; the workgroup's NW waves take the
+// columns in turn, so every lane of a wave computes the same column of
 // the same degree and the constants V are wave-uniform (scalar loads).  Finished
 // (2l+1)^2 blocks go to LDS, an odd number of values from edge to edge (no bank
 // conflicts), and the matrices leave in rows of consecutive addresses, zeros
@@ -36,6 +36,7 @@ namespace {
 constexpr int kLaneEdges = 64;
 
 constexpr size_t kFlatLds = 48 * 1024;   // three workgroups per CU
+constexpr size_t kFewLds = 128 * 1024;   // one, where there is no more than one
 
 // FLAT: place of matrix element j in an edge's staged blocks, -1 outside them.
 __device__ __forceinline__ void flat_table(const WignerArgs& A, const int32_t* __restrict__ perm, int16_t* at) {
@@ -57,8 +58,8 @@ __device__ __forceinline__ int quotient(int q, float inv) {
     return static_cast<int>((static_cast<float>(q) + 0.5f) * inv);
 }
 
-template <int LMAX, class T, bool FLAT>
-__global__ void __launch_bounds__(256)
+template <int LMAX, class T, bool FLAT, int NW>
+__global__ void __launch_bounds__(64 * NW)
 k_wigner_lane(WignerArgs A, int stride, const double* __restrict__ plan, const int32_t* __restrict__ perm,
               int64_t E, const T* __restrict__ dirs, T* __restrict__ out) {
     extern __shared__ __align__(16) char sBraw[];
@@ -75,7 +76,7 @@ k_wigner_lane(WignerArgs A, int stride, const double* __restrict__ plan, const i
     int16_t* sAt = reinterpret_cast<int16_t*>(sB + kLaneEdges * stride);
     if constexpr (FLAT) flat_table(A, perm, sAt);
     int off = 0;
-    for (int k = 0; k < A.nirr; ++k) {
+    for (int k = 0, id = 0; k < A.nirr; id += 2 * A.lvals[k] + 1, ++k) {   // id: columns before
         const int l = A.lvals[k], base = A.off[k], n = 2 * l + 1;
         const double* V = plan + A.plan_off[k];
         T* mine = sB + (FLAT ? lane * stride + off : lane * n * n);
@@ -85,7 +86,7 @@ k_wigner_lane(WignerArgs A, int stride, const double* __restrict__ plan, const i
 #define FEQ_WCASE(LL)                                                                     \
     case LL:                                                                              \
         if constexpr (LL <= LMAX)                                                         \
-            for (int c = wave; c < n; c += 4)                                             \
+            for (int c = (wave - id) & (NW - 1); c < n; c += NW)                          \
                 column_into<LL>(V, c, tr, f.ident, mine + c, n);                          \
         break;
             FEQ_WCASE(0) FEQ_WCASE(1) FEQ_WCASE(2) FEQ_WCASE(3) FEQ_WCASE(4) FEQ_WCASE(5) FEQ_WCASE(6)
@@ -105,7 +106,7 @@ k_wigner_lane(WignerArgs A, int stride, const double* __restrict__ plan, const i
                 const int c = q < row ? sPerm[j] - base : -1;
                 at[i] = c >= 0 && c < n ? r * n + c : -1;
             }
-            for (int e = wave; e < ne; e += 4) {
+            for (int e = wave; e < ne; e += NW) {
                 T* o = out + (e0 + e) * dd + base * dim + q0;
                 const T* b = sB + e * n * n;
 #pragma unroll
@@ -119,7 +120,7 @@ k_wigner_lane(WignerArgs A, int stride, const double* __restrict__ plan, const i
         const float inv = 1.0f / static_cast<float>(dd);
         T* o = out + e0 * dd;
 #pragma unroll 4
-        for (int q = threadIdx.x; q < ne * dd; q += 256) {
+        for (int q = threadIdx.x; q < ne * dd; q += 64 * NW) {
             const int e = quotient(q, inv), at = sAt[q - e * dd];
             o[q] = at >= 0 ? sB[e * stride + at] : T(0);
         }
@@ -127,15 +128,15 @@ k_wigner_lane(WignerArgs A, int stride, const double* __restrict__ plan, const i
 }
 
 // One lane per edge (see k_wigner_lane): the block of dL/dM goes to LDS, every
-// wave adds its columns' terms, and the first wave sums the four in order.
-template <int LMAX, class T, bool FLAT>
-__global__ void __launch_bounds__(256)
+// wave adds its columns' terms, and the first wave sums them in order.
+template <int LMAX, class T, bool FLAT, int NW>
+__global__ void __launch_bounds__(64 * NW)
 k_wigner_lane_bwd(WignerArgs A, int stride, const double* __restrict__ plan, const int32_t* __restrict__ perm,
                   int64_t E, const T* __restrict__ dirs, const T* __restrict__ gM, T* __restrict__ gdirs) {
     extern __shared__ __align__(16) char sBraw[];
     T* sB = reinterpret_cast<T*>(sBraw);              // kLaneEdges x (2l+1)^2
     __shared__ int sInv[FEQ_MAX_SLOTS];
-    __shared__ double sT0[256], sT1[256];
+    __shared__ double sT0[64 * NW], sT1[64 * NW];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int dim = A.dim, dd = dim * dim;
@@ -153,7 +154,7 @@ k_wigner_lane_bwd(WignerArgs A, int stride, const double* __restrict__ plan, con
         const float inv = 1.0f / static_cast<float>(dd);
         const T* src = gM + e0 * dd;
 #pragma unroll 8
-        for (int q = threadIdx.x; q < ne * dd; q += 256) {
+        for (int q = threadIdx.x; q < ne * dd; q += 64 * NW) {
             const T v = src[q];
             const int e = quotient(q, inv), at = sAt[q - e * dd];
             if (at >= 0) sB[e * stride + at] = v;
@@ -161,7 +162,7 @@ k_wigner_lane_bwd(WignerArgs A, int stride, const double* __restrict__ plan, con
         __syncthreads();
     }
     int off = 0;
-    for (int k = 0; k < A.nirr; ++k) {
+    for (int k = 0, id = 0; k < A.nirr; id += 2 * A.lvals[k] + 1, ++k) {
         const int l = A.lvals[k], base = A.off[k], n = 2 * l + 1, nn = n * n, at = off;
         off += nn;
         if (l == 0) continue;                         // D = 1 is constant
@@ -173,7 +174,7 @@ k_wigner_lane_bwd(WignerArgs A, int stride, const double* __restrict__ plan, con
             const bool ok = q < nn;
             const T* src = gM + e0 * dd + (ok ? (base + r) * dim + sInv[base + q - r * n] : 0);
 #pragma unroll 4
-            for (int e = wave; e < ne; e += 4) {
+            for (int e = wave; e < ne; e += NW) {
                 const T v = src[static_cast<int64_t>(e) * dd];
                 if (ok) sB[e * nn + q] = v;
             }
@@ -186,7 +187,7 @@ k_wigner_lane_bwd(WignerArgs A, int stride, const double* __restrict__ plan, con
 #define FEQ_WCASE(LL)                                                                     \
     case LL:                                                                              \
         if constexpr (LL <= LMAX)                                                         \
-            for (int c = wave; c < n; c += 4) {                                           \
+            for (int c = (wave - id) & (NW - 1); c < n; c += NW) {                        \
                 double u0, u1;                                                            \
                 column_grad<LL>(V, c, tr, X.f.ident, b + c, b + n - 1 - c, n, u0, u1);    \
                 t0 += u0;                                                                 \
@@ -203,7 +204,7 @@ k_wigner_lane_bwd(WignerArgs A, int stride, const double* __restrict__ plan, con
     __syncthreads();
     if (wave || lane >= ne) return;
     double s0 = 0.0, s1 = 0.0;
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < NW; ++w) {
         s0 += sT0[64 * w + lane];
         s1 += sT1[64 * w + lane];
     }
@@ -221,18 +222,22 @@ int with_lane_lmax(const WignerArgs& A, Fn&& f) {
 }
 // Values from edge to edge of the FLAT form, 0 where its LDS would exceed
 // kFlatLds or, backward, where it would read the zeros of degrees over 2 for
-// nothing (lvals 0..3, 40 000 edges: 83 us against 41), and the LDS of the form that runs (else the widest block of the edges).
+// nothing (lvals 0..3, 40 000 edges: 83 us against 41).  With few edges the
+// columns' latency is what counts forward: all degrees at once, kFewLds.  And the LDS of the form that runs (else the widest block of the edges).
 template <class T>
-int lane_shape(const WignerArgs& A, bool backward, size_t* lds) {
+int lane_shape(const WignerArgs& A, bool backward, bool few, size_t* lds) {
     size_t sum = 0;
     for (int i = 0; i < A.nirr; ++i) sum += (2 * A.lvals[i] + 1) * (2 * A.lvals[i] + 1);
     sum |= 1;
     const size_t flat = sizeof(T) * kLaneEdges * sum + 2 * static_cast<size_t>(A.dim) * A.dim;
     const size_t n = 2 * static_cast<size_t>(max_degree(A)) + 1;
-    const bool use = flat <= kFlatLds && (!backward || max_degree(A) <= 2);
+    const bool use = backward ? flat <= kFlatLds && max_degree(A) <= 2 : flat <= (few ? kFewLds : kFlatLds);
     *lds = use ? flat : sizeof(T) * kLaneEdges * n * n;
     return use ? static_cast<int>(sum) : 0;
 }
+// Fewer than two workgroups per CU: more waves share an edge's columns (16
+// forward, 8 backward, as the registers allow).
+bool few_edges(int64_t E) { return ceil_div(E, kLaneEdges) < 512; }
 int set_lds(const void* fn, size_t lds) {
     if (lds > 64 * 1024)
         FEQ_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
@@ -284,12 +289,15 @@ int wigner_fwd(const int32_t* lvals, int32_t n, const double* plan, const int32_
     if (E == 0) return FEQ_OK;
     if (!plan || !perm || !dirs || !out) return fail(FEQ_ERR_INVALID, "NULL pointer");
     size_t lds;
-    if (max_degree(A) <= kLaneL)
+    if (lane_form(A, E))
         return with_lane_lmax(A, [&](auto LL) -> int {
-            const int stride = lane_shape<T>(A, false, &lds);
-            auto kern = stride ? k_wigner_lane<decltype(LL)::value, T, true> : k_wigner_lane<decltype(LL)::value, T, false>;
+            constexpr int L = decltype(LL)::value;
+            const bool few = few_edges(E);
+            const int stride = lane_shape<T>(A, false, few, &lds);
+            auto kern = few ? (stride ? k_wigner_lane<L, T, true, 16> : k_wigner_lane<L, T, false, 16>)
+                            : (stride ? k_wigner_lane<L, T, true, 4> : k_wigner_lane<L, T, false, 4>);
             if (int rc = set_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
-            FEQ_LAUNCH("k_wigner", kern, dim3(ceil_div(E, kLaneEdges)), dim3(256), lds, stream_of(stream),
+            FEQ_LAUNCH("k_wigner", kern, dim3(ceil_div(E, kLaneEdges)), dim3(few ? 1024 : 256), lds, stream_of(stream),
                        A, stride, plan, perm, E, dirs, out);
             return FEQ_OK;
         });
@@ -305,12 +313,15 @@ int wigner_bwd(const int32_t* lvals, int32_t n, const double* plan, const int32_
     if (E == 0) return FEQ_OK;
     if (!plan || !perm || !dirs || !grad_out || !grad_dirs) return fail(FEQ_ERR_INVALID, "NULL pointer");
     size_t lds;
-    if (max_degree(A) <= kLaneL)
+    if (lane_form(A, E))
         return with_lane_lmax(A, [&](auto LL) -> int {
-            const int stride = lane_shape<T>(A, true, &lds);
-            auto kern = stride ? k_wigner_lane_bwd<decltype(LL)::value, T, true> : k_wigner_lane_bwd<decltype(LL)::value, T, false>;
+            constexpr int L = decltype(LL)::value;
+            const bool few = few_edges(E);
+            const int stride = lane_shape<T>(A, true, few, &lds);
+            auto kern = few ? (stride ? k_wigner_lane_bwd<L, T, true, 8> : k_wigner_lane_bwd<L, T, false, 8>)
+                            : (stride ? k_wigner_lane_bwd<L, T, true, 4> : k_wigner_lane_bwd<L, T, false, 4>);
             if (int rc = set_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
-            FEQ_LAUNCH("k_wigner_bwd", kern, dim3(ceil_div(E, kLaneEdges)), dim3(256), lds, stream_of(stream),
+            FEQ_LAUNCH("k_wigner_bwd", kern, dim3(ceil_div(E, kLaneEdges)), dim3(few ? 512 : 256), lds, stream_of(stream),
                        A, stride, plan, perm, E, dirs, grad_out, grad_dirs);
             return FEQ_OK;
         });

@@ -1,4 +1,5 @@
-// Wigner-D bases with degrees over kLaneL: a thread per (edge, column).
+// Wigner-D bases with degrees over kLaneL, and of few edges: a thread per (edge,
+// column) (lane_form tells which calls come here).
 #include "wigner_math.h"
 
 namespace feq {
@@ -117,6 +118,7 @@ k_wigner_bwd(WignerArgs A, int epb, const double* __restrict__ plan, const int32
 
 template <class Fn>
 int with_lmax(const WignerArgs& A, Fn&& f) {
+    if (max_degree(A) <= kLaneL) return f(std::integral_constant<int, kLaneL>{});
     if (max_degree(A) <= 10) return f(std::integral_constant<int, 10>{});
     return f(std::integral_constant<int, 16>{});
 }

@@ -19,7 +19,7 @@ struct WignerArgs {
     int32_t plan_off[FEQ_MAX_IRREPS];  // offset of every irrep's plan block (doubles)
 };
 
-// Degrees over kLaneL (wigner_high.hip).
+// The other form (wigner_high.hip).
 constexpr int kLaneL = 6;
 template <class T>
 int wigner_high_fwd(const WignerArgs& A, const double* plan, const int32_t* perm, int64_t E, const T* dirs, T* out,
@@ -28,10 +28,20 @@ template <class T>
 int wigner_high_bwd(const WignerArgs& A, const double* plan, const int32_t* perm, int64_t E, const T* dirs,
                     const T* grad_out, T* grad_dirs, hipStream_t s);
 
+// The lane kernels take degrees up to kLaneL.  Degrees 5 and 6 on few edges are
+// bound by a column's latency (its unrolled code is fetched anew in each launch),
+// and a thread per column has all columns at once: lvals 0..6, forward and
+// backward, 523 edges 23 and 40 us against 33 and 66, 5000 edges 56 and 170
+// against 35 and 69.
+constexpr int64_t kColumnEdges = 1536;
 inline int max_degree(const WignerArgs& A) {
     int lmax = 0;
     for (int i = 0; i < A.nirr; ++i) lmax = A.lvals[i] > lmax ? A.lvals[i] : lmax;
     return lmax;
+}
+inline bool lane_form(const WignerArgs& A, int64_t E) {
+    const int l = max_degree(A);
+    return l <= 4 || (l <= kLaneL && E > kColumnEdges);
 }
 
 namespace {
