@@ -7,6 +7,7 @@ library they raise ``ImportError`` naming the build command.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from typing import Optional, Sequence
@@ -205,12 +206,20 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     return lib
 
 
+_gpu_seen = False
+
+
 def lib() -> ctypes.CDLL:
-    """The library, for compute calls: requires a visible GPU."""
+    """The library, for compute calls: requires a visible GPU (asked until one was seen:
+    ``is_available`` takes about 2 us, and a training step of a block calls this 40 times)."""
+    global _gpu_seen
+    if _gpu_seen and _lib is not None:
+        return _lib
     if not torch.cuda.is_available():
         raise CUDANotAvailableError(
             "flash-eq (MI355X build) requires a ROCm GPU. No GPU was detected: "
             "torch.cuda.is_available() is False.")
+    _gpu_seen = True
     return load_library()
 
 
@@ -225,7 +234,19 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    if device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)     # without a Stream object
+
+
+_NO_CHANGE = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """``torch.cuda.device(device)``, or nothing where the thread's device is that one already."""
+    if device.index is not None and device.index == torch._C._cuda_getDevice():
+        return _NO_CHANGE
+    return torch.cuda.device(device)
 
 
 def make_layout(lvals_in: Sequence[int], lvals_out: Sequence[int], cin: int, cout: int) -> FeqLayout:

@@ -98,7 +98,7 @@ class Graph:
         offsets = torch.empty(Nn + 1, dtype=torch.int32, device=dev)
         lib = N.lib()
         ws = N.workspace(lib.feq_csr_workspace(E, Nn), dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = lib.feq_csr_by_dst(N.ptr(idx) if E else None, E, Nn, N.ptr(perm) if E else None,
                                     N.ptr(offsets), N.ptr(ws), ws.numel(), N.stream_ptr(dev))
         N.check(rc, "feq_csr_by_dst")

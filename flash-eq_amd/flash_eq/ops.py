@@ -26,7 +26,10 @@ def _f32(t: torch.Tensor, name: str) -> torch.Tensor:
         raise TypeError(f"{name}: float64 is not supported by the MI355X kernels (use float32)")
     if t.dtype not in _SUPPORTED:
         raise TypeError(f"{name}: unsupported dtype {t.dtype}")
-    return t.detach().to(torch.float32).contiguous()
+    d = t.detach()
+    if d.dtype == torch.float32 and d.is_contiguous():
+        return d
+    return d.to(torch.float32).contiguous()
 
 
 def _f64(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -71,7 +74,7 @@ class EdgewiseLinearFn(torch.autograd.Function):
             lib = N.lib()
             ws = N.workspace(lib.feq_edgewise_fwd_workspace(N.ctypes.byref(layout),
                                                             N.ctypes.byref(binning), rank, E), dev)
-            with torch.cuda.device(dev):
+            with N.on_device(dev):
                 if keep:
                     rc = lib.feq_edgewise_fwd_ym(N.ctypes.byref(layout), N.ctypes.byref(binning), rank, E,
                                                  N.ptr(xs), 0, None, N.ptr(Ps), N.ptr(Qs), N.ptr(rs),
@@ -104,7 +107,7 @@ class EdgewiseLinearFn(torch.autograd.Function):
         lib = N.lib()
         ws = N.workspace(lib.feq_edgewise_workspace(N.ctypes.byref(layout), N.ctypes.byref(binning),
                                                     rank, E), dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             if ym is not None:
                 rc = lib.feq_edgewise_bwd_pq(N.ctypes.byref(layout), N.ctypes.byref(binning), rank, E,
                                              N.ptr(g), N.ptr(xs), 0, None, None, None, N.ptr(Ps), N.ptr(Qs),
@@ -161,7 +164,7 @@ class EdgewiseLinearSrcFn(torch.autograd.Function):
             lib = N.lib()
             ws = N.workspace(lib.feq_edgewise_fwd_workspace(N.ctypes.byref(layout),
                                                             N.ctypes.byref(binning), rank, E), dev)
-            with torch.cuda.device(dev):
+            with N.on_device(dev):
                 if keep:
                     rc = lib.feq_edgewise_fwd_ym(N.ctypes.byref(layout), N.ctypes.byref(binning), rank, E,
                                                  N.ptr(xs), xs.shape[0], N.ptr(si), N.ptr(Ps), N.ptr(Qs),
@@ -194,7 +197,7 @@ class EdgewiseLinearSrcFn(torch.autograd.Function):
         lib = N.lib()
         ws = N.workspace(lib.feq_edgewise_bwd_src_nodes_workspace(
             N.ctypes.byref(layout), N.ctypes.byref(binning), rank, E), dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             if ym is not None:
                 rc = lib.feq_edgewise_bwd_pq(
                     N.ctypes.byref(layout), N.ctypes.byref(binning), rank, E, N.ptr(g), N.ptr(xs),
@@ -284,7 +287,7 @@ class EdgewiseAttnPoolFn(torch.autograd.Function):
         lib = N.lib()
         ws = N.workspace(lib.feq_edgewise_fwd_src_pool_workspace(N.ctypes.byref(layout),
                                                                  N.ctypes.byref(binning), rank, E), dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             args = (N.ctypes.byref(layout), N.ctypes.byref(binning), rank, E, N.ptr(xs), xs.shape[0],
                     N.ptr(si), N.ptr(Ps), N.ptr(Qs), N.ptr(rs), N.ptr(Cs), N.ptr(Fs), N.ptr(As), heads,
                     chan_per_head, N.ptr(di), N.ptr(perm_d) if E else None, N.ptr(offsets_d), num_dst,
@@ -314,7 +317,7 @@ class EdgewiseAttnPoolFn(torch.autograd.Function):
         if need[1]:
             gA = torch.empty_like(As)
             if E:
-                with torch.cuda.device(dev):
+                with N.on_device(dev):
                     rc = lib.feq_attn_pool_grad_attn(N.ptr(y_pos), N.ptr(g), N.ptr(perm_d), N.ptr(offsets_d),
                                                      E, num_dst, layout.cout, layout.dout, heads, N.ptr(gA),
                                                      N.stream_ptr(dev))
@@ -327,7 +330,7 @@ class EdgewiseAttnPoolFn(torch.autograd.Function):
         gF = torch.empty_like(Fs)
         ws = N.workspace(lib.feq_edgewise_bwd_src_nodes_workspace(
             N.ctypes.byref(layout), N.ctypes.byref(binning), rank, E), dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             head = (N.ctypes.byref(layout), N.ctypes.byref(binning), rank, E, N.ptr(g) if num_dst else None,
                     N.ptr(As), heads, cph, N.ptr(di), num_dst, N.ptr(xs), xs.shape[0], N.ptr(si),
                     N.ptr(perm_s) if E else None, N.ptr(offsets_s), N.ptr(Ps), N.ptr(Qs), N.ptr(rs),
@@ -521,7 +524,7 @@ class EdgewiseLinearHLFn(torch.autograd.Function):
             lib = N.lib()
             ws = N.workspace(lib.feq_edgewise_hl_workspace(N.ctypes.byref(layout),
                                                            N.ctypes.byref(binning), rank, E, 0), dev)
-            with torch.cuda.device(dev):
+            with N.on_device(dev):
                 rc = lib.feq_edgewise_hl_fwd(N.ctypes.byref(layout), N.ctypes.byref(binning), rank, E,
                                              N.ptr(xs), N.ptr(Ps), N.ptr(Qs), N.ptr(rs), N.ptr(Cs),
                                              N.ptr(Fs), N.ptr(y), N.ptr(fs), N.ptr(ws), ws.numel(),
@@ -546,7 +549,7 @@ class EdgewiseLinearHLFn(torch.autograd.Function):
         lib = N.lib()
         ws = N.workspace(lib.feq_edgewise_hl_workspace(N.ctypes.byref(layout), N.ctypes.byref(binning),
                                                        rank, E, 1), dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = lib.feq_edgewise_hl_bwd(N.ctypes.byref(layout), N.ctypes.byref(binning), rank, E,
                                          N.ptr(g), N.ptr(xs), N.ptr(Ps), N.ptr(Qs), N.ptr(rs),
                                          N.ptr(Cs), N.ptr(Fs), N.ptr(gx), N.ptr(gC), N.ptr(gF),
@@ -600,7 +603,7 @@ class BlockDiagonalFn(torch.autograd.Function):
         y = torch.empty(E, layout.cout, layout.dout, dtype=xs.dtype, device=dev)
         if E:
             lib = N.lib()
-            with torch.cuda.device(dev):
+            with N.on_device(dev):
                 if f64:
                     rc = lib.feq_blockdiag_fwd_f64(N.ctypes.byref(layout), N.ctypes.byref(binning), E,
                                                    N.ptr(xs), N.ptr(ts), N.ptr(rs), N.ptr(y),
@@ -630,7 +633,7 @@ class BlockDiagonalFn(torch.autograd.Function):
         ws = N.workspace(lib.feq_blockdiag_workspace(N.ctypes.byref(layout), N.ctypes.byref(binning),
                                                      E), dev)
         fn = lib.feq_blockdiag_bwd_f64 if xs.dtype == torch.float64 else lib.feq_blockdiag_bwd
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = fn(N.ctypes.byref(layout), N.ctypes.byref(binning), E, N.ptr(g) if E else None,
                     N.ptr(xs), N.ptr(ts), N.ptr(rs), N.ptr(gx), N.ptr(gt), N.ptr(gr), N.ptr(ws),
                     ws.numel(), N.stream_ptr(dev))
@@ -651,7 +654,7 @@ class SegmentSumFn(torch.autograd.Function):
         E = xs.shape[0]
         row = int(xs[0].numel()) if E else int(torch.tensor(xs.shape[1:]).prod())
         out = torch.empty((num_nodes,) + tuple(xs.shape[1:]), dtype=torch.float32, device=dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = N.lib().feq_segment_sum(N.ptr(xs) if E else None, row, N.ptr(perm) if E else None,
                                          N.ptr(offsets), num_nodes, N.ptr(out), N.stream_ptr(dev))
         N.check(rc, "feq_segment_sum")
@@ -668,7 +671,7 @@ class SegmentSumFn(torch.autograd.Function):
         gx = torch.empty(shape, dtype=torch.float32, device=dev)
         if E:
             d64 = dst.to(torch.int64).contiguous()
-            with torch.cuda.device(dev):
+            with N.on_device(dev):
                 rc = N.lib().feq_gather_rows(N.ptr(g), num_nodes, row, N.ptr(d64), E, N.ptr(gx),
                                              N.stream_ptr(dev))
             N.check(rc, "feq_gather_rows")
@@ -689,7 +692,7 @@ class GatherRowsFn(torch.autograd.Function):
         out = torch.empty((E,) + tuple(xs.shape[1:]), dtype=torch.float32, device=dev)
         i64 = idx.to(torch.int64).contiguous()
         if E:
-            with torch.cuda.device(dev):
+            with N.on_device(dev):
                 rc = N.lib().feq_gather_rows(N.ptr(xs), num_src, row, N.ptr(i64), E, N.ptr(out),
                                              N.stream_ptr(dev))
             N.check(rc, "feq_gather_rows")
@@ -704,7 +707,7 @@ class GatherRowsFn(torch.autograd.Function):
         dev = perm.device
         g = gout.detach().to(torch.float32).contiguous()
         gx = torch.empty(shape, dtype=torch.float32, device=dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = N.lib().feq_segment_sum(N.ptr(g) if E else None, row, N.ptr(perm) if E else None,
                                          N.ptr(offsets), num_src, N.ptr(gx), N.stream_ptr(dev))
         N.check(rc, "feq_segment_sum")
@@ -731,7 +734,7 @@ class EdgeSoftmaxFn(torch.autograd.Function):
         attn = torch.empty(E, H, dtype=torch.float32, device=dev)
         qk = torch.empty(E, H, dtype=torch.float32, device=dev)
         if E:
-            with torch.cuda.device(dev):
+            with N.on_device(dev):
                 rc = N.lib().feq_attn_softmax_fwd(N.ptr(Qs), H * Dh, N.ptr(Ks), H * Dh, None, None,
                                                   E, N.ptr(rs), E, H, Dh, N.ptr(scale_t),
                                                   float(decay), N.ptr(perm), N.ptr(offsets),
@@ -755,7 +758,7 @@ class EdgeSoftmaxFn(torch.autograd.Function):
         gK = torch.empty_like(Ks)
         glog = torch.empty(E, H, dtype=torch.float32, device=dev)
         if E:
-            with torch.cuda.device(dev):
+            with N.on_device(dev):
                 rc = N.lib().feq_attn_softmax_bwd(N.ptr(Qs), H * Dh, N.ptr(Ks), H * Dh, None, None,
                                                   E, N.ptr(attn), N.ptr(ga), E, H, Dh,
                                                   N.ptr(scale_t), N.ptr(perm),
@@ -813,7 +816,7 @@ class NodeSoftmaxFn(torch.autograd.Function):
         attn = torch.empty(E, heads, dtype=torch.float32, device=dev)
         qkv = torch.empty(E, heads, dtype=torch.float32, device=dev)
         if E:
-            with torch.cuda.device(dev):
+            with N.on_device(dev):
                 if cm:
                     rc = N.lib().feq_attn_softmax_fwd_cm(N.ptr(qs), N.ptr(qs) + 4 * mult, two_mult,
                                                          Nn * two_mult, dim, N.ptr(dst), N.ptr(src), Nn,
@@ -853,7 +856,7 @@ class NodeSoftmaxFn(torch.autograd.Function):
             return (torch.zeros_like(qs).to(qdt), g_dist, g_log, None, None, None, None, None, None,
                     None, None, None, None)
         gqk = torch.empty_like(qs)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             if cm:
                 rc = N.lib().feq_attn_softmax_bwd_cm(N.ptr(qs), N.ptr(qs) + 4 * mult, two_mult, Nn * two_mult,
                                                      dim, N.ptr(dst), N.ptr(src), Nn, N.ptr(attn), N.ptr(ga),
@@ -883,7 +886,7 @@ class AttnPoolFn(torch.autograd.Function):
         Vs, As = _f32(V, "V"), _f32(attn, "attention")
         E, mult, dim = Vs.shape
         out = torch.empty(num_nodes, mult, dim, dtype=torch.float32, device=dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = N.lib().feq_attn_pool_fwd(N.ptr(Vs) if E else None, N.ptr(As) if E else None, E,
                                            mult, dim, heads, N.ptr(perm) if E else None,
                                            N.ptr(offsets), num_nodes, N.ptr(out), N.stream_ptr(dev))
@@ -902,7 +905,7 @@ class AttnPoolFn(torch.autograd.Function):
         gV = torch.empty_like(Vs)
         gA = torch.empty_like(As)
         if E:
-            with torch.cuda.device(dev):
+            with N.on_device(dev):
                 rc = N.lib().feq_attn_pool_bwd(N.ptr(Vs), N.ptr(As), N.ptr(g), N.ptr(perm),
                                                N.ptr(offsets), E, num_nodes, mult, dim, heads,
                                                N.ptr(gV), N.ptr(gA), N.stream_ptr(dev))
@@ -918,7 +921,7 @@ def bin_edges(dist: torch.Tensor, binning: N.FeqBinning) -> Tuple[torch.Tensor, 
     lo = torch.empty(E, dtype=torch.int32, device=dev)
     t = torch.empty(E, dtype=torch.float32, device=dev)
     if E:
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = N.lib().feq_bin_edges(N.ctypes.byref(binning), E, N.ptr(rs), N.ptr(lo), N.ptr(t),
                                        N.stream_ptr(dev))
         N.check(rc, "feq_bin_edges")
@@ -975,7 +978,7 @@ class SepNormFn(torch.autograd.Function):
         y = torch.empty(dim, n, mult, dtype=xs.dtype, device=xs.device) if cm else torch.empty_like(xs)
         if n:
             fn = N.lib().feq_sepnorm_fwd_cm if cm else N.lib().feq_sepnorm_fwd
-            with torch.cuda.device(xs.device):
+            with N.on_device(xs.device):
                 rc = fn(_lvals_i32(lvals), len(lvals), mult, n, N.ptr(xs), N.ptr(w_s), N.ptr(b_s),
                         N.ptr(w_h), eps, N.ptr(y), N.stream_ptr(xs.device))
             N.check(rc, "feq_sepnorm_fwd")
@@ -1001,7 +1004,7 @@ class SepNormFn(torch.autograd.Function):
         lib = N.lib()
         arr = _lvals_i32(lvals)
         ws = N.workspace(lib.feq_sepnorm_workspace(arr, len(lvals), mult, n), dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             if ga is not None:
                 ga = ga.contiguous()
                 rc = lib.feq_sepnorm_bwd_add(arr, len(lvals), mult, n, N.ptr(gy), N.ptr(xs), N.ptr(w_s),
@@ -1030,7 +1033,7 @@ class EqNormFn(torch.autograd.Function):
         y = torch.empty(dim, n, mult, dtype=xs.dtype, device=xs.device) if cm else torch.empty_like(xs)
         if n:
             fn = N.lib().feq_eqnorm_fwd_cm if cm else N.lib().feq_eqnorm_fwd
-            with torch.cuda.device(xs.device):
+            with N.on_device(xs.device):
                 rc = fn(_lvals_i32(lvals), len(lvals), mult, n, N.ptr(xs),
                                             N.ptr(w_ln), N.ptr(b_ln), eps, ln_eps, N.ptr(y),
                                             N.stream_ptr(xs.device))
@@ -1056,7 +1059,7 @@ class EqNormFn(torch.autograd.Function):
         lib = N.lib()
         arr = _lvals_i32(lvals)
         ws = N.workspace(lib.feq_eqnorm_workspace(arr, len(lvals), mult, n), dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             if ga is not None:
                 ga = ga.contiguous()
                 rc = lib.feq_eqnorm_bwd_add(arr, len(lvals), mult, n, N.ptr(gy), N.ptr(xs), N.ptr(w_ln),
@@ -1085,7 +1088,7 @@ def transpose_last2(t: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
     if not t.is_cuda:
         return t.view(-1, rows, cols).transpose(1, 2).contiguous().view(t.shape)
     out = torch.empty_like(t)
-    with torch.cuda.device(t.device):
+    with N.on_device(t.device):
         rc = N.lib().feq_transpose(N.ptr(t), n // (rows * cols), rows, cols, t.element_size(),
                                    N.ptr(out), N.stream_ptr(t.device))
     N.check(rc, "feq_transpose")
@@ -1105,7 +1108,7 @@ def column_sums(t: torch.Tensor) -> torch.Tensor:
     lib = N.lib()
     es = ts.element_size()
     ws = N.workspace(lib.feq_column_sums_workspace(rows, cols, es), ts.device)
-    with torch.cuda.device(ts.device):
+    with N.on_device(ts.device):
         rc = lib.feq_column_sums(N.ptr(ts), rows, cols, es, N.ptr(out), N.ptr(ws), ws.numel(),
                                  N.stream_ptr(ts.device))
     N.check(rc, "feq_column_sums")
@@ -1125,7 +1128,7 @@ def dot_f64(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
         out = torch.empty((), dtype=torch.float32, device=a_.device)
         lib = N.lib()
         ws = N.workspace(lib.feq_dot_f64_workspace(), a_.device)
-        with torch.cuda.device(a_.device):
+        with N.on_device(a_.device):
             rc = lib.feq_dot_f64(N.ptr(a_), N.ptr(b_), a_.numel(), N.ptr(out), N.ptr(ws),
                                  ws.numel(), N.stream_ptr(a_.device))
         N.check(rc, "feq_dot_f64")
@@ -1180,7 +1183,7 @@ class ResidualScaleFn(torch.autograd.Function):
         if xs.shape != ys.shape:
             raise RuntimeError(f"residual: shapes {tuple(xs.shape)} and {tuple(ys.shape)}")
         out = torch.empty_like(xs)
-        with torch.cuda.device(xs.device):
+        with N.on_device(xs.device):
             rc = N.lib().feq_scale_add(N.ptr(xs), N.ptr(ys), N.ptr(gamma), xs.numel(), N.ptr(out),
                                        N.stream_ptr(xs.device))
         N.check(rc, "feq_scale_add")
@@ -1196,7 +1199,7 @@ class ResidualScaleFn(torch.autograd.Function):
         if gy is not None or gg is not None:
             lib = N.lib()
             ws = N.workspace(lib.feq_dot_f64_workspace(), g.device)
-            with torch.cuda.device(g.device):
+            with N.on_device(g.device):
                 rc = lib.feq_scale_add_bwd(N.ptr(g), N.ptr(ys), N.ptr(gamma), g.numel(),
                                            N.ptr(gy) if gy is not None else None,
                                            N.ptr(gg) if gg is not None else None, N.ptr(ws), ws.numel(),
@@ -1220,7 +1223,7 @@ class ResidualScaleCmFn(torch.autograd.Function):
         if ys.shape != (dim, n, mult):
             raise RuntimeError(f"residual: component-major branch {tuple(ys.shape)} for rows {tuple(xs.shape)}")
         out = torch.empty_like(xs)
-        with torch.cuda.device(xs.device):
+        with N.on_device(xs.device):
             rc = N.lib().feq_scale_add_cm(N.ptr(xs), N.ptr(ys), N.ptr(gamma), n, mult, dim, N.ptr(out),
                                           N.stream_ptr(xs.device))
         N.check(rc, "feq_scale_add_cm")
@@ -1238,7 +1241,7 @@ class ResidualScaleCmFn(torch.autograd.Function):
         if gy is not None or gg is not None:
             lib = N.lib()
             ws = N.workspace(lib.feq_scale_add_cm_workspace(), g.device)
-            with torch.cuda.device(g.device):
+            with N.on_device(g.device):
                 rc = lib.feq_scale_add_cm_bwd(N.ptr(g), N.ptr(ys), N.ptr(gamma), n, mult, dim,
                                               N.ptr(gy) if gy is not None else None,
                                               N.ptr(gg) if gg is not None else None, N.ptr(ws), ws.numel(),
@@ -1295,7 +1298,7 @@ class FanOutFn(torch.autograd.Function):
             gc = [g.contiguous() for g in gs]
             out = torch.empty_like(gc[0])
             ptrs = (N.ctypes.c_void_p * len(gc))(*[g.data_ptr() for g in gc])
-            with torch.cuda.device(out.device):
+            with N.on_device(out.device):
                 rc = N.lib().feq_sum_tables(ptrs, len(gc), out.numel(), N.ptr(out), N.stream_ptr(out.device))
             N.check(rc, "feq_sum_tables")
             return out, None
@@ -1326,13 +1329,13 @@ class GatingFn(torch.autograd.Function):
         lib = N.lib()
         arr = _lvals_i32(lvals)
         norms = torch.empty(n, mult * nreps, dtype=torch.float32, device=dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = lib.feq_gate_norms(arr, nreps, mult, n, int(cm), N.ptr(xs), eps, N.ptr(norms),
                                     N.stream_ptr(dev))
         N.check(rc, "feq_gate_norms")
         lin = torch.addmm(bias.detach(), norms, weight.detach().t())
         y = torch.empty_like(xs)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = lib.feq_gate_apply(arr, nreps, mult, n, int(cm), N.ptr(xs), N.ptr(lin), N.ptr(y),
                                     N.stream_ptr(dev))
         N.check(rc, "feq_gate_apply")
@@ -1350,7 +1353,7 @@ class GatingFn(torch.autograd.Function):
         arr = _lvals_i32(lvals)
         nreps = len(lvals)
         dlin = torch.empty_like(lin)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = lib.feq_gate_bwd_lin(arr, nreps, mult, n, int(cm), N.ptr(gy), N.ptr(xs),
                                       N.ptr(lin), N.ptr(dlin), N.stream_ptr(dev))
         N.check(rc, "feq_gate_bwd_lin")
@@ -1358,7 +1361,7 @@ class GatingFn(torch.autograd.Function):
         gw = rows_weight_grad(dlin, norms, weight.dtype) if ctx.needs_input_grad[1] else None
         gb = column_sums(dlin) if ctx.needs_input_grad[2] else None
         gx = torch.empty_like(xs)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = lib.feq_gate_bwd_x(arr, nreps, mult, n, int(cm), N.ptr(gy), N.ptr(xs),
                                     N.ptr(lin), N.ptr(norms), N.ptr(dnorms), N.ptr(gx),
                                     N.stream_ptr(dev))
@@ -1406,7 +1409,7 @@ class EqLinearFn(torch.autograd.Function):
             wc = weight.detach().contiguous()
             bc = bias.detach().contiguous() if bias is not None else None
             ws = N.workspace(lib.feq_eqlinear_workspace(nreps, cin, cout), fd.device)
-            with torch.cuda.device(fd.device):
+            with N.on_device(fd.device):
                 rc = lib.feq_eqlinear_fwd(_lvals_i32(_slice_lvals(slices)), nreps, rows, cin, cout,
                                           N.ptr(fd), N.ptr(wc), N.ptr(bc) if bc is not None else None,
                                           bc.shape[1] if bc is not None else 0,
@@ -1438,18 +1441,19 @@ class EqLinearFn(torch.autograd.Function):
         gfd = torch.empty_like(fd) if ctx.needs_input_grad[0] else None
         gw = torch.empty_like(w) if ctx.needs_input_grad[1] else None
         gb = torch.zeros_like(bias) if bias is not None and ctx.needs_input_grad[2] else None
-        fused_x = gfd is not None and eqlinear_kernels_ok(gyd, weight, slices, cin, cout)
+        kernels = eqlinear_kernels_ok(gyd, weight, slices, cin, cout)
+        fused_x = gfd is not None and kernels
         if fused_x:
             lib = N.lib()
             nreps = len(slices)
             wc = weight.detach().contiguous()
             ws = N.workspace(lib.feq_eqlinear_workspace(nreps, cin, cout), gyd.device)
-            with torch.cuda.device(gyd.device):
+            with N.on_device(gyd.device):
                 rc = lib.feq_eqlinear_bwd_x(_lvals_i32(_slice_lvals(slices)), nreps, gyd.shape[1], cin,
                                             cout, N.ptr(gyd), N.ptr(wc), N.ptr(gfd), N.ptr(ws), ws.numel(),
                                             N.stream_ptr(gyd.device))
             N.check(rc, "feq_eqlinear_bwd_x")
-        fused_w = (gw is not None or gb is not None) and eqlinear_kernels_ok(gyd, weight, slices, cin, cout)
+        fused_w = (gw is not None or gb is not None) and kernels
         if fused_w:
             lib = N.lib()
             nreps = len(slices)
@@ -1457,7 +1461,7 @@ class EqLinearFn(torch.autograd.Function):
             rows = gyd.shape[1]
             gwk = gw if gw is not None else torch.empty_like(w)
             ws = N.workspace(lib.feq_eqlinear_bwd_w_workspace(lv, nreps, rows, cin, cout), gyd.device)
-            with torch.cuda.device(gyd.device):
+            with N.on_device(gyd.device):
                 rc = lib.feq_eqlinear_bwd_w(lv, nreps, rows, cin, cout, N.ptr(gyd), N.ptr(fd),
                                             gb.shape[1] if gb is not None else 0,
                                             _lvals_i32(bias_cols) if gb is not None else None, N.ptr(gwk),
@@ -1495,7 +1499,7 @@ class RadialMLPFn(torch.autograd.Function):
         F = torch.empty(B, O, dtype=torch.float32, device=dev)
         acts = torch.empty(B, 4 * H, dtype=torch.float32, device=dev)
         ts = [t.detach().contiguous() for t in (basis, W1, b1, W2, b2, W3, b3)]
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = N.lib().feq_radial_fwd(N.ptr(ts[0]), B, I, H, O, *[N.ptr(t) for t in ts[1:]], N.ptr(F),
                                         N.ptr(acts), N.stream_ptr(dev))
         N.check(rc, "feq_radial_fwd")
@@ -1514,7 +1518,7 @@ class RadialMLPFn(torch.autograd.Function):
                  torch.empty(H, device=dev), torch.empty_like(W3), torch.empty(O, device=dev)]
         lib = N.lib()
         ws = N.workspace(lib.feq_radial_workspace(B, H), dev)
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = lib.feq_radial_bwd(N.ptr(basis), B, I, H, O, N.ptr(W2), N.ptr(W3), N.ptr(acts), N.ptr(g),
                                     *[N.ptr(t) for t in grads], N.ptr(ws), ws.numel(), N.stream_ptr(dev))
         N.check(rc, "feq_radial_bwd")
@@ -1540,7 +1544,7 @@ class SumSquaresFn(torch.autograd.Function):
         lib = N.lib()
         fn = lib.feq_sum_squares if ys.dtype == torch.float32 else lib.feq_sum_squares_bf16
         ws = N.workspace(lib.feq_sum_squares_workspace(), ys.device)
-        with torch.cuda.device(ys.device):
+        with N.on_device(ys.device):
             rc = fn(N.ptr(ys), ys.numel(), N.ptr(out), N.ptr(ws), ws.numel(), N.stream_ptr(ys.device))
         N.check(rc, "feq_sum_squares")
         ctx.save_for_backward(ys)

@@ -181,7 +181,7 @@ class _WignerBasisFn(torch.autograd.Function):
         out = torch.empty(E, dim, dim, dtype=wdt, device=dev)
         lv = (N.ctypes.c_int32 * len(lvals_i32))(*lvals_i32)
         fn = "feq_wigner_basis_f64" if wdt == torch.float64 else "feq_wigner_basis"
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = getattr(N.lib(), fn)(lv, len(lvals_i32), N.ptr(plan), N.ptr(perm_i32), E,
                                       N.ptr(dirs) if E else None, N.ptr(out) if E else None,
                                       N.stream_ptr(dev))
@@ -200,7 +200,7 @@ class _WignerBasisFn(torch.autograd.Function):
         gd = torch.empty_like(dirs)
         lv = (N.ctypes.c_int32 * len(lvals))(*lvals)
         fn = "feq_wigner_basis_bwd_f64" if dirs.dtype == torch.float64 else "feq_wigner_basis_bwd"
-        with torch.cuda.device(dev):
+        with N.on_device(dev):
             rc = getattr(N.lib(), fn)(lv, len(lvals), N.ptr(plan), N.ptr(perm_i32), E,
                                       N.ptr(dirs) if E else None, N.ptr(g) if E else None,
                                       N.ptr(gd) if E else None, N.stream_ptr(dev))
