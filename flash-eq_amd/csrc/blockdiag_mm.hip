@@ -20,10 +20,11 @@
 // the staged rows and split the (m, output) pairs.  Sums run in a fixed order.
 //
 // Lvals 0..2 x 32, 20 000 edges, 65 table rows, the per-edge kernels and these:
-// forward 1163 us, now 94 + 15 (pack) + 35 (sort by bin); input and distance
-// gradients 816 + 1724, now 154 + 17 (pack); table gradient 2256, now 232 + 10.
+// forward 1163 us, now 71 + 15 (pack) + 35 (sort by bin); input and distance
+// gradients 816 + 1724, now 126 + 16 (pack); table gradient 2256, now 154 + 10.
 // The matrix steps alone would take 20 to 40 us each: the staging of 16 edges'
-// rows, one memory latency per 16 channels, bounds these.
+// rows, one memory latency per 16 channels, bounds these.  (Tiles dealt to the
+// L2s in turn, so that each read every bin's fragments: 94 and 154 us.)
 #include "feq_internal.h"
 
 namespace feq {
@@ -83,27 +84,38 @@ __device__ __forceinline__ EdgeRow edge_row(const feq_binning& B, const int32_t*
     return R;
 }
 
-// Rows c0 .. c0 + 15 of (E, nch, dim) of the 16 edges at e[], times scale[edge][l],
-// and weight[edge], to st[slot][channel][edge] (EDGE_MINOR) or st[slot][edge][channel]; zeros for
-// channels outside and for edges from n on.
+// q / d for q < 2^15 and d < 2^10, inv = 1 / d.
+__device__ __forceinline__ int quotient(int q, float inv) {
+    return static_cast<int>((static_cast<float>(q) + 0.5f) * inv);
+}
+
+// Rows c0 .. c0 + 15 of (E, nch, dim) of the 16 edges at e[], times scale[edge][l]
+// and weight[edge], to st[slot][channel][edge] (EDGE_MINOR) or
+// st[slot][edge][channel]; zeros for channels outside and for edges from n on.  A
+// thread requests kInFlight elements before it uses the first (four at a time took
+// the table gradient 232 us instead of 154).
+constexpr int kInFlight = 10;
 template <bool EDGE_MINOR>
 __device__ __forceinline__ void stage_rows(const float* __restrict__ x, int nch, int c0, int dim, const int64_t* e,
-                                           const float* scale, int sstride, const int8_t* deg, int n, float* st,
+                                           const float* scale, int sstride, const int* deg, int n, float* st,
                                            const float* weight = nullptr) {
-    const int per = 16 * dim;
-    for (int q0 = threadIdx.x; q0 < 16 * per; q0 += 4 * kThreads) {
-        float v[4];
+    const int per = 16 * dim, all = 16 * per;
+    const float iper = 1.0f / static_cast<float>(per), idim = 1.0f / static_cast<float>(dim);
+    for (int q0 = threadIdx.x; q0 < all; q0 += kInFlight * kThreads) {
+        float v[kInFlight];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int q = q0 + u * kThreads, ed = q / per, rest = q - ed * per, ch = rest / dim;
-            const bool ok = q < 16 * per && ed < n && c0 + ch < nch;
-            v[u] = x[ok ? (e[ed & 15] * nch + c0) * dim + rest : 0];
+        for (int u = 0; u < kInFlight; ++u) {
+            const int q = q0 + u * kThreads < all ? q0 + u * kThreads : all - 1;
+            const int ed = quotient(q, iper), rest = q - ed * per, ch = quotient(rest, idim);
+            const bool ok = ed < n && c0 + ch < nch;
+            v[u] = x[ok ? (e[ed] * nch + c0) * dim + rest : 0];
             v[u] = ok ? v[u] : 0.0f;
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int q = q0 + u * kThreads, ed = q / per, rest = q - ed * per, ch = rest / dim, d = rest - ch * dim;
-            if (q < 16 * per) {
+        for (int u = 0; u < kInFlight; ++u) {
+            const int q = q0 + u * kThreads;
+            if (q < all) {
+                const int ed = quotient(q, iper), rest = q - ed * per, ch = quotient(rest, idim), d = rest - ch * dim;
                 float sc = scale[ed * sstride + deg[d]];
                 if (weight) sc *= weight[ed];
                 st[d * kSS + (EDGE_MINOR ? ch * 16 + ed : ed * 16 + ch)] = v[u] * sc;
@@ -164,7 +176,7 @@ struct TileAcc {
 template <int MAXP, bool GD, int SIGN>
 __device__ __forceinline__ void tile_product(const Pairs& PT, int wave, const float* __restrict__ frag, int64_t bin, int wd,
                                              int nrow, int row, int nred, int red, const float* st, float mask, float t,
-                                             const int8_t* deg, TileAcc<MAXP, GD>& A) {
+                                             const int* deg, TileAcc<MAXP, GD>& A) {
     const int lane = threadIdx.x & 63;
     const int64_t wstride = static_cast<int64_t>(nrow) * nred * 512;
     const float* f0 = frag + ((bin * wd * nrow + row) * nred + red) * 512;
@@ -172,18 +184,26 @@ __device__ __forceinline__ void tile_product(const Pairs& PT, int wave, const fl
     for (int p = 0; p < MAXP; ++p) {
         if (wave + 4 * p >= PT.n) break;
         const Pair P = PT.p[wave + 4 * p];
-        for (int k = 0; k < P.n; ++k) {
+        v4f Tn[2], Dn[2];       // the next summed index's fragments
+        auto fetch = [&](int k) {
             const float* fa = f0 + (P.w + k * P.step) * wstride;
+            Tn[0] = *reinterpret_cast<const v4f*>(fa + 4 * lane);
+            Dn[0] = *reinterpret_cast<const v4f*>(fa + 256 + 4 * lane);
+            if (P.z == 2) {
+                Tn[1] = *reinterpret_cast<const v4f*>(fa + wstride + 4 * lane);
+                Dn[1] = *reinterpret_cast<const v4f*>(fa + wstride + 256 + 4 * lane);
+            }
+        };
+        fetch(0);
+        for (int k = 0; k < P.n; ++k) {
             const float* sr = st + (P.other + P.z * k) * kSS;
-            v4f T[2], D[2], S[2];
-            T[0] = *reinterpret_cast<const v4f*>(fa + 4 * lane);
-            D[0] = *reinterpret_cast<const v4f*>(fa + 256 + 4 * lane);
+            const v4f T[2] = {Tn[0], Tn[1]}, D[2] = {Dn[0], Dn[1]};
+            v4f S[2];
+            if (k + 1 < P.n) fetch(k + 1);
 #pragma unroll
             for (int r = 0; r < 4; ++r) S[0][r] = sr[64 * r + lane] * mask;
             const float l = GD ? static_cast<float>(deg[P.other + P.z * k]) : 0.0f;
             if (P.z == 2) {
-                T[1] = *reinterpret_cast<const v4f*>(fa + wstride + 4 * lane);
-                D[1] = *reinterpret_cast<const v4f*>(fa + wstride + 256 + 4 * lane);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) S[1][r] = sr[kSS + 64 * r + lane] * mask;
             }
@@ -246,7 +266,7 @@ __global__ void __launch_bounds__(kThreads, 2)
 k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __restrict__ perm,
             const float* __restrict__ dist, const float* __restrict__ x, int nch, int din, int noch, int dout, int wd,
             const float* __restrict__ frag, const float* __restrict__ xo, float* __restrict__ y,
-            float* __restrict__ gpart) {
+            float* __restrict__ gpart, unsigned tiles) {
     extern __shared__ float st[];
     __shared__ float sPow[16 * (kPow + 1)];
     __shared__ int64_t sE[16];
@@ -254,10 +274,16 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
     __shared__ float sRed[4 * 64];
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t p0 = static_cast<int64_t>(blockIdx.x) * 16;
+    // the eight L2s (workgroups go to them in turn) take an eighth of the sorted
+    // tiles each: a bin's fragments are then read into one or two of them
+    const unsigned each = gridDim.x / 8;
+    const unsigned tile = (blockIdx.x & 7) * each + (blockIdx.x >> 3);
+    if (tile >= tiles) return;
+    const int64_t p0 = static_cast<int64_t>(tile) * 16;
     const int n = static_cast<int>(E - p0 < 16 ? E - p0 : 16);
-    const int8_t* din_deg = SIGN > 0 ? L.lslot_in : L.lslot_out;
-    const int8_t* dout_deg = SIGN > 0 ? L.lslot_out : L.lslot_in;
+    __shared__ int din_deg[kMaxSlots + 1], dout_deg[kMaxSlots + 1];
+    for (int q = threadIdx.x; q < din; q += kThreads) din_deg[q] = SIGN > 0 ? L.lslot_in[q] : L.lslot_out[q];
+    for (int q = threadIdx.x; q < dout; q += kThreads) dout_deg[q] = SIGN > 0 ? L.lslot_out[q] : L.lslot_in[q];
     const EdgeRow R = edge_row(B, perm, dist, p0 + (c < n ? c : n - 1), E);
     if (threadIdx.x < 16) {
         sE[c] = R.e;
@@ -336,8 +362,9 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
     }
     __syncthreads();
     const int per = 16 * dout;
+    const float iper = 1.0f / static_cast<float>(per), idim = 1.0f / static_cast<float>(dout);
     for (int q = threadIdx.x; q < n * per; q += kThreads) {
-        const int ed = q / per, rest = q - ed * per, ch = rest / dout, d = rest - ch * dout;
+        const int ed = quotient(q, iper), rest = q - ed * per, ch = quotient(rest, idim), d = rest - ch * dout;
         if (16 * row + ch < noch) y[(sE[ed] * noch + 16 * row) * dout + rest] = st[d * kSS + ch * 16 + ed];
     }
 }
@@ -356,7 +383,7 @@ __global__ void k_bdm_dr(const float* __restrict__ part, int n, int64_t E, float
 // row's edges): the edges of bin b (weight 1 - t) and of bin b - 1 (weight t) in
 // sorted order, 16 at a time, their indices, bins and powers 64 at a time (one
 // memory latency for four tiles).  Few table rows leave the chip idle (65 rows
-// and 4 tiles: 260 workgroups, 577 us, 232 with eight splits), so the edges
+// and 4 tiles: 260 workgroups, 577 us, 232 with eight splits and 154 with kInFlight), so the edges
 // are then split and the splits' sums added in order (k_bdm_sum).
 constexpr int kMaxU = 8;
 constexpr int kHead = 64;
@@ -369,11 +396,14 @@ k_bdm_table(feq_layout L, Units UT, feq_binning B, int64_t E, const int32_t* __r
     __shared__ float sPow[kHead * (kPow + 1)];
     __shared__ int64_t sE[kHead];
     __shared__ float sW[kHead];
+    __shared__ int sDegI[kMaxSlots + 1], sDegO[kMaxSlots + 1];
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int cin = L.cin, cout = L.cout, din = L.din, dout = L.dout, wd = L.wdim, nb = B.num_bins;
     const int b = blockIdx.x, nci = (cin + 15) / 16, cot = blockIdx.y / nci, cit = blockIdx.y % nci;
     const int split = blockIdx.z % splits;
+    for (int q = threadIdx.x; q < din; q += kThreads) sDegI[q] = L.lslot_in[q];
+    for (int q = threadIdx.x; q < dout; q += kThreads) sDegO[q] = L.lslot_out[q];
     const int u0 = (blockIdx.z / splits) * 4 * kMaxU + wave;
     float* sg = st;
     float* sx = st + dout * kSS;
@@ -401,9 +431,9 @@ k_bdm_table(feq_layout L, Units UT, feq_binning B, int64_t E, const int32_t* __r
             }
             __syncthreads();
         }
-        stage_rows<false>(gy, cout, 16 * cot, dout, sE + head, sPow + head * (kPow + 1), kPow + 1, L.lslot_out, n, sg,
+        stage_rows<false>(gy, cout, 16 * cot, dout, sE + head, sPow + head * (kPow + 1), kPow + 1, sDegO, n, sg,
                           sW + head);
-        stage_rows<false>(x, cin, 16 * cit, din, sE + head, sPow + head * (kPow + 1), kPow + 1, L.lslot_in, n, sx);
+        stage_rows<false>(x, cin, 16 * cit, din, sE + head, sPow + head * (kPow + 1), kPow + 1, sDegI, n, sx);
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < kMaxU; ++u) {
@@ -574,9 +604,9 @@ int bdm_fwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* x
     auto k = P.n <= 16 ? k_bdm_apply<4, false, 1> : k_bdm_apply<kMaxP, false, 1>;
     const size_t lds = sizeof(float) * kSS * (L.din > L.dout ? L.din : L.dout);
     if (int rc = bdm_lds(reinterpret_cast<const void*>(k), lds)) return rc;
-    FEQ_LAUNCH("k_bdm_fwd", k, dim3(static_cast<unsigned>(ceil_div(E, 16)), tiles16(L.cout)), dim3(kThreads), lds, s, L,
+    FEQ_LAUNCH("k_bdm_fwd", k, dim3(static_cast<unsigned>(ceil_div(ceil_div(E, 16), 8) * 8), tiles16(L.cout)), dim3(kThreads), lds, s, L,
                P, B, E, perm, dist, x, L.cin, L.din, L.cout, L.dout, L.wdim, frag, static_cast<const float*>(nullptr), y,
-               static_cast<float*>(nullptr));
+               static_cast<float*>(nullptr), static_cast<unsigned>(ceil_div(E, 16)));
     return FEQ_OK;
 }
 
@@ -596,8 +626,9 @@ int bdm_bwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* g
     const size_t lds = sizeof(float) * kSS * (L.din > L.dout ? L.din : L.dout);
     if (int rc = bdm_lds(reinterpret_cast<const void*>(k), lds)) return rc;
     const int nt = tiles16(L.cin);
-    FEQ_LAUNCH("k_bdm_bwd_x", k, dim3(static_cast<unsigned>(ceil_div(E, 16)), nt), dim3(kThreads), lds, s, L, P, B, E,
-               perm, dist, gy, L.cout, L.dout, L.cin, L.din, L.wdim, frag, x, gx, gpart);
+    FEQ_LAUNCH("k_bdm_bwd_x", k, dim3(static_cast<unsigned>(ceil_div(ceil_div(E, 16), 8) * 8), nt), dim3(kThreads), lds, s,
+               L, P, B, E, perm, dist, gy, L.cout, L.dout, L.cin, L.din, L.wdim, frag, x, gx, gpart,
+               static_cast<unsigned>(ceil_div(E, 16)));
     if (gd)
         FEQ_LAUNCH("k_bdm_dr", k_bdm_dr, dim3(static_cast<unsigned>(ceil_div(E, 256))), dim3(256), 0, s, gpart, nt, E,
                    gdist);
