@@ -427,7 +427,8 @@ extern "C" size_t feq_edgewise_workspace(const feq_layout* L, const feq_binning*
     // dC partials, the per-edge radial-function gradient dF_e and the tail's buffers
     const size_t generic = b ? sizeof(float) * (static_cast<size_t>(groups_for(E)) * ncc + 64 +
                                                 static_cast<size_t>(E) * kw + 64 +
-                                                ew_tail_floats(*b, static_cast<int>(kw), E, groups_for(E), ncc)) + 256
+                                                ew_tail_floats(*b, static_cast<int>(kw), E, groups_for(E), ncc)) + 512 +
+                                   (ew_wave_supported(*L, rank) ? ew_wave_workspace(*L) : 0)
                              : 0;
     const size_t split = b ? ew_split_bwd_workspace(*L, *b, rank, E, false) : 0;
     return generic > split ? generic : split;
@@ -436,7 +437,8 @@ extern "C" size_t feq_edgewise_workspace(const feq_layout* L, const feq_binning*
 extern "C" size_t feq_edgewise_fwd_workspace(const feq_layout* L, const feq_binning*, int32_t rank,
                                              int64_t) {
     if (!L || rank < 1) return 0;
-    return ew_split_workspace(*L, rank) + 256;
+    const size_t split = ew_split_workspace(*L, rank);
+    return split ? split + 256 : ew_wave_supported(*L, rank) ? ew_wave_workspace(*L) + 256 : 256;
 }
 
 extern "C" int feq_edgewise_fwd(const feq_layout* L, const feq_binning* b, int32_t rank,
@@ -455,7 +457,7 @@ extern "C" int feq_edgewise_fwd(const feq_layout* L, const feq_binning* b, int32
         const int rc = ew_split_fwd(*L, *b, rank, E, x, nullptr, 0, P, Q, dist, C, F, y, ws,
                                     ws_bytes, false, stream_of(stream));
         if (rc != -1) return rc;
-        const int rw = ew_wave_fwd(*L, *b, rank, E, x, P, Q, dist, C, F, y, stream_of(stream));
+        const int rw = ew_wave_fwd(*L, *b, rank, E, x, P, Q, dist, C, F, y, ws, ws_bytes, stream_of(stream));
         if (rw != -1) return rw;
     }
     const size_t clds = c_lds(*L, rank, fwd_lds(*L, rank)), lds = fwd_lds(*L, rank) + clds;
@@ -512,7 +514,8 @@ extern "C" int feq_edgewise_bwd(const feq_layout* L, const feq_binning* b, int32
     float* dFe = part + align_up(static_cast<size_t>(G) * ncc, 64);
     float* tail = dFe + align_up(static_cast<size_t>(E) * kw, 64);
     if (wave) {
-        if (int rc = ew_wave_bwd(*L, *b, rank, E, gy, x, P, Q, dist, C, F, gx, dFe, part, s)) return rc;
+        void* patterns = tail + align_up(ew_tail_floats(*b, kw, E, G, ncc), 64);
+        if (int rc = ew_wave_bwd(*L, *b, rank, E, gy, x, P, Q, dist, C, F, gx, dFe, part, patterns, s)) return rc;
         return ew_tail(*L, *b, rank, E, dist, F, dFe, part, ew_wave_groups(*L, E), ncc, gC, gF, gdist, tail, s);
     }
     EwDims D{rank, b->num_bins};

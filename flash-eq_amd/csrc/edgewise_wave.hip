@@ -23,23 +23,26 @@
 // each wave works alone, and x, P, Q and C go from memory to the operands.
 //
 // What bounds them: the float32 matrix cores (a step of 16x16x4 takes 32
-// cycles).  lvals 0..6 x 32 channels take 568 steps forward, 810 for the input
-// gradient and 624 for the pattern gradient per edge, against 30 KB of memory.
-// At 50 000 such edges: 0.71, 1.21 and 0.91 ms (matrix cores busy 55%, 45% and 47%
-// of the time, the vector unit another 15 to 19%, which two waves per SIMD overlap
-// little), where edgewise.hip's vector kernels (a workgroup per edge, every
-// product through LDS) took 7.1 ms forward and 18.3 ms backward; at lvals 0..4 x
-// 32 and 20 000 edges 0.14, 0.23 and 0.18 ms against 1.24 and 3.29.  Reading the
-// operands from memory without the LDS copy of the basis took 1.5, 2.9 and 1.6 ms
-// (requests of 4 rows x 16 scattered columns); loads under lane conditions 1.0, 2.0
-// and 1.0; eight waves of the grid per resident wave, so that each read its tables
-// for two or three edges only, 0.73, 1.23 and 0.91.
+// cycles).  lvals 0..6 x 32 channels take 312 steps and 128 of 16 cycles forward,
+// 554 and 128 for the input gradient and 624 for the pattern gradient per edge,
+// against 30 KB of memory.
+// At 50 000 such edges 0.58, 1.06 and 0.91 ms, where edgewise.hip's vector
+// kernels (a workgroup per edge, every product through LDS) took 7.1 ms forward and
+// 18.3 ms backward; at lvals 0..4 x 32 and 20 000 edges 0.11, 0.20
+// and 0.18 against 1.24 and 3.29.
+// What did not carry: operands from memory without the LDS copy of the basis
+// (1.5, 2.9 and 1.6 ms: requests of 4 rows x 16 scattered columns); loads under lane
+// conditions (1.0, 2.0 and 1.0); float32 steps for the channel mixes too (0.71, 1.21
+// and 0.91: matrix cores busy 55%, 45% and 47% of the time, the vector unit another
+// 15 to 19%, which two waves per SIMD overlap little); Z_k summed over the channel
+// tiles (2% faster, errors 5% larger: one chain instead of two).
 #include "feq_internal.h"
 
 namespace feq {
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
 constexpr int kMaxNB = 4;       // 16-slot blocks
 constexpr int kMaxCT = 4;       // 16-channel tiles
@@ -70,6 +73,111 @@ __device__ __forceinline__ int lane_id() {
     int lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane));
     return lane;
+}
+
+// The channel mixes (G_k and H_k, a third to a half of the float32 steps) run on
+// the fp16 matrix cores with split operands, as edgewise_split.hip's: a = 2^-e (hi
+// + lo), e from the largest magnitude (in [2^14, 2^15) after scaling), a product as
+// lo lo + hi lo + lo hi + hi hi with float32 accumulation.  All four: the errors
+// against float64 (geometric mean over every output, five layouts, five seeds) are
+// 3.87e-7, 3.90e-7 with float32 steps and 3.97e-7 without lo lo (the vector kernels
+// 3.94e-7).  Two 16-channel tiles make one 32-step: lane group g holds the reduction
+// indices 4 g + r of both, in the order of the float32 registers, so the halves are
+// converted in place.  16x16x32 takes 16 cycles, four of them 64 against 256.
+__device__ __forceinline__ v4f mfma_h(h8 a, h8 b, v4f c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ int scale_exp(float m) {
+    int e = 141 - static_cast<int>((__float_as_uint(m) >> 23) & 0xffu);
+    e = e < -113 ? -113 : e;
+    return e > 126 ? 126 : e;
+}
+__device__ __forceinline__ float exp2i(int e) { return __uint_as_float(static_cast<unsigned>(e + 127) << 23); }
+__device__ __forceinline__ float max4(float m, const v4f& v) {
+    return fmaxf(fmaxf(m, fmaxf(fabsf(v[0]), fabsf(v[1]))), fmaxf(fabsf(v[2]), fabsf(v[3])));
+}
+struct Halves {
+    h8 hi, lo;
+};
+__device__ __forceinline__ Halves split8(const v4f& a, const v4f& b, float sc) {
+    Halves h;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float v = j < 4 ? a[j & 3] : b[j & 3];
+        h.hi[j] = static_cast<_Float16>(__builtin_fmaf(v, sc, 0.0f));
+        h.lo[j] = static_cast<_Float16>(__builtin_fmaf(v, sc, -static_cast<float>(h.hi[j])));
+    }
+    return h;
+}
+// Tiles of one operand, split with one scale for the wave; e: its exponent.
+template <int CT, int NB>
+struct SplitTiles {
+    Halves t[(CT + 1) / 2][NB];
+    int e;
+};
+template <int CT, int NB>
+__device__ __forceinline__ void split_tiles(const v4f (&v)[CT][NB], SplitTiles<CT, NB>& S) {
+    float m = 0.0f;
+#pragma unroll
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) m = max4(m, v[t][b]);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+    S.e = scale_exp(m);
+    const float sc = exp2i(S.e);
+    const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int h = 0; h < (CT + 1) / 2; ++h)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+            S.t[h][b] = split8(v[2 * h][b], 2 * h + 1 < CT ? v[2 * h + 1 < CT ? 2 * h + 1 : 0][b] : zero, sc);
+}
+// The patterns in operand order, split once per call by k_ewg_prep: for rank k and
+// column tile c0 / 16, the halves of the reduction tiles' pairs, one scale per
+// column (exponents at the end).  (Split by every wave for every edge, they took a
+// third of the vector instructions at lvals 0..4 x 32.)
+struct Patterns {
+    const Halves* frag;     // [rank][column tile][pair][lane]
+    const int* exps;        // [rank][column tile][16]
+    int ncol;               // column tiles
+};
+template <int CT>
+struct Mixer {
+    Halves q[(CT + 1) / 2];
+    int e;
+};
+template <int CT>
+__device__ __forceinline__ void load_mixer(const Patterns& W, int k, int col, Mixer<CT>& M) {
+    constexpr int NH = (CT + 1) / 2;
+    const unsigned lane = lane_id();
+    const Halves* f = W.frag + (k * W.ncol + col) * NH * 64;
+#pragma unroll
+    for (int h = 0; h < NH; ++h) M.q[h] = f[64 * h + lane];
+    M.e = W.exps[(k * W.ncol + col) * 16 + (lane & 15)];
+}
+// out[b] (rows: the tiles' positions, columns: the patterns' channels) =
+// sum over channels of the tiles and the patterns.
+template <int CT, int NB>
+__device__ __forceinline__ void mix_channels(const SplitTiles<CT, NB>& S, const Mixer<CT>& M, v4f (&out)[NB]) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) out[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int h = 0; h < (CT + 1) / 2; ++h) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) out[b] = mfma_h(S.t[h][b].lo, M.q[h].lo, out[b]);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) out[b] = mfma_h(S.t[h][b].hi, M.q[h].lo, out[b]);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) out[b] = mfma_h(S.t[h][b].lo, M.q[h].hi, out[b]);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) out[b] = mfma_h(S.t[h][b].hi, M.q[h].hi, out[b]);
+    }
+    const int back = -(M.e + S.e);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[b][r] = __builtin_amdgcn_ldexpf(out[b][r], back);
 }
 
 // Orders a wave's LDS writes before its later reads by other lanes (LDS
@@ -347,6 +455,28 @@ __device__ __forceinline__ v4f load_c(const float* __restrict__ Ck, int co0, int
     return v;
 }
 
+// One wave per (rank, column tile): columns co and reduction ci, or BWD the other
+// way round.
+template <bool BWD>
+__global__ void __launch_bounds__(64)
+k_ewg_prep(const float* __restrict__ C, int cout, int cin, Halves* __restrict__ frag, int* __restrict__ exps) {
+    const int lane = threadIdx.x, k = blockIdx.x, col = blockIdx.y, ncol = gridDim.y;
+    const int ct = ((BWD ? cout : cin) + 15) / 16, nh = (ct + 1) / 2;
+    const float* Ck = C + static_cast<int64_t>(k) * cout * cin;
+    auto tile = [&](int t) {
+        return BWD ? load_c<true>(Ck, 16 * t, 16 * col, cout, cin) : load_c<false>(Ck, 16 * col, 16 * t, cout, cin);
+    };
+    float m = 0.0f;
+    for (int t = 0; t < ct; ++t) m = max4(m, tile(t));
+    m = fmaxf(m, __shfl_xor(m, 16, 64));
+    m = fmaxf(m, __shfl_xor(m, 32, 64));
+    const int e = scale_exp(m);
+    const float sc = exp2i(e);
+    for (int h = 0; h < nh; ++h)
+        frag[((k * ncol + col) * nh + h) * 64 + lane] = split8(tile(2 * h), tile(2 * h + 1), sc);
+    if (lane < 16) exps[(k * ncol + col) * 16 + lane] = e;
+}
+
 // Workgroups per CU: what the registers allow without (much) spilling.  The grids
 // are one such set of workgroups, each wave taking every (grid * 4)-th edge: its
 // tables are read once.
@@ -357,7 +487,7 @@ constexpr int bwd_x_groups(int nb) { return nb == 1 ? 3 : 2; }
 template <int CT, int NB>
 __global__ void __launch_bounds__(256, fwd_groups(CT, NB))
 k_ewg_fwd(GenTab T, feq_binning B, int64_t E, const float* __restrict__ x, const float* __restrict__ P,
-          const float* __restrict__ Q, const float* __restrict__ dist, const float* __restrict__ C,
+          const float* __restrict__ Q, const float* __restrict__ dist, Patterns W,
           const float* __restrict__ F, float* __restrict__ y) {
     extern __shared__ float sm[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -383,31 +513,22 @@ k_ewg_fwd(GenTab T, feq_binning B, int64_t E, const float* __restrict__ x, const
             stage_basis<NB>(P + e * din * din, din, sB, [&] { edge_weights(T, B, dist[e], F, sFe, deg); });
         }
         rotate_in<CT, NB, false>(x + e * cin * din, 0, cin, sB, din, in_col, fs);
+        SplitTiles<CT, NB> S;
+        split_tiles<CT, NB>(fs, S);
         if (Q != P) stage_basis<NB>(Q + e * dout * dout, dout, sB, [] {});
         for (int co0 = 0; co0 < cout; co0 += 16) {
             v4f m[NB];
 #pragma unroll
             for (int b = 0; b < NB; ++b) m[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
             // the patterns one rank ahead: the products cover their latency
-            v4f cv[CT], cn[CT];
-#pragma unroll
-            for (int t = 0; t < CT; ++t) cv[t] = load_c<false>(C, co0, 16 * t, cout, cin);
+            Mixer<CT> M, next;
+            load_mixer<CT>(W, 0, co0 / 16, M);
 #pragma unroll 1
             for (int k = 0; k < kRank; ++k) {
-                const float* Cn = C + static_cast<int64_t>(k + 1 < kRank ? k + 1 : k) * cout * cin;
                 v4f G[NB];
-#pragma unroll
-                for (int t = 0; t < CT; ++t) cn[t] = load_c<false>(Cn, co0, 16 * t, cout, cin);
-#pragma unroll
-                for (int b = 0; b < NB; ++b) G[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int t = 0; t < CT; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-#pragma unroll
-                        for (int b = 0; b < NB; ++b) G[b] = mfma4(fs[t][b][r], cv[t][r], G[b]);
-#pragma unroll
-                for (int t = 0; t < CT; ++t) cv[t] = cn[t];
+                load_mixer<CT>(W, k + 1 < kRank ? k + 1 : k, co0 / 16, next);
+                mix_channels<CT, NB>(S, M, G);
+                M = next;
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -432,10 +553,10 @@ template <int CT, int NB>
 __global__ void __launch_bounds__(256, bwd_x_groups(NB))
 k_ewg_bwd_x(GenTab T, feq_binning B, int64_t E, const float* __restrict__ gy, const float* __restrict__ x,
             const float* __restrict__ P, const float* __restrict__ Q, const float* __restrict__ dist,
-            const float* __restrict__ C, const float* __restrict__ F, float* __restrict__ gx,
+            Patterns W, const float* __restrict__ F, float* __restrict__ gx,
             float* __restrict__ dFe) {
     extern __shared__ float sm[];
-    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int cin = T.cin, cout = T.cout, din = T.din, dout = T.dout, wd = T.wd, last = T.last;
     float* sB = sm + wave * bwd_x_floats(wd, din, dout, NB);
@@ -459,6 +580,24 @@ k_ewg_bwd_x(GenTab T, feq_binning B, int64_t E, const float* __restrict__ gy, co
     for (int64_t e = first; e < E; e += step) {
         v4f gd[CT][NB];
         float dF[kRank][kMaxW / 64] = {};   // of the weights lane + 64 j
+        // a weight's gradient from the tiles: its one (m = 0) or two entries
+        auto weights_of = [&](const v4f (&Z)[NB], float (&d)[kMaxW / 64]) {
+            const int ln = lane_id(), c = ln & 15, g = ln >> 4;
+            wave_sync();
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sT[(16 * b + 4 * g + r) * kZS + c] = Z[b][r];
+            wave_sync();
+#pragma unroll
+            for (int j = 0; j < kMaxW / 64; ++j)
+                if (64 * j < wd) {
+                    const float u = sT[(pos[j] >> 16) & 0x3fff];
+                    float v = sT[pos[j] & 0x3fff];
+                    v += pos[j] < 0 ? 0.0f : pos[j] & 0x40000000 ? -u : u;
+                    d[j] += v;
+                }
+        };
         if constexpr (ahead(NB)) {
             edge_weights(T, B, dist[e], F, sFe, deg);
             stage_end<NB>(Q + e * dout * dout, dout * dout, st, sB);
@@ -467,32 +606,26 @@ k_ewg_bwd_x(GenTab T, feq_binning B, int64_t E, const float* __restrict__ gy, co
             stage_basis<NB>(Q + e * dout * dout, dout, sB, [&] { edge_weights(T, B, dist[e], F, sFe, deg); });
         }
         rotate_in<CT, NB, false>(gy + e * cout * dout, 0, cout, sB, dout, out_col, gd);
+        SplitTiles<CT, NB> S;
+        split_tiles<CT, NB>(gd, S);
         if (Q != P) stage_basis<NB>(P + e * din * din, din, sB, [] {});
         for (int ci0 = 0; ci0 < cin; ci0 += 16) {
             v4f fs[1][NB], dfs[NB];
             rotate_in<1, NB, false>(x + e * cin * din, ci0, cin, sB, din, in_col, fs);
 #pragma unroll
             for (int b = 0; b < NB; ++b) dfs[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-            v4f cv[CT], cn[CT];     // the patterns one rank ahead
-#pragma unroll
-            for (int t = 0; t < CT; ++t) cv[t] = load_c<true>(C, 16 * t, ci0, cout, cin);
+            Mixer<CT> M, next;      // the patterns one rank ahead
+            load_mixer<CT>(W, 0, ci0 / 16, M);
 #pragma unroll
             for (int k = 0; k < kRank; ++k) {
-                const float* Cn = C + static_cast<int64_t>(k + 1 < kRank ? k + 1 : k) * cout * cin;
-#pragma unroll
-                for (int t = 0; t < CT; ++t) cn[t] = load_c<true>(Cn, 16 * t, ci0, cout, cin);
+                load_mixer<CT>(W, k + 1 < kRank ? k + 1 : k, ci0 / 16, next);
                 const float* sFk = sFe + k * (wd + 1);
-                v4f H[NB], Z[NB];
+                v4f H[NB];
+                v4f Z[NB];
 #pragma unroll
-                for (int b = 0; b < NB; ++b) H[b] = Z[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int t = 0; t < CT; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-#pragma unroll
-                        for (int b = 0; b < NB; ++b) H[b] = mfma4(gd[t][b][r], cv[t][r], H[b]);
-#pragma unroll
-                for (int t = 0; t < CT; ++t) cv[t] = cn[t];
+                for (int b = 0; b < NB; ++b) Z[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+                mix_channels<CT, NB>(S, M, H);
+                M = next;
                 const int ln = lane_id(), c = ln & 15, g = ln >> 4;
                 wave_sync();    // the previous rank's reads
 #pragma unroll
@@ -511,21 +644,7 @@ k_ewg_bwd_x(GenTab T, feq_binning B, int64_t E, const float* __restrict__ gy, co
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
                         if (b < NB - 1 || r < last) dfs[b] = mfma4(coef(sFk, code[b], r), H[b][r], dfs[b]);
-                wave_sync();
-#pragma unroll
-                for (int b = 0; b < NB; ++b)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) sT[(16 * b + 4 * g + r) * kZS + c] = Z[b][r];
-                wave_sync();
-                // a weight's gradient: its one (m = 0) or two entries of the tiles
-#pragma unroll
-                for (int j = 0; j < kMaxW / 64; ++j)
-                    if (64 * j < wd) {
-                        const float u = sT[(pos[j] >> 16) & 0x3fff];
-                        float v = sT[pos[j] & 0x3fff];
-                        v += pos[j] < 0 ? 0.0f : pos[j] & 0x40000000 ? -u : u;
-                        dF[k][j] += v;
-                    }
+                weights_of(Z, dF[k]);
             }
             rotate_out<NB>(dfs, sB, din, last, in_red, gx + e * cin * din, ci0 / 16, cin);
         }
@@ -651,6 +770,7 @@ k_ewg_bwd_c(GenTab T, feq_binning B, int64_t E, int ncot, int subs, const float*
 // group first); 0 when they do not fit kMaxNB.  Slot q of a block takes row
 // 4 (q % 4) + q / 4: n slots then need ceil(n / 4) reduction steps.
 int build_tab(const feq_layout& L, GenTab& T) {
+    if (L.nblocks < 1 || L.nblocks > FEQ_MAX_BLOCKS || L.din < 1 || L.dout < 1 || L.cin < 1 || L.cout < 1) return 0;
     // the staged basis: four waves in a workgroup's LDS
     if (bwd_x_floats(L.wdim, L.din, L.dout, kMaxNB) > 160 * 1024 / 16) return 0;
     if (L.wdim > kMaxW || L.cin > 16 * kMaxCT || L.cout > 16 * kMaxCT || L.wdim < 1) return 0;
@@ -734,13 +854,34 @@ int ew_wave_groups(const feq_layout& L, int64_t E) {
     return static_cast<int>(n < 512 ? n : 512);
 }
 
+// The split patterns: fragments of the wider of the two forms, and the exponents.
+size_t ew_wave_workspace(const feq_layout& L) {
+    const int ci = tiles(L.cin), co = tiles(L.cout);
+    const int frags = kRank * (co * ((ci + 1) / 2) > ci * ((co + 1) / 2) ? co * ((ci + 1) / 2) : ci * ((co + 1) / 2));
+    return frags * 64 * sizeof(Halves) + sizeof(int) * kRank * 16 * (ci > co ? ci : co) + 256;
+}
+
+template <bool BWD>
+static int prep(const feq_layout& L, const float* C, void* ws, Patterns& W, hipStream_t s) {
+    const int ci = tiles(L.cin), co = tiles(L.cout), ncol = BWD ? ci : co, nh = ((BWD ? co : ci) + 1) / 2;
+    Halves* frag = reinterpret_cast<Halves*>(align_up(reinterpret_cast<uintptr_t>(ws), 32));
+    int* exps = reinterpret_cast<int*>(frag + kRank * ncol * nh * 64);
+    W = Patterns{frag, exps, ncol};
+    auto k = k_ewg_prep<BWD>;
+    FEQ_LAUNCH("k_ewg_prep", k, dim3(kRank, ncol), dim3(64), 0, s, C, L.cout, L.cin, frag, exps);
+    return FEQ_OK;
+}
+
 int ew_wave_fwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, const float* x, const float* P,
-                const float* Q, const float* dist, const float* C, const float* F, float* y, hipStream_t s) {
+                const float* Q, const float* dist, const float* C, const float* F, float* y, void* ws,
+                size_t ws_bytes, hipStream_t s) {
     GenTab T;
     if (rank != kRank) return -1;
     const int nb = build_tab(L, T), ct = tiles(L.cin);
-    if (!nb) return -1;
-    void (*kern)(GenTab, feq_binning, int64_t, const float*, const float*, const float*, const float*, const float*,
+    if (!nb || !ws || ws_bytes < ew_wave_workspace(L)) return -1;
+    Patterns W;
+    if (int rc = prep<false>(L, C, ws, W, s)) return rc;
+    void (*kern)(GenTab, feq_binning, int64_t, const float*, const float*, const float*, const float*, Patterns,
                  const float*, float*) = nullptr;
 #define FEQ_PICK(c, n) if (ct == c && nb == n) kern = k_ewg_fwd<c, n>;
     FEQ_EWG_SHAPES(FEQ_PICK)
@@ -749,19 +890,21 @@ int ew_wave_fwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, 
     const dim3 grid(static_cast<unsigned>(wgs < most ? wgs : most));
     const size_t lds = 4 * sizeof(float) * wave_floats(L.wdim, L.din, L.dout);
     if (int rc = set_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
-    FEQ_LAUNCH("k_ewg_fwd", kern, grid, dim3(256), lds, s, T, B, E, x, P, Q, dist, C, F, y);
+    FEQ_LAUNCH("k_ewg_fwd", kern, grid, dim3(256), lds, s, T, B, E, x, P, Q, dist, W, F, y);
     return FEQ_OK;
 }
 
 int ew_wave_bwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, const float* gy, const float* x,
                 const float* P, const float* Q, const float* dist, const float* C, const float* F, float* gx,
-                float* dFe, float* dC_part, hipStream_t s) {
+                float* dFe, float* dC_part, void* ws, hipStream_t s) {
     GenTab T;
     if (rank != kRank) return -1;
     const int nb = build_tab(L, T), cti = tiles(L.cin), cto = tiles(L.cout);
     if (!nb) return -1;
+    Patterns W;
+    if (int rc = prep<true>(L, C, ws, W, s)) return rc;
     void (*kx)(GenTab, feq_binning, int64_t, const float*, const float*, const float*, const float*, const float*,
-               const float*, const float*, float*, float*) = nullptr;
+               Patterns, const float*, float*, float*) = nullptr;
     void (*kc)(GenTab, feq_binning, int64_t, int, int, const float*, const float*, const float*, const float*,
                const float*, const float*, float*) = nullptr;
 #define FEQ_PICK(c, n)                               \
@@ -773,7 +916,7 @@ int ew_wave_bwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, 
     const dim3 grid(static_cast<unsigned>(wgs < most ? wgs : most));
     const size_t lds = 4 * sizeof(float) * bwd_x_floats(L.wdim, L.din, L.dout, nb);
     if (int rc = set_lds(reinterpret_cast<const void*>(kx), lds)) return rc;
-    FEQ_LAUNCH("k_ewg_bwd_x", kx, grid, dim3(256), lds, s, T, B, E, gy, x, P, Q, dist, C, F, gx, dFe);
+    FEQ_LAUNCH("k_ewg_bwd_x", kx, grid, dim3(256), lds, s, T, B, E, gy, x, P, Q, dist, W, F, gx, dFe);
     const int subs = 4 / cto, waves = subs * cto;
     const size_t sums = sizeof(float) * static_cast<size_t>(cto) * kRank * cti * 4 * 64;
     const size_t fe = sizeof(float) * waves * wave_floats(L.wdim, L.din, L.dout), clds = fe > sums ? fe : sums;

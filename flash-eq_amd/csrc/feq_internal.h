@@ -217,11 +217,13 @@ int bdm_bwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* g
 // writes dF_e and ew_wave_groups(L, E) partials of dC for ew_tail.
 bool ew_wave_supported(const feq_layout& L, int rank);
 int ew_wave_groups(const feq_layout& L, int64_t E);
+size_t ew_wave_workspace(const feq_layout& L);
 int ew_wave_fwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, const float* x, const float* P,
-                const float* Q, const float* dist, const float* C, const float* F, float* y, hipStream_t s);
+                const float* Q, const float* dist, const float* C, const float* F, float* y, void* ws,
+                size_t ws_bytes, hipStream_t s);
 int ew_wave_bwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, const float* gy, const float* x,
                 const float* P, const float* Q, const float* dist, const float* C, const float* F, float* gx,
-                float* dFe, float* dC_part, hipStream_t s);
+                float* dFe, float* dC_part, void* ws, hipStream_t s);
 
 // Kernel family of the fused edgewise layer.  The default tries the split-fp16
 // kernels, then the wave-per-edge ones, then the shape-generic ones; FEQ_EW_PATH=generic (or
