@@ -1,6 +1,6 @@
 // The closed form of one column of a Wigner-D basis and of its gradient, and the
 // edge frame (see wigner.hip): shared by the kernels of wigner.hip (degrees up to
-// kLaneL) and wigner_high.hip (the rest).
+// kLaneL) and wigner_high.h (the rest).
 #pragma once
 
 #include "feq_internal.h"
@@ -19,7 +19,7 @@ struct WignerArgs {
     int32_t plan_off[FEQ_MAX_IRREPS];  // offset of every irrep's plan block (doubles)
 };
 
-// The other form (wigner_high.hip).
+// The other form (wigner_high.h).
 constexpr int kLaneL = 6;
 template <class T>
 int wigner_high_fwd(const WignerArgs& A, const double* plan, const int32_t* perm, int64_t E, const T* dirs, T* out,
