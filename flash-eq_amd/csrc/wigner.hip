@@ -288,6 +288,7 @@ int wigner_fwd(const int32_t* lvals, int32_t n, const double* plan, const int32_
     if (E < 0) return fail(FEQ_ERR_INVALID, "negative edge count");
     if (E == 0) return FEQ_OK;
     if (!plan || !perm || !dirs || !out) return fail(FEQ_ERR_INVALID, "NULL pointer");
+    if (int rc = check_dim<T>(A)) return rc;
     size_t lds;
     if (lane_form(A, E))
         return with_lane_lmax(A, [&](auto LL) -> int {
@@ -312,6 +313,7 @@ int wigner_bwd(const int32_t* lvals, int32_t n, const double* plan, const int32_
     if (E < 0) return fail(FEQ_ERR_INVALID, "negative edge count");
     if (E == 0) return FEQ_OK;
     if (!plan || !perm || !dirs || !grad_out || !grad_dirs) return fail(FEQ_ERR_INVALID, "NULL pointer");
+    if (int rc = check_dim<T>(A)) return rc;
     size_t lds;
     if (lane_form(A, E))
         return with_lane_lmax(A, [&](auto LL) -> int {

@@ -128,16 +128,14 @@ int with_lmax(const WignerArgs& A, Fn&& f) {
 }
 
 // Edges per workgroup: one thread per (edge, column), the edges' matrices
-// (dim x dim values of T) staged in at most 64 KB of LDS.
+// (dim x dim values of T, see check_dim) staged in at most 64 KB of LDS.
 template <class T>
-int wigner_epb(int dim, int* epb, size_t* lds) {
-    int e = 256 / dim;
-    const int cap = static_cast<int>((64 * 1024) / (sizeof(T) * static_cast<size_t>(dim) * dim));
-    e = e < cap ? e : cap;
-    if (e < 1) return fail(FEQ_ERR_UNSUPPORTED, "representation dimension %d too large", dim);
-    *epb = e;
-    *lds = sizeof(T) * static_cast<size_t>(e) * dim * dim;
-    return FEQ_OK;
+int wigner_epb(int dim, size_t* lds) {
+    const int e = 256 / dim;
+    const int cap = static_cast<int>(kMatrixBytes / (sizeof(T) * static_cast<size_t>(dim) * dim));
+    const int epb = e < cap ? e : cap;
+    *lds = sizeof(T) * static_cast<size_t>(epb) * dim * dim;
+    return epb;
 }
 
 }  // namespace
@@ -145,9 +143,8 @@ int wigner_epb(int dim, int* epb, size_t* lds) {
 template <class T>
 int wigner_high_fwd(const WignerArgs& A, const double* plan, const int32_t* perm, int64_t E, const T* dirs, T* out,
                     hipStream_t s) {
-    int epb;
     size_t lds;
-    if (int rc = wigner_epb<T>(A.dim, &epb, &lds)) return rc;
+    const int epb = wigner_epb<T>(A.dim, &lds);
     return with_lmax(A, [&](auto LL) -> int {
         auto kern = k_wigner<decltype(LL)::value, T>;
         FEQ_LAUNCH("k_wigner", kern, dim3(ceil_div(E, epb)), dim3(256), lds, s, A, epb, plan, perm, E, dirs, out);
@@ -158,9 +155,8 @@ int wigner_high_fwd(const WignerArgs& A, const double* plan, const int32_t* perm
 template <class T>
 int wigner_high_bwd(const WignerArgs& A, const double* plan, const int32_t* perm, int64_t E, const T* dirs,
                     const T* grad_out, T* grad_dirs, hipStream_t s) {
-    int epb;
     size_t lds;
-    if (int rc = wigner_epb<T>(A.dim, &epb, &lds)) return rc;
+    const int epb = wigner_epb<T>(A.dim, &lds);
     return with_lmax(A, [&](auto LL) -> int {
         auto kern = k_wigner_bwd<decltype(LL)::value, T>;
         FEQ_LAUNCH("k_wigner_bwd", kern, dim3(ceil_div(E, epb)), dim3(256), lds, s, A, epb, plan, perm, E, dirs,

@@ -44,6 +44,18 @@ inline bool lane_form(const WignerArgs& A, int64_t E) {
     return l <= 4 || (l <= kLaneL && E > kColumnEdges);
 }
 
+// Representations whose matrix exceeds 64 KB are refused (dimensions over 128 in
+// float32, 90 in float64), whatever kernel the call would take: the column kernel
+// stages whole matrices, and every kernel holds perm in FEQ_MAX_SLOTS entries.
+constexpr size_t kMatrixBytes = 64 * 1024;
+template <class T>
+int check_dim(const WignerArgs& A) {
+    static_assert(kMatrixBytes / sizeof(float) <= FEQ_MAX_SLOTS * FEQ_MAX_SLOTS, "perm's LDS copy");
+    if (sizeof(T) * static_cast<size_t>(A.dim) * A.dim > kMatrixBytes)
+        return fail(FEQ_ERR_UNSUPPORTED, "representation dimension %d too large", A.dim);
+    return FEQ_OK;
+}
+
 namespace {
 
 // nan_to_num(x, 0.0) in the output type: NaN -> 0, +-inf -> +-max

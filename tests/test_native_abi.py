@@ -186,3 +186,19 @@ def test_sum_tables_argument_checks():
     assert lib.feq_sum_tables(ptrs, 17, 10, ctypes.c_void_p(256), None) != 0
     assert lib.feq_sum_tables(ptrs, 2, 10, ctypes.c_void_p(256), None) != 0
     assert "NULL table" in lib.feq_last_error().decode()
+
+
+@pytest.mark.parametrize("suffix,lvals", [("", [4] * 15), ("", [2] * 26), ("", [6] * 10), ("_f64", [4] * 11),
+                                          ("_f64", [6] * 7), ("_f64", [1] * 31)])
+def test_wigner_dimension_limit(suffix, lvals):
+    """feq_wigner_basis*: a representation whose matrix exceeds 64 KB (dimensions over 128 in
+    float32, 90 in float64) is refused before any launch, for every kernel form, that is at few
+    and at many edges, and accepted without edges (nothing to do)."""
+    lib = N.load_library()
+    one = ctypes.c_void_p(256)          # never dereferenced: the check fails first
+    lv = (ctypes.c_int32 * len(lvals))(*lvals)
+    for E in (1, 1000, 2000, 40000):
+        for rc in (getattr(lib, "feq_wigner_basis" + suffix)(lv, len(lvals), one, one, E, one, one, None),
+                   getattr(lib, "feq_wigner_basis_bwd" + suffix)(lv, len(lvals), one, one, E, one, one, one, None)):
+            assert rc != 0 and "too large" in lib.feq_last_error().decode(), (E, rc, lib.feq_last_error())
+    assert getattr(lib, "feq_wigner_basis" + suffix)(lv, len(lvals), one, one, 0, None, None, None) == 0
