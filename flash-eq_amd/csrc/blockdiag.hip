@@ -14,7 +14,7 @@
 // contributions of the edges in bins b (weight 1 - t) and b - 1 (weight t) in a
 // fixed order: no atomics, every row written, the same bits on every run.
 // Distance gradient: one workgroup per edge, a fixed-order workgroup sum.
-#include "feq_internal.h"
+#include "blockdiag_edge.h"
 
 #include <type_traits>
 
@@ -22,76 +22,6 @@ namespace feq {
 namespace {
 
 constexpr int kThreads = 256;
-
-struct SlotRef {
-    int blk;  // m-block index, -1 when the slot has no partner block
-    int o;    // index inside the block
-    int c;    // 0 = +m (re) component, 1 = -m (im)
-};
-
-__device__ __forceinline__ SlotRef find_out_slot(const feq_layout& L, int slot) {
-    for (int k = 0; k < L.nblocks; ++k) {
-        const int m = L.blk[k][0], no = L.blk[k][2], off = L.blk[k][4];
-        const int w = m == 0 ? 1 : 2;
-        if (slot >= off && slot < off + w * no) {
-            const int rel = slot - off;
-            return {k, rel / w, rel % w};
-        }
-    }
-    return {-1, 0, 0};
-}
-
-__device__ __forceinline__ SlotRef find_in_slot(const feq_layout& L, int slot) {
-    for (int k = 0; k < L.nblocks; ++k) {
-        const int m = L.blk[k][0], ni = L.blk[k][1], off = L.blk[k][3];
-        const int w = m == 0 ? 1 : 2;
-        if (slot >= off && slot < off + w * ni) {
-            const int rel = slot - off;
-            return {k, rel / w, rel % w};
-        }
-    }
-    return {-1, 0, 0};
-}
-
-template <class T>
-__device__ __forceinline__ T lerp_t(T lo, T hi, T t) {
-    return lo + t * (hi - lo);
-}
-
-// Weight w's place in the layout: input slot (the +m slot of a pair), output
-// slot, degree sum and the component (0: a, 1: b of the 2x2 block; m = 0: -1).
-struct WeightRef {
-    int is, os, lsum, comp;
-};
-
-__device__ __forceinline__ WeightRef weight_ref(const feq_layout& L, int w) {
-    int k = L.nblocks - 1;
-    while (k > 0 && w < L.blk[k][5]) --k;
-    const int m = L.blk[k][0], ni = L.blk[k][1];
-    const int in_off = L.blk[k][3], out_off = L.blk[k][4], w_off = L.blk[k][5];
-    const int rel = w - w_off;
-    WeightRef r;
-    if (m == 0) {
-        r.is = in_off + rel % ni;
-        r.os = out_off + rel / ni;
-        r.comp = -1;
-    } else {
-        const int pair = rel >> 1;
-        r.is = in_off + 2 * (pair % ni);
-        r.os = out_off + 2 * (pair / ni);
-        r.comp = rel & 1;
-    }
-    r.lsum = L.lslot_in[r.is] + L.lslot_out[r.os];
-    return r;
-}
-
-// d y / d T for one weight, before the solid-harmonic factor (block_diagonal.cu:514-517)
-template <class T>
-__device__ __forceinline__ T weight_grad(const WeightRef& r, const T* xr, const T* gr) {
-    if (r.comp < 0) return xr[r.is] * gr[r.os];
-    const T fr = xr[r.is], fi = xr[r.is + 1], g_r = gr[r.os], g_i = gr[r.os + 1];
-    return r.comp == 0 ? fr * g_r + fi * g_i : fi * g_r - fr * g_i;
-}
 
 template <class T>
 __global__ void __launch_bounds__(kThreads)
@@ -110,38 +40,8 @@ k_bd_fwd(feq_layout L, feq_binning B, const T* __restrict__ x, const T* __restri
     const int64_t tstride = static_cast<int64_t>(cout) * cin * wd;
     const T* tlo = table + eb.lo * tstride;
     const T* thi = tlo + tstride;
-    for (int q = threadIdx.x; q < cout * dout; q += kThreads) {
-        const int co = q / dout, slot = q % dout;
-        const SlotRef s = find_out_slot(L, slot);
-        T acc = T(0);
-        if (s.blk >= 0) {
-            const int m = L.blk[s.blk][0], ni = L.blk[s.blk][1];
-            const int in_off = L.blk[s.blk][3], w_off = L.blk[s.blk][5];
-            const int lo_l = L.lslot_out[slot];
-            for (int i = 0; i < ni; ++i) {
-                const int islot = in_off + (m == 0 ? i : 2 * i);
-                const T sc = ipow_t<T>(sw, lo_l + L.lslot_in[islot]);
-                const int64_t wb = static_cast<int64_t>(co) * cin * wd;
-                if (m == 0) {
-                    const int w = w_off + s.o * ni + i;
-                    for (int ci = 0; ci < cin; ++ci) {
-                        const int64_t a = wb + static_cast<int64_t>(ci) * wd + w;
-                        acc += lerp_t<T>(tlo[a], thi[a], t) * sc * sx[ci * din + islot];
-                    }
-                } else {
-                    const int w = w_off + 2 * (s.o * ni + i);
-                    for (int ci = 0; ci < cin; ++ci) {
-                        const int64_t a = wb + static_cast<int64_t>(ci) * wd + w;
-                        const T wa = lerp_t<T>(tlo[a], thi[a], t) * sc;
-                        const T wb2 = lerp_t<T>(tlo[a + 1], thi[a + 1], t) * sc;
-                        const T fr = sx[ci * din + islot], fi = sx[ci * din + islot + 1];
-                        acc += s.c == 0 ? (wa * fr + wb2 * fi) : (wa * fi - wb2 * fr);
-                    }
-                }
-            }
-        }
-        y[e * cout * dout + q] = acc;
-    }
+    for (int q = threadIdx.x; q < cout * dout; q += kThreads)
+        y[e * cout * dout + q] = out_entry<T>(L, sx, q / dout, q % dout, tlo, thi, t, sw);
 }
 
 template <class T>
@@ -161,37 +61,8 @@ k_bd_bwd_x(feq_layout L, feq_binning B, const T* __restrict__ gy, const T* __res
     const int64_t tstride = static_cast<int64_t>(cout) * cin * wd;
     const T* tlo = table + eb.lo * tstride;
     const T* thi = tlo + tstride;
-    for (int q = threadIdx.x; q < cin * din; q += kThreads) {
-        const int ci = q / din, slot = q % din;
-        const SlotRef s = find_in_slot(L, slot);
-        T acc = T(0);
-        if (s.blk >= 0) {
-            const int m = L.blk[s.blk][0], ni = L.blk[s.blk][1], no = L.blk[s.blk][2];
-            const int out_off = L.blk[s.blk][4], w_off = L.blk[s.blk][5];
-            const int li = L.lslot_in[slot];
-            for (int o = 0; o < no; ++o) {
-                const int oslot = out_off + (m == 0 ? o : 2 * o);
-                const T sc = ipow_t<T>(sw, li + L.lslot_out[oslot]);
-                if (m == 0) {
-                    const int w = w_off + o * ni + s.o;
-                    for (int co = 0; co < cout; ++co) {
-                        const int64_t a = (static_cast<int64_t>(co) * cin + ci) * wd + w;
-                        acc += lerp_t<T>(tlo[a], thi[a], t) * sc * sg[co * dout + oslot];
-                    }
-                } else {
-                    const int w = w_off + 2 * (o * ni + s.o);
-                    for (int co = 0; co < cout; ++co) {
-                        const int64_t a = (static_cast<int64_t>(co) * cin + ci) * wd + w;
-                        const T wa = lerp_t<T>(tlo[a], thi[a], t) * sc;
-                        const T wb2 = lerp_t<T>(tlo[a + 1], thi[a + 1], t) * sc;
-                        const T gr = sg[co * dout + oslot], gi = sg[co * dout + oslot + 1];
-                        acc += s.c == 0 ? (wa * gr - wb2 * gi) : (wb2 * gr + wa * gi);
-                    }
-                }
-            }
-        }
-        gx[e * cin * din + q] = acc;
-    }
+    for (int q = threadIdx.x; q < cin * din; q += kThreads)
+        gx[e * cin * din + q] = in_entry<T>(L, sg, q / din, q % din, tlo, thi, t, sw);
 }
 
 // ---- table gradient by bin ---------------------------------------------------------
@@ -341,12 +212,7 @@ k_bd_bwd_r(feq_layout L, feq_binning B, const T* __restrict__ gy, const T* __res
         const int w = static_cast<int>(q % wd);
         const int ci = static_cast<int>((q / wd) % cin);
         const int co = static_cast<int>(q / (static_cast<int64_t>(wd) * cin));
-        const WeightRef ref = weight_ref(L, w);
-        const T u = weight_grad<T>(ref, sx + ci * din, sg + co * dout);
-        const T sc = ipow_t<T>(sw, ref.lsum);
-        const T wl = tlo[q], wh = thi[q];
-        acc_t += (wh - wl) * sc * u;
-        if (ref.lsum > 0) acc_s += lerp_t<T>(wl, wh, t) * u * sc * static_cast<T>(ref.lsum) * deriv;
+        dist_terms<T>(L, w, sx + ci * din, sg + co * dout, tlo[q], thi[q], t, sw, deriv, acc_t, acc_s);
     }
     const T st = block_sum<T>(acc_t, red);
     const T ss = block_sum<T>(acc_s, red);
@@ -477,12 +343,12 @@ int blockdiag_bwd(const feq_layout* L, const feq_binning* b, int64_t E, const T*
                 return rc;
     }
     if (!mm) {
-    auto kx = k_bd_bwd_x<T>;
-    FEQ_LAUNCH("k_bd_bwd_x", kx, dim3(E), dim3(kThreads), lds_x, s, *L, *b, gy, table, dist, gx);
-    const int nslices = static_cast<int>(ceil_div(L->cout, ob) * ceil_div(L->cin, ib));
-    auto kt = k_bd_bwd_table<T>;
-    FEQ_LAUNCH("k_bd_bwd_table", kt, dim3(b->num_bins + 1, nslices), dim3(kThreads), lds_t, s, *L,
-               *b, E, gy, x, dist, perm, offsets, ob, ib, gtable);
+        auto kx = k_bd_bwd_x<T>;
+        FEQ_LAUNCH("k_bd_bwd_x", kx, dim3(E), dim3(kThreads), lds_x, s, *L, *b, gy, table, dist, gx);
+        const int nslices = static_cast<int>(ceil_div(L->cout, ob) * ceil_div(L->cin, ib));
+        auto kt = k_bd_bwd_table<T>;
+        FEQ_LAUNCH("k_bd_bwd_table", kt, dim3(b->num_bins + 1, nslices), dim3(kThreads), lds_t, s, *L,
+                   *b, E, gy, x, dist, perm, offsets, ob, ib, gtable);
     }
     if (gdist && !dr_done) {
         auto kr = k_bd_bwd_r<T>;

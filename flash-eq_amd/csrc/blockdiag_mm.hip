@@ -6,7 +6,7 @@
 // them.  Here a workgroup takes 16 edges in the order of their bins (the stable
 // CSR by bin), one 16-channel tile of outputs, and reads each table row once for
 // the 16:
-//   forward   Y[co, e] (o)  += T_w[co, ci] X[ci, e] (i) + D_w[co, ci] (t_e X[ci, e] (i))
+//   forward   Y[co, e] (o)  += T_w[co, ci] X[ci, e] (i) + t_e D_w[co, ci] X[ci, e] (i)
 //   gradient  GX[ci, e] (i) += T_w[co, ci]^T G[co, e] (o) + t_e D_w^T G
 //   table     dT_w[co, ci]  += sum over e of G[co, e] (o) X[ci, e] (i)
 // with X = s^l x, G = s^l gy, T the bin's row and D the next row's difference to
@@ -17,7 +17,8 @@
 // Lane l = (c = l % 16, g = l / 16); a reduction step r takes the indices
 // 4 r + g: the staged rows [slot][channel][edge] (257 floats from slot to slot)
 // are then read as 64 consecutive floats.  The four waves of a workgroup share
-// the staged rows and split the (m, output) pairs.  Sums run in a fixed order.
+// the staged rows and split the (m, output) pairs.  Sums run in a fixed order, the
+// products of one summed index and 16 channels by themselves, then added.
 //
 // Lvals 0..2 x 32, 20 000 edges, 65 table rows, the per-edge kernels and these:
 // forward 1163 us, now 71 + 15 (pack) + 35 (sort by bin); input and distance
@@ -25,7 +26,9 @@
 // The matrix steps alone would take 20 to 40 us each: the staging of 16 edges'
 // rows, one memory latency per 16 channels, bounds these.  (Tiles dealt to the
 // L2s in turn, so that each read every bin's fragments: 94 and 154 us.)
-#include "feq_internal.h"
+#include "blockdiag_edge.h"
+
+#include <cfloat>
 
 namespace feq {
 namespace {
@@ -124,6 +127,8 @@ __device__ __forceinline__ void stage_rows(const float* __restrict__ x, int nch,
     }
 }
 
+__device__ __forceinline__ bool finite(float v) { return fabsf(v) <= FLT_MAX; }
+
 constexpr int kPow = 32;        // powers of s kept per edge (+ 1: no bank conflicts)
 
 // Operand order of the table: fragment (b, w, row tile, reduction tile) holds for
@@ -161,8 +166,8 @@ k_bdm_pack(const float* __restrict__ table, int cout, int cin, int wd, int wchun
 }
 
 // ---------------------------------------------------------------------------
-// A tile's product for up to MAXP pairs per wave: acc[p] += T S + D (t S), or with
-// GD acc[p] += T S, accD[p] += D S, accS[p] += T (l S) + D (t l S) (S: the staged
+// A tile's product for up to MAXP pairs per wave: acc[p] += T S + t (D S), or with
+// GD acc[p] += T S, accD[p] += D S, accS[p] += T (l S) + t (D (l S)) (S: the staged
 // rows, l: the degree of the summed slot; the distance gradient's three sums).
 template <int MAXP, bool GD>
 struct TileAcc {
@@ -172,14 +177,18 @@ struct TileAcc {
 };
 
 // SIGN: +1 forward (re += a re + b im, im += a im - b re), -1 transposed
-// (re += a re - b im, im += a im + b re).
+// (re += a re - b im, im += a im + b re).  in: whether the lane's column, an edge,
+// is of this bin.  The other columns' products are formed and not taken: multiplied
+// by zeros instead, a row of the table with an infinity or NaN would reach edges
+// that never read it.
 template <int MAXP, bool GD, int SIGN>
 __device__ __forceinline__ void tile_product(const Pairs& PT, int wave, const float* __restrict__ frag, int64_t bin, int wd,
-                                             int nrow, int row, int nred, int red, const float* st, float mask, float t,
+                                             int nrow, int row, int nred, int red, const float* st, bool in, float t,
                                              const int* deg, TileAcc<MAXP, GD>& A) {
     const int lane = threadIdx.x & 63;
     const int64_t wstride = static_cast<int64_t>(nrow) * nred * 512;
     const float* f0 = frag + ((bin * wd * nrow + row) * nred + red) * 512;
+    const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int p = 0; p < MAXP; ++p) {
         if (wave + 4 * p >= PT.n) break;
@@ -201,45 +210,42 @@ __device__ __forceinline__ void tile_product(const Pairs& PT, int wave, const fl
             v4f S[2];
             if (k + 1 < P.n) fetch(k + 1);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) S[0][r] = sr[64 * r + lane] * mask;
-            const float l = GD ? static_cast<float>(deg[P.other + P.z * k]) : 0.0f;
+            for (int r = 0; r < 4; ++r) S[0][r] = sr[64 * r + lane];
             if (P.z == 2) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) S[1][r] = sr[kSS + 64 * r + lane] * mask;
+                for (int r = 0; r < 4; ++r) S[1][r] = sr[kSS + 64 * r + lane];
             }
-            // component c of the products with the (a, b) fragments Q and the rows R
-            auto add = [&](const v4f (&Q)[2], const v4f (&R)[2], v4f (&acc)[2]) {
+            // component c of the product of the (a, b) fragments Q and the rows S
+            auto product = [&](const v4f (&Q)[2], v4f (&acc)[2]) {
+                acc[0] = acc[1] = zero;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) acc[0] = mfma4(Q[0][r], R[0][r], acc[0]);
+                for (int r = 0; r < 4; ++r) acc[0] = mfma4(Q[0][r], S[0][r], acc[0]);
                 if (P.z == 2) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        acc[1] = mfma4(Q[0][r], R[1][r], acc[1]);
-                        acc[0] = mfma4(Q[1][r], SIGN > 0 ? R[1][r] : -R[1][r], acc[0]);
-                        acc[1] = mfma4(Q[1][r], SIGN > 0 ? -R[0][r] : R[0][r], acc[1]);
+                        acc[1] = mfma4(Q[0][r], S[1][r], acc[1]);
+                        acc[0] = mfma4(Q[1][r], SIGN > 0 ? S[1][r] : -S[1][r], acc[0]);
+                        acc[1] = mfma4(Q[1][r], SIGN > 0 ? -S[0][r] : S[0][r], acc[1]);
                     }
                 }
             };
-            auto times = [&](float q) {
-                struct { v4f v[2]; } R;
+            v4f ts[2], ds[2];
+            product(T, ts);
+            product(D, ds);
+            const float l = GD ? static_cast<float>(deg[P.other + P.z * k]) : 0.0f;
 #pragma unroll
-                for (int z = 0; z < 2; ++z)
+            for (int z = 0; z < 2; ++z)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) R.v[z][r] = S[z][r] * q;
-                return R;
-            };
-            add(T, S, A.a[p]);
-            if constexpr (GD) {
-                add(D, S, A.d[p]);
-                if (l != 0.0f) {
-                    const auto L0 = times(l), L1 = times(l * t);
-                    add(T, L0.v, A.s[p]);
-                    add(D, L1.v, A.s[p]);
+                for (int r = 0; r < 4; ++r) {
+                    const float both = fmaf(t, ds[z][r], ts[z][r]);
+                    if constexpr (GD) {
+                        A.a[p][z][r] = in ? A.a[p][z][r] + ts[z][r] : A.a[p][z][r];
+                        A.d[p][z][r] = in ? A.d[p][z][r] + ds[z][r] : A.d[p][z][r];
+                        A.s[p][z][r] = in && l != 0.0f ? fmaf(l, both, A.s[p][z][r]) : A.s[p][z][r];
+                    } else {
+                        A.a[p][z][r] = in ? A.a[p][z][r] + both : A.a[p][z][r];
+                    }
                 }
-            } else {
-                const auto S1 = times(t);
-                add(D, S1.v, A.a[p]);
-            }
         }
     }
 }
@@ -260,18 +266,22 @@ __device__ __forceinline__ void clear(TileAcc<MAXP, GD>& A) {
 // Workgroup (tile of 16 sorted positions, 16-channel tile of outputs); x: the
 // summed side (E, nch, din) scaled by s^l, y: the produced side (E, noch, dout).
 // GD: the distance gradient's share of this channel tile to gpart[tile of
-// channels][position's edge], from xo, the features on the produced side.
+// channels][position's edge], from xo, the features on the produced side.  Edges
+// whose results hold an infinity or NaN are formed again from the unpacked table,
+// as the per-edge kernels form them: T + t D of infinite terms is NaN where
+// the interpolated weight is not.
 template <int MAXP, bool GD, int SIGN>
 __global__ void __launch_bounds__(kThreads, 2)
 k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __restrict__ perm,
             const float* __restrict__ dist, const float* __restrict__ x, int nch, int din, int noch, int dout, int wd,
-            const float* __restrict__ frag, const float* __restrict__ xo, float* __restrict__ y,
-            float* __restrict__ gpart, unsigned tiles) {
+            const float* __restrict__ table, const float* __restrict__ frag, const float* __restrict__ xo,
+            float* __restrict__ y, float* __restrict__ gpart, unsigned tiles) {
     extern __shared__ float st[];
     __shared__ float sPow[16 * (kPow + 1)];
     __shared__ int64_t sE[16];
     __shared__ int sLo[16];
     __shared__ float sRed[4 * 64];
+    __shared__ int sBad[16];
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // the eight L2s (workgroups go to them in turn) take an eighth of the sorted
@@ -288,6 +298,7 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
     if (threadIdx.x < 16) {
         sE[c] = R.e;
         sLo[c] = R.lo;
+        sBad[c] = 0;
         float p = 1.0f;
         for (int l = 0; l < kPow; ++l) {
             sPow[c * (kPow + 1) + l] = p;
@@ -305,7 +316,7 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
         for (int p = 0; p < n;) {       // the tile's bins, in order
             const int bin = sLo[p];
             tile_product<MAXP, GD, SIGN>(PT, wave, frag, bin, wd, nrow, row, nred, red, st,
-                                         R.lo == bin ? 1.0f : 0.0f, R.t, din_deg, A);
+                                         R.lo == bin, R.t, din_deg, A);
             while (p < n && sLo[p] == bin) ++p;
         }
     }
@@ -338,6 +349,7 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
             float sum = 0.0f;
             for (int k = 0; k < 16; ++k) sum += sRed[16 * k + threadIdx.x];
             gpart[static_cast<int64_t>(row) * E + sE[threadIdx.x]] = sum;
+            if (!finite(sum)) sBad[threadIdx.x] = 1;
         }
     }
     // the produced rows through LDS, so that they leave in whole runs
@@ -365,7 +377,43 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
     const float iper = 1.0f / static_cast<float>(per), idim = 1.0f / static_cast<float>(dout);
     for (int q = threadIdx.x; q < n * per; q += kThreads) {
         const int ed = quotient(q, iper), rest = q - ed * per, ch = quotient(rest, idim), d = rest - ch * dout;
-        if (16 * row + ch < noch) y[(sE[ed] * noch + 16 * row) * dout + rest] = st[d * kSS + ch * 16 + ed];
+        if (16 * row + ch < noch) {
+            const float v = st[d * kSS + ch * 16 + ed];
+            y[(sE[ed] * noch + 16 * row) * dout + rest] = v;
+            if (!finite(v)) sBad[ed] = 1;
+        }
+    }
+    __syncthreads();
+    const int nc = noch - 16 * row < 16 ? noch - 16 * row : 16;
+    for (int ed = 0; ed < n; ++ed) {
+        if (!sBad[ed]) continue;
+        const int64_t e = sE[ed];
+        const float r = dist[e], sw = r / (r + B.sh_scale);
+        const EdgeBinT<float> eb = edge_bin_t<float>(r, B);
+        const int64_t ts = static_cast<int64_t>(L.cout) * L.cin * wd;
+        const float* tlo = table + eb.lo * ts;
+        const float* xr = x + e * nch * din;
+        float* yr = y + (e * noch + 16 * row) * dout;
+        for (int q = threadIdx.x; q < nc * dout; q += kThreads)
+            yr[q] = SIGN > 0 ? out_entry<float>(L, xr, 16 * row + q / dout, q % dout, tlo, tlo + ts, eb.t, sw)
+                             : in_entry<float>(L, xr, 16 * row + q / dout, q % dout, tlo, tlo + ts, eb.t, sw);
+        if constexpr (GD) {
+            float at = 0.0f, as = 0.0f;
+            for (int q = threadIdx.x; q < L.cout * nc * wd; q += kThreads) {
+                const int w = q % wd, ci = 16 * row + q / wd % nc, co = q / (wd * nc);
+                const float* tw = tlo + (static_cast<int64_t>(co) * L.cin + ci) * wd + w;
+                dist_terms<float>(L, w, xo + (e * noch + ci) * dout, xr + co * din, tw[0], tw[ts], eb.t, sw,
+                                  B.sh_scale / (r * (r + B.sh_scale)), at, as);
+            }
+            sRed[threadIdx.x] = at * eb.dtdr + as;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                float sum = 0.0f;
+                for (int k = 0; k < kThreads; ++k) sum += sRed[k];
+                gpart[static_cast<int64_t>(row) * E + e] = sum;
+            }
+            __syncthreads();
+        }
     }
 }
 
@@ -605,7 +653,7 @@ int bdm_fwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* x
     const size_t lds = sizeof(float) * kSS * (L.din > L.dout ? L.din : L.dout);
     if (int rc = bdm_lds(reinterpret_cast<const void*>(k), lds)) return rc;
     FEQ_LAUNCH("k_bdm_fwd", k, dim3(static_cast<unsigned>(ceil_div(ceil_div(E, 16), 8) * 8), tiles16(L.cout)), dim3(kThreads), lds, s, L,
-               P, B, E, perm, dist, x, L.cin, L.din, L.cout, L.dout, L.wdim, frag, static_cast<const float*>(nullptr), y,
+               P, B, E, perm, dist, x, L.cin, L.din, L.cout, L.dout, L.wdim, table, frag, static_cast<const float*>(nullptr), y,
                static_cast<float*>(nullptr), static_cast<unsigned>(ceil_div(E, 16)));
     return FEQ_OK;
 }
@@ -627,7 +675,7 @@ int bdm_bwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* g
     if (int rc = bdm_lds(reinterpret_cast<const void*>(k), lds)) return rc;
     const int nt = tiles16(L.cin);
     FEQ_LAUNCH("k_bdm_bwd_x", k, dim3(static_cast<unsigned>(ceil_div(ceil_div(E, 16), 8) * 8), nt), dim3(kThreads), lds, s,
-               L, P, B, E, perm, dist, gy, L.cout, L.dout, L.cin, L.din, L.wdim, frag, x, gx, gpart,
+               L, P, B, E, perm, dist, gy, L.cout, L.dout, L.cin, L.din, L.wdim, table, frag, x, gx, gpart,
                static_cast<unsigned>(ceil_div(E, 16)));
     if (gd)
         FEQ_LAUNCH("k_bdm_dr", k_bdm_dr, dim3(static_cast<unsigned>(ceil_div(E, 256))), dim3(256), 0, s, gpart, nt, E,

@@ -43,3 +43,58 @@ def test_products_match_oracle(dev, lin, lout, cin, cout, nb, E, log):
     assert rel_err(xg.grad, gx) < 1e-5
     assert rel_err(Tg.grad, gt) < 1e-5
     assert rel_err(rg.grad, gr) < 1e-4
+
+
+def _raw(dev, lin, lout, b, nb, log, x, T, r, gy, products):
+    """y, dx, dT, dr of the C entry points: the products, or the per-edge kernels (which run where
+    the workspace holds no more than the edges' sort)."""
+    lib, C = NAT.lib(), NAT.ctypes
+    L = NAT.make_layout(lin, lout, x.shape[1], gy.shape[1])
+    B = NAT.make_binning(b.p1, b.p2, nb, log, 0.1)
+    E = x.shape[0]
+    sort_only = NAT.make_layout([0], [0], 1, 1)
+    n = lib.feq_blockdiag_workspace(C.byref(L if products else sort_only), C.byref(B), E)
+    ws = NAT.workspace(n, dev)
+    y, gx, gT, gr = torch.empty_like(gy), torch.empty_like(x), torch.empty_like(T), torch.empty_like(r)
+    p = NAT.ptr
+    NAT.profile_summary()
+    NAT.profile_enable(True)
+    try:
+        NAT.check(lib.feq_blockdiag_fwd(C.byref(L), C.byref(B), E, p(x), p(T), p(r), p(y), p(ws), n,
+                                        NAT.stream_ptr(dev)), "feq_blockdiag_fwd")
+        NAT.check(lib.feq_blockdiag_bwd(C.byref(L), C.byref(B), E, p(gy), p(x), p(T), p(r), p(gx), p(gT), p(gr),
+                                        p(ws), n, NAT.stream_ptr(dev)), "feq_blockdiag_bwd")
+    finally:
+        NAT.profile_enable(False)
+    launched = NAT.profile_summary()
+    assert ("k_bdm_fwd" in launched) == products and ("k_bd_fwd" in launched) != products, launched
+    return y, gx, gT, gr
+
+
+@pytest.mark.parametrize("where", ["table", "rows", "none"])
+@pytest.mark.parametrize("lin,lout,cin,cout,nb,E,log", [
+    ([0, 1, 2], [0, 1, 2], 32, 32, 40, 1601, False),          # the distance gradient rides along
+    ([0, 1, 2, 3], [1, 2], 17, 24, 9, 2700, True),
+    ([0, 1, 2, 3, 4, 5, 6], [0, 1, 2, 3, 4, 5, 6], 16, 16, 16, 450, False),
+])
+def test_infinities_and_nan_stay_where_the_per_edge_kernels_leave_them(dev, lin, lout, cin, cout, nb, E, log, where):
+    """The same values, infinities and NaN as the per-edge kernels: a row of the table reaches only
+    the edges of its two bins, a feature only its own edge."""
+    b, x, T, r, gy = (t.float().to(dev) if isinstance(t, torch.Tensor) else t
+                      for t in _case(lin, lout, cin, cout, nb, E, log, seed=E))
+    inf, nan = float("inf"), float("nan")
+    if where == "table":
+        T[3, 5, 7, 0], T[5, 0, 1, -1], T[8, 2, 3, 1] = inf, nan, -inf
+    elif where == "rows":
+        x[11, 3, 1], x[40, 0, -1], x[41, 5, 0] = inf, -inf, nan
+        gy[90, 2, 1], gy[91, 4, 0], gy[40, 1, 1] = inf, nan, -inf
+        r[200] = 0.0        # the distance gradient is NaN there
+    got = _raw(dev, lin, lout, b, nb, log, x, T, r, gy, True)
+    ref = _raw(dev, lin, lout, b, nb, log, x, T, r, gy, False)
+    for name, a, c in zip(("y", "gx", "gT", "gr"), got, ref):
+        fin = torch.isfinite(c)
+        assert torch.equal(torch.isfinite(a), fin), (name, int((torch.isfinite(a) != fin).sum()))
+        if name != "gT":        # (an infinite and a zero factor may meet in another order there)
+            assert torch.equal(torch.isnan(a), torch.isnan(c)), name
+            assert torch.equal(a == inf, c == inf) and torch.equal(a == -inf, c == -inf), name
+        assert rel_err(a[fin], c[fin]) < (1e-4 if name == "gr" else 1e-5), name
