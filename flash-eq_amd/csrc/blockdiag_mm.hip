@@ -6,13 +6,16 @@
 // them.  Here a workgroup takes 16 edges in the order of their bins (the stable
 // CSR by bin), one 16-channel tile of outputs, and reads each table row once for
 // the 16:
-//   forward   Y[co, e] (o)  += T_w[co, ci] X[ci, e] (i) + t_e D_w[co, ci] X[ci, e] (i)
-//   gradient  GX[ci, e] (i) += T_w[co, ci]^T G[co, e] (o) + t_e D_w^T G
+//   forward   Y[co, e] (o)  += M_w[co, ci] X[ci, e] (i) + u_e D_w[co, ci] X[ci, e] (i)
+//   gradient  GX[ci, e] (i) += M_w[co, ci]^T G[co, e] (o) + u_e D_w^T G
 //   table     dT_w[co, ci]  += sum over e of G[co, e] (o) X[ci, e] (i)
-// with X = s^l x, G = s^l gy, T the bin's row and D the next row's difference to
-// it: T + t D is the well-conditioned form where linear bins extrapolate
-// (|t| >> 1), as in the per-edge kernels.  The table is first packed into operand
-// order (k_bdm_pack), T and D side by side, zero-padded to 16 channels.
+// with X = s^l x, G = s^l gy, M the mean of the bin's row and the next one, D the
+// next row's difference to it, u = t - 1/2.  M + u D keeps the per-edge kernels'
+// precision: inside a bin its two terms are no larger than they have to be (with the
+// row itself and t D, the errors of y and dx are 1.1 to 1.5 times theirs), and where
+// linear bins extrapolate (|t| >> 1) it stays well conditioned.  The table is first
+// packed into operand order (k_bdm_pack), M and D side by side, zero-padded to 16
+// channels.
 //
 // Lane l = (c = l % 16, g = l / 16); a reduction step r takes the indices
 // 4 r + g: the staged rows [slot][channel][edge] (257 floats from slot to slot)
@@ -21,8 +24,8 @@
 // products of one summed index and 16 channels by themselves, then added.
 //
 // Lvals 0..2 x 32, 20 000 edges, 65 table rows, the per-edge kernels and these:
-// forward 1163 us, now 71 + 15 (pack) + 35 (sort by bin); input and distance
-// gradients 816 + 1724, now 126 + 16 (pack); table gradient 2256, now 154 + 10.
+// forward 1163 us, now 82 + 18 (pack) + 35 (sort by bin); input and distance
+// gradients 816 + 1724, now 133 + 18 (pack); table gradient 2256, now 156 + 12.
 // The matrix steps alone would take 20 to 40 us each: the staging of 16 edges'
 // rows, one memory latency per 16 channels, bounds these.  (Tiles dealt to the
 // L2s in turn, so that each read every bin's fragments: 94 and 154 us.)
@@ -132,7 +135,7 @@ __device__ __forceinline__ bool finite(float v) { return fabsf(v) <= FLT_MAX; }
 constexpr int kPow = 32;        // powers of s kept per edge (+ 1: no bank conflicts)
 
 // Operand order of the table: fragment (b, w, row tile, reduction tile) holds for
-// lane (c, g) the four values r of T, then of D: T[co, ci] with, forward, co = 16
+// lane (c, g) the four values r of M, then of D: M[co, ci] with, forward, co = 16
 // row + c and ci = 16 red + 4 r + g, and transposed (TR) with ci = 16 row + c and
 // co = 16 red + 4 r + g.  A workgroup packs the 16 x 16 channels of one bin.
 template <bool TR>
@@ -152,7 +155,7 @@ k_bdm_pack(const float* __restrict__ table, int cout, int cin, int wd, int wchun
             const bool ok = co < cout && ci < cin;
             const int64_t at = ok ? b * ts + (static_cast<int64_t>(co) * cin + ci) * wd + w0 + w : 0;
             const float lo = table[at], hi = table[ok ? at + ts : 0];
-            sm[ch * ls + w] = ok ? lo : 0.0f;
+            sm[ch * ls + w] = ok ? 0.5f * lo + 0.5f * hi : 0.0f;
             sm[(256 + ch) * ls + w] = ok ? hi - lo : 0.0f;
         }
         __syncthreads();
@@ -166,8 +169,8 @@ k_bdm_pack(const float* __restrict__ table, int cout, int cin, int wd, int wchun
 }
 
 // ---------------------------------------------------------------------------
-// A tile's product for up to MAXP pairs per wave: acc[p] += T S + t (D S), or with
-// GD acc[p] += T S, accD[p] += D S, accS[p] += T (l S) + t (D (l S)) (S: the staged
+// A tile's product for up to MAXP pairs per wave: acc[p] += M S + u (D S), or with
+// GD acc[p] += M S, accD[p] += D S, accS[p] += l (M S + u (D S)) (S: the staged
 // rows, l: the degree of the summed slot; the distance gradient's three sums).
 template <int MAXP, bool GD>
 struct TileAcc {
@@ -183,7 +186,7 @@ struct TileAcc {
 // that never read it.
 template <int MAXP, bool GD, int SIGN>
 __device__ __forceinline__ void tile_product(const Pairs& PT, int wave, const float* __restrict__ frag, int64_t bin, int wd,
-                                             int nrow, int row, int nred, int red, const float* st, bool in, float t,
+                                             int nrow, int row, int nred, int red, const float* st, bool in, float u,
                                              const int* deg, TileAcc<MAXP, GD>& A) {
     const int lane = threadIdx.x & 63;
     const int64_t wstride = static_cast<int64_t>(nrow) * nred * 512;
@@ -193,20 +196,20 @@ __device__ __forceinline__ void tile_product(const Pairs& PT, int wave, const fl
     for (int p = 0; p < MAXP; ++p) {
         if (wave + 4 * p >= PT.n) break;
         const Pair P = PT.p[wave + 4 * p];
-        v4f Tn[2], Dn[2];       // the next summed index's fragments
+        v4f Mn[2], Dn[2];       // the next summed index's fragments
         auto fetch = [&](int k) {
             const float* fa = f0 + (P.w + k * P.step) * wstride;
-            Tn[0] = *reinterpret_cast<const v4f*>(fa + 4 * lane);
+            Mn[0] = *reinterpret_cast<const v4f*>(fa + 4 * lane);
             Dn[0] = *reinterpret_cast<const v4f*>(fa + 256 + 4 * lane);
             if (P.z == 2) {
-                Tn[1] = *reinterpret_cast<const v4f*>(fa + wstride + 4 * lane);
+                Mn[1] = *reinterpret_cast<const v4f*>(fa + wstride + 4 * lane);
                 Dn[1] = *reinterpret_cast<const v4f*>(fa + wstride + 256 + 4 * lane);
             }
         };
         fetch(0);
         for (int k = 0; k < P.n; ++k) {
             const float* sr = st + (P.other + P.z * k) * kSS;
-            const v4f T[2] = {Tn[0], Tn[1]}, D[2] = {Dn[0], Dn[1]};
+            const v4f M[2] = {Mn[0], Mn[1]}, D[2] = {Dn[0], Dn[1]};
             v4f S[2];
             if (k + 1 < P.n) fetch(k + 1);
 #pragma unroll
@@ -229,17 +232,17 @@ __device__ __forceinline__ void tile_product(const Pairs& PT, int wave, const fl
                     }
                 }
             };
-            v4f ts[2], ds[2];
-            product(T, ts);
+            v4f ms[2], ds[2];
+            product(M, ms);
             product(D, ds);
             const float l = GD ? static_cast<float>(deg[P.other + P.z * k]) : 0.0f;
 #pragma unroll
             for (int z = 0; z < 2; ++z)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float both = fmaf(t, ds[z][r], ts[z][r]);
+                    const float both = fmaf(u, ds[z][r], ms[z][r]);
                     if constexpr (GD) {
-                        A.a[p][z][r] = in ? A.a[p][z][r] + ts[z][r] : A.a[p][z][r];
+                        A.a[p][z][r] = in ? A.a[p][z][r] + ms[z][r] : A.a[p][z][r];
                         A.d[p][z][r] = in ? A.d[p][z][r] + ds[z][r] : A.d[p][z][r];
                         A.s[p][z][r] = in && l != 0.0f ? fmaf(l, both, A.s[p][z][r]) : A.s[p][z][r];
                     } else {
@@ -268,7 +271,7 @@ __device__ __forceinline__ void clear(TileAcc<MAXP, GD>& A) {
 // GD: the distance gradient's share of this channel tile to gpart[tile of
 // channels][position's edge], from xo, the features on the produced side.  Edges
 // whose results hold an infinity or NaN are formed again from the unpacked table,
-// as the per-edge kernels form them: T + t D of infinite terms is NaN where
+// as the per-edge kernels form them: M + u D of infinite terms is NaN where
 // the interpolated weight is not.
 template <int MAXP, bool GD, int SIGN>
 __global__ void __launch_bounds__(kThreads, 2)
@@ -316,12 +319,12 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
         for (int p = 0; p < n;) {       // the tile's bins, in order
             const int bin = sLo[p];
             tile_product<MAXP, GD, SIGN>(PT, wave, frag, bin, wd, nrow, row, nred, red, st,
-                                         R.lo == bin, R.t, din_deg, A);
+                                         R.lo == bin, R.t - 0.5f, din_deg, A);
             while (p < n && sLo[p] == bin) ++p;
         }
     }
     if constexpr (GD) {
-        // x on the produced side: sum of x accD, and of l x (accT + t accD) + x accS
+        // x on the produced side: sum of x accD, and of l x (acc + u accD) + x accS
         __syncthreads();
         stage_rows<true>(xo, noch, 16 * row, dout, sE, sPow, kPow + 1, dout_deg, n, st);
         __syncthreads();
@@ -337,7 +340,7 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
                     const float q = st[(P.slot + z) * kSS + (4 * g + r) * 16 + c];
                     const v4f a = z ? A.a[p][1] : A.a[p][0], d = z ? A.d[p][1] : A.d[p][0], s = z ? A.s[p][1] : A.s[p][0];
                     at += q * d[r];
-                    as += q * (l * (a[r] + R.t * d[r]) + s[r]);
+                    as += q * (l * (a[r] + (R.t - 0.5f) * d[r]) + s[r]);
                 }
             }
         }
@@ -367,7 +370,7 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     float v = A.a[p][z][r];
-                    if constexpr (GD) v += R.t * A.d[p][z][r];
+                    if constexpr (GD) v += (R.t - 0.5f) * A.d[p][z][r];
                     st[(P.slot + z) * kSS + (4 * g + r) * 16 + c] = v * sc;
                 }
             }
@@ -431,12 +434,13 @@ __global__ void k_bdm_dr(const float* __restrict__ part, int n, int64_t E, float
 // row's edges): the edges of bin b (weight 1 - t) and of bin b - 1 (weight t) in
 // sorted order, 16 at a time, their indices, bins and powers 64 at a time (one
 // memory latency for four tiles).  Few table rows leave the chip idle (65 rows
-// and 4 tiles: 260 workgroups, 577 us, 232 with eight splits and 154 with kInFlight), so the edges
-// are then split and the splits' sums added in order (k_bdm_sum).
+// and 4 tiles: 260 workgroups, 577 us, 232 with eight splits and 156 with kInFlight), so the edges
+// are then split and the splits' sums added in order (k_bdm_sum).  Three workgroups
+// per CU, with a few registers spilled: 190 us with two.
 constexpr int kMaxU = 8;
 constexpr int kHead = 64;
 
-__global__ void __launch_bounds__(kThreads, 2)
+__global__ void __launch_bounds__(kThreads, 3)
 k_bdm_table(feq_layout L, Units UT, feq_binning B, int64_t E, const int32_t* __restrict__ perm,
             const int32_t* __restrict__ offsets, const float* __restrict__ dist, const float* __restrict__ gy,
             const float* __restrict__ x, int splits, float* __restrict__ gtable) {
@@ -489,17 +493,22 @@ k_bdm_table(feq_layout L, Units UT, feq_binning B, int64_t E, const int32_t* __r
             const Unit U = UT.u[u0 + 4 * u];
             const float* ga = sg + U.o * kSS;
             const float* xa = sx + U.i * kSS;
+            // the 16 edges' sum by itself, then added: a short chain of additions and
+            // one over the tiles, not one over all edges
+            v4f one[2] = {v4f{0.0f, 0.0f, 0.0f, 0.0f}, v4f{0.0f, 0.0f, 0.0f, 0.0f}};
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float gr = ga[64 * r + lane], fr = xa[64 * r + lane];
-                acc[u][0] = mfma4(gr, fr, acc[u][0]);
+                one[0] = mfma4(gr, fr, one[0]);
                 if (U.z == 2) {     // a: fr gr + fi gi, b: fi gr - fr gi
                     const float gi = ga[kSS + 64 * r + lane], fi = xa[kSS + 64 * r + lane];
-                    acc[u][0] = mfma4(gi, fi, acc[u][0]);
-                    acc[u][1] = mfma4(gr, fi, acc[u][1]);
-                    acc[u][1] = mfma4(gi, -fr, acc[u][1]);
+                    one[0] = mfma4(gi, fi, one[0]);
+                    one[1] = mfma4(gr, fi, one[1]);
+                    one[1] = mfma4(gi, -fr, one[1]);
                 }
             }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[u][0][r] += one[0][r], acc[u][1][r] += one[1][r];
         }
     }
     const int ci = 16 * cit + c;
