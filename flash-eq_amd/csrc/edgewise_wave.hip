@@ -42,7 +42,6 @@ namespace feq {
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
 constexpr int kMaxNB = 4;       // 16-slot blocks
 constexpr int kMaxCT = 4;       // 16-channel tiles
@@ -75,109 +74,40 @@ __device__ __forceinline__ int lane_id() {
     return lane;
 }
 
-// The channel mixes (G_k and H_k, a third to a half of the float32 steps) run on
-// the fp16 matrix cores with split operands, as edgewise_split.hip's: a = 2^-e (hi
-// + lo), e from the largest magnitude (in [2^14, 2^15) after scaling), a product as
-// lo lo + hi lo + lo hi + hi hi with float32 accumulation.  All four: the errors
-// against float64 (geometric mean over every output, five layouts, five seeds) are
-// 3.87e-7, 3.90e-7 with float32 steps and 3.97e-7 without lo lo (the vector kernels
-// 3.94e-7).  Two 16-channel tiles make one 32-step: lane group g holds the reduction
-// indices 4 g + r of both, in the order of the float32 registers, so the halves are
-// converted in place.  16x16x32 takes 16 cycles, four of them 64 against 256.
-__device__ __forceinline__ v4f mfma_h(h8 a, h8 b, v4f c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ int scale_exp(float m) {
-    int e = 141 - static_cast<int>((__float_as_uint(m) >> 23) & 0xffu);
-    e = e < -113 ? -113 : e;
-    return e > 126 ? 126 : e;
-}
-__device__ __forceinline__ float exp2i(int e) { return __uint_as_float(static_cast<unsigned>(e + 127) << 23); }
-__device__ __forceinline__ float max4(float m, const v4f& v) {
-    return fmaxf(fmaxf(m, fmaxf(fabsf(v[0]), fabsf(v[1]))), fmaxf(fabsf(v[2]), fabsf(v[3])));
-}
-struct Halves {
-    h8 hi, lo;
-};
-__device__ __forceinline__ Halves split8(const v4f& a, const v4f& b, float sc) {
-    Halves h;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const float v = j < 4 ? a[j & 3] : b[j & 3];
-        h.hi[j] = static_cast<_Float16>(__builtin_fmaf(v, sc, 0.0f));
-        h.lo[j] = static_cast<_Float16>(__builtin_fmaf(v, sc, -static_cast<float>(h.hi[j])));
-    }
-    return h;
-}
-// Tiles of one operand, split with one scale for the wave; e: its exponent.
-template <int CT, int NB>
-struct SplitTiles {
-    Halves t[(CT + 1) / 2][NB];
-    int e;
-};
-template <int CT, int NB>
-__device__ __forceinline__ void split_tiles(const v4f (&v)[CT][NB], SplitTiles<CT, NB>& S) {
-    float m = 0.0f;
-#pragma unroll
-    for (int t = 0; t < CT; ++t)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) m = max4(m, v[t][b]);
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-    S.e = scale_exp(m);
-    const float sc = exp2i(S.e);
-    const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int h = 0; h < (CT + 1) / 2; ++h)
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-            S.t[h][b] = split8(v[2 * h][b], 2 * h + 1 < CT ? v[2 * h + 1 < CT ? 2 * h + 1 : 0][b] : zero, sc);
-}
-// The patterns in operand order, split once per call by k_ewg_prep: for rank k and
-// column tile c0 / 16, the halves of the reduction tiles' pairs, one scale per
-// column (exponents at the end).  (Split by every wave for every edge, they took a
-// third of the vector instructions at lvals 0..4 x 32.)
+// The patterns in operand order, packed once per call by k_ewg_prep: for rank k and
+// column tile c0 / 16, the reduction tiles' B operands, zero-padded to 16 channels.
+// (Ragged channel counts then need no conditions in the edge loop.)
 struct Patterns {
-    const Halves* frag;     // [rank][column tile][pair][lane]
-    const int* exps;        // [rank][column tile][16]
+    const v4f* frag;        // [rank][column tile][reduction tile][lane]
     int ncol;               // column tiles
 };
 template <int CT>
 struct Mixer {
-    Halves q[(CT + 1) / 2];
-    int e;
+    v4f q[CT];
 };
 template <int CT>
 __device__ __forceinline__ void load_mixer(const Patterns& W, int k, int col, Mixer<CT>& M) {
-    constexpr int NH = (CT + 1) / 2;
     const unsigned lane = lane_id();
-    const Halves* f = W.frag + (k * W.ncol + col) * NH * 64;
+    const v4f* f = W.frag + (k * W.ncol + col) * CT * 64;
 #pragma unroll
-    for (int h = 0; h < NH; ++h) M.q[h] = f[64 * h + lane];
-    M.e = W.exps[(k * W.ncol + col) * 16 + (lane & 15)];
+    for (int t = 0; t < CT; ++t) M.q[t] = f[64 * t + lane];
 }
-// out[b] (rows: the tiles' positions, columns: the patterns' channels) =
-// sum over channels of the tiles and the patterns.
+// out[b] (rows: the tiles' positions, columns: the patterns' channels) = sum over
+// channels of the tiles and the patterns.  (On the fp16 matrix cores with operands split
+// in two halves these products take a fourth of the cycles, 0.58 against 0.71 ms forward at
+// lvals 0..6 x 32, 50 000 edges; but two halves hold 22 bits below one exponent per
+// edge, and the gradients of the radial functions of a degree whose values are small
+// beside the edge's largest lose theirs.)
 template <int CT, int NB>
-__device__ __forceinline__ void mix_channels(const SplitTiles<CT, NB>& S, const Mixer<CT>& M, v4f (&out)[NB]) {
+__device__ __forceinline__ void mix_channels(const v4f (&v)[CT][NB], const Mixer<CT>& M, v4f (&out)[NB]) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) out[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int h = 0; h < (CT + 1) / 2; ++h) {
+    for (int t = 0; t < CT; ++t)
 #pragma unroll
-        for (int b = 0; b < NB; ++b) out[b] = mfma_h(S.t[h][b].lo, M.q[h].lo, out[b]);
+        for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int b = 0; b < NB; ++b) out[b] = mfma_h(S.t[h][b].hi, M.q[h].lo, out[b]);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) out[b] = mfma_h(S.t[h][b].lo, M.q[h].hi, out[b]);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) out[b] = mfma_h(S.t[h][b].hi, M.q[h].hi, out[b]);
-    }
-    const int back = -(M.e + S.e);
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) out[b][r] = __builtin_amdgcn_ldexpf(out[b][r], back);
+            for (int b = 0; b < NB; ++b) out[b] = mfma4(v[t][b][r], M.q[t][r], out[b]);
 }
 
 // Orders a wave's LDS writes before its later reads by other lanes (LDS
@@ -459,22 +389,13 @@ __device__ __forceinline__ v4f load_c(const float* __restrict__ Ck, int co0, int
 // way round.
 template <bool BWD>
 __global__ void __launch_bounds__(64)
-k_ewg_prep(const float* __restrict__ C, int cout, int cin, Halves* __restrict__ frag, int* __restrict__ exps) {
-    const int lane = threadIdx.x, k = blockIdx.x, col = blockIdx.y, ncol = gridDim.y;
-    const int ct = ((BWD ? cout : cin) + 15) / 16, nh = (ct + 1) / 2;
+k_ewg_prep(const float* __restrict__ C, int cout, int cin, v4f* __restrict__ frag) {
+    const int k = blockIdx.x, col = blockIdx.y, ncol = gridDim.y;
+    const int ct = ((BWD ? cout : cin) + 15) / 16;
     const float* Ck = C + static_cast<int64_t>(k) * cout * cin;
-    auto tile = [&](int t) {
-        return BWD ? load_c<true>(Ck, 16 * t, 16 * col, cout, cin) : load_c<false>(Ck, 16 * col, 16 * t, cout, cin);
-    };
-    float m = 0.0f;
-    for (int t = 0; t < ct; ++t) m = max4(m, tile(t));
-    m = fmaxf(m, __shfl_xor(m, 16, 64));
-    m = fmaxf(m, __shfl_xor(m, 32, 64));
-    const int e = scale_exp(m);
-    const float sc = exp2i(e);
-    for (int h = 0; h < nh; ++h)
-        frag[((k * ncol + col) * nh + h) * 64 + lane] = split8(tile(2 * h), tile(2 * h + 1), sc);
-    if (lane < 16) exps[(k * ncol + col) * 16 + lane] = e;
+    for (int t = 0; t < ct; ++t)
+        frag[((k * ncol + col) * ct + t) * 64 + threadIdx.x] =
+            BWD ? load_c<true>(Ck, 16 * t, 16 * col, cout, cin) : load_c<false>(Ck, 16 * col, 16 * t, cout, cin);
 }
 
 // Workgroups per CU: what the registers allow without (much) spilling.  The grids
@@ -513,8 +434,6 @@ k_ewg_fwd(GenTab T, feq_binning B, int64_t E, const float* __restrict__ x, const
             stage_basis<NB>(P + e * din * din, din, sB, [&] { edge_weights(T, B, dist[e], F, sFe, deg); });
         }
         rotate_in<CT, NB, false>(x + e * cin * din, 0, cin, sB, din, in_col, fs);
-        SplitTiles<CT, NB> S;
-        split_tiles<CT, NB>(fs, S);
         if (Q != P) stage_basis<NB>(Q + e * dout * dout, dout, sB, [] {});
         for (int co0 = 0; co0 < cout; co0 += 16) {
             v4f m[NB];
@@ -527,7 +446,7 @@ k_ewg_fwd(GenTab T, feq_binning B, int64_t E, const float* __restrict__ x, const
             for (int k = 0; k < kRank; ++k) {
                 v4f G[NB];
                 load_mixer<CT>(W, k + 1 < kRank ? k + 1 : k, co0 / 16, next);
-                mix_channels<CT, NB>(S, M, G);
+                mix_channels<CT, NB>(fs, M, G);
                 M = next;
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
@@ -606,8 +525,6 @@ k_ewg_bwd_x(GenTab T, feq_binning B, int64_t E, const float* __restrict__ gy, co
             stage_basis<NB>(Q + e * dout * dout, dout, sB, [&] { edge_weights(T, B, dist[e], F, sFe, deg); });
         }
         rotate_in<CT, NB, false>(gy + e * cout * dout, 0, cout, sB, dout, out_col, gd);
-        SplitTiles<CT, NB> S;
-        split_tiles<CT, NB>(gd, S);
         if (Q != P) stage_basis<NB>(P + e * din * din, din, sB, [] {});
         for (int ci0 = 0; ci0 < cin; ci0 += 16) {
             v4f fs[1][NB], dfs[NB];
@@ -624,7 +541,7 @@ k_ewg_bwd_x(GenTab T, feq_binning B, int64_t E, const float* __restrict__ gy, co
                 v4f Z[NB];
 #pragma unroll
                 for (int b = 0; b < NB; ++b) Z[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-                mix_channels<CT, NB>(S, M, H);
+                mix_channels<CT, NB>(gd, M, H);
                 M = next;
                 const int ln = lane_id(), c = ln & 15, g = ln >> 4;
                 wave_sync();    // the previous rank's reads
@@ -854,21 +771,17 @@ int ew_wave_groups(const feq_layout& L, int64_t E) {
     return static_cast<int>(n < 512 ? n : 512);
 }
 
-// The split patterns: fragments of the wider of the two forms, and the exponents.
+// The packed patterns.
 size_t ew_wave_workspace(const feq_layout& L) {
-    const int ci = tiles(L.cin), co = tiles(L.cout);
-    const int frags = kRank * (co * ((ci + 1) / 2) > ci * ((co + 1) / 2) ? co * ((ci + 1) / 2) : ci * ((co + 1) / 2));
-    return frags * 64 * sizeof(Halves) + sizeof(int) * kRank * 16 * (ci > co ? ci : co) + 256;
+    return kRank * tiles(L.cin) * tiles(L.cout) * 64 * sizeof(v4f) + 256;
 }
 
 template <bool BWD>
 static int prep(const feq_layout& L, const float* C, void* ws, Patterns& W, hipStream_t s) {
-    const int ci = tiles(L.cin), co = tiles(L.cout), ncol = BWD ? ci : co, nh = ((BWD ? co : ci) + 1) / 2;
-    Halves* frag = reinterpret_cast<Halves*>(align_up(reinterpret_cast<uintptr_t>(ws), 32));
-    int* exps = reinterpret_cast<int*>(frag + kRank * ncol * nh * 64);
-    W = Patterns{frag, exps, ncol};
+    v4f* frag = reinterpret_cast<v4f*>(align_up(reinterpret_cast<uintptr_t>(ws), sizeof(v4f)));
+    W = Patterns{frag, tiles(BWD ? L.cin : L.cout)};
     auto k = k_ewg_prep<BWD>;
-    FEQ_LAUNCH("k_ewg_prep", k, dim3(kRank, ncol), dim3(64), 0, s, C, L.cout, L.cin, frag, exps);
+    FEQ_LAUNCH("k_ewg_prep", k, dim3(kRank, W.ncol), dim3(64), 0, s, C, L.cout, L.cin, frag);
     return FEQ_OK;
 }
 

@@ -4,8 +4,11 @@ whose widest groups share blocks, repeated, missing and unmixed degrees, and edg
 up.  The launch log shows that they ran.  Tolerance: every stage accumulates in float32, as the
 shape-generic kernels do, and is held to the same 1e-5 of the largest entry."""
 import pytest
+import torch
 
 from flash_eq import _native as NAT
+from flash_eq.ops import edgewise_linear
+from oracle import wigner as OW
 from test_gpu_edgewise import _run_parity, _select
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +45,54 @@ def test_wave_parity(dev, monkeypatch, lin, lout, cin, cout, E):
 def test_wave_parity_log_bins(dev, monkeypatch):
     _select(monkeypatch, "split")
     _run_parity(dev, [0, 1, 2, 3], [0, 1, 2, 3], 32, 32, 515, seed=4, log=True, rmin=0.2)
+
+
+def _weights_of(layout, side, l):
+    """The radial weights that join slots of degree l on that side ('in' or 'out')."""
+    ws = []
+    for k in range(layout.nblocks):
+        m, ni, no, ioff, ooff, woff = layout.blk[k]
+        z = 2 if m else 1
+        for o in range(no):
+            for i in range(ni):
+                deg = layout.lslot_in[ioff + z * i] if side == "in" else layout.lslot_out[ooff + z * o]
+                if deg == l:
+                    ws += [woff + z * (o * ni + i) + c for c in range(z)]
+    return ws
+
+
+@pytest.mark.parametrize("lv,c", [([0, 1, 2, 3], 32), ([0, 1, 2, 3, 4], 24)])
+def test_small_degrees_keep_their_precision(dev, monkeypatch, lv, c):
+    """A degree 2^-32 below the others loses nothing to them.  Its terms are sums of their own
+    in float32, and a power of two scales every one of them exactly: what a call gives for it beside
+    the large degrees is 2^-32 times what it gives without them, bit for bit."""
+    _select(monkeypatch, "split")
+    top, E, nb, tiny = lv[-1], 300, 20, 2.0 ** -32
+    L, B = NAT.make_layout(lv, lv, c, c), NAT.make_binning(0.0, nb / 10.0, nb, False, 0.1)
+    g = torch.Generator().manual_seed(3)
+    dim = L.din
+    small = torch.zeros(dim, dtype=torch.bool)
+    small[dim - (2 * top + 1):] = True
+    x, gy = torch.randn(E, c, dim, generator=g), torch.randn(E, c, dim, generator=g)
+    P = OW.basis(lv, torch.randn(E, 3, generator=g)).float().to(dev)
+    r = (torch.rand(E, generator=g) * 9 + 0.3).to(dev)
+    C, F = torch.randn(4, c, c, generator=g).to(dev), torch.randn(nb + 1, 4, L.wdim, generator=g)
+
+    def grads(x, F, gy):
+        xs, Fs = x.to(dev).requires_grad_(True), F.to(dev).requires_grad_(True)
+        y = edgewise_linear(xs, P, P, r, C, Fs, L, B, 4)
+        y.backward(gy.to(dev))
+        return y.detach(), Fs.grad
+
+    # outputs from the small degree alone: the weights of the other inputs are zero
+    w_in, w_out = _weights_of(L, "in", top), _weights_of(L, "out", top)
+    Fi = torch.zeros_like(F)
+    Fi[..., w_in] = F[..., w_in]
+    y, _ = grads(torch.where(small, x * tiny, x), Fi, gy)
+    y1, _ = grads(torch.where(small, x, 0.0), Fi, gy)
+    assert torch.equal(y, y1 * tiny)
+    # the radial functions' gradients of the weights that lead to it
+    _, gF = grads(x, F, torch.where(small, gy * tiny, gy))
+    _, gF1 = grads(x, F, torch.where(small, gy, 0.0))
+    assert gF1[..., w_out].abs().max() > 0
+    assert torch.equal(gF[..., w_out], gF1[..., w_out] * tiny)
