@@ -22,20 +22,20 @@
 // one 16-slot block (GenTab): M_k has diagonal block tiles only.  No barriers:
 // each wave works alone, and x, P, Q and C go from memory to the operands.
 //
-// What bounds them: the float32 matrix cores (a step of 16x16x4 takes 32
-// cycles).  lvals 0..6 x 32 channels take 312 steps and 128 of 16 cycles forward,
-// 554 and 128 for the input gradient and 624 for the pattern gradient per edge,
-// against 30 KB of memory.
-// At 50 000 such edges 0.58, 1.06 and 0.91 ms, where edgewise.hip's vector
-// kernels (a workgroup per edge, every product through LDS) took 7.1 ms forward and
-// 18.3 ms backward; at lvals 0..4 x 32 and 20 000 edges 0.11, 0.20
-// and 0.18 against 1.24 and 3.29.
+// lvals 0..6 x 32 channels take 568 float32 steps (16x16x4, 32 cycles) forward, 800
+// for the input gradient and 624 for the pattern gradient per edge, against 30 KB of
+// memory.  At 50 000 such edges 0.68, 1.17 and 0.90 ms, of which these steps take 0.37,
+// 0.52 and 0.41 with every matrix core busy: what bounds them is a wave's chain of dependent
+// steps, LDS reads and scalar work between them, which the two waves per SIMD that the
+// registers allow cover in part.  edgewise.hip's vector kernels (a workgroup per
+// edge, every product through LDS) took 7.1 ms forward and 18.3 ms backward; at
+// lvals 0..4 x 32 and 20 000 edges 0.13, 0.22 and 0.18 against 1.24 and 3.29.
 // What did not carry: operands from memory without the LDS copy of the basis
 // (1.5, 2.9 and 1.6 ms: requests of 4 rows x 16 scattered columns); loads under lane
-// conditions (1.0, 2.0 and 1.0); float32 steps for the channel mixes too (0.71, 1.21
-// and 0.91: matrix cores busy 55%, 45% and 47% of the time, the vector unit another
-// 15 to 19%, which two waves per SIMD overlap little); Z_k summed over the channel
-// tiles (2% faster, errors 5% larger: one chain instead of two).
+// conditions (1.0, 2.0 and 1.0); Z_k summed over the channel tiles (2% faster,
+// errors 5% larger: one chain instead of two).  Where an edge's values are not finite,
+// its results are not either, but an infinity may come out as NaN: the tiles multiply
+// positions that no weight joins by zeros.
 #include "feq_internal.h"
 
 namespace feq {
@@ -94,7 +94,7 @@ __device__ __forceinline__ void load_mixer(const Patterns& W, int k, int col, Mi
 }
 // out[b] (rows: the tiles' positions, columns: the patterns' channels) = sum over
 // channels of the tiles and the patterns.  (On the fp16 matrix cores with operands split
-// in two halves these products take a fourth of the cycles, 0.58 against 0.71 ms forward at
+// in two halves these products take a fourth of the cycles, 0.58 against 0.68 ms forward at
 // lvals 0..6 x 32, 50 000 edges; but two halves hold 22 bits below one exponent per
 // edge, and the gradients of the radial functions of a degree whose values are small
 // beside the edge's largest lose theirs.)
@@ -177,6 +177,23 @@ __device__ __forceinline__ void edge_weights(const GenTab& T, const feq_binning&
 __device__ __forceinline__ float coef(const float* sFk, const int (&code)[2], int r) {
     const unsigned q = static_cast<unsigned>(code[r >> 1]) >> (16 * (r & 1));
     return __uint_as_float(__float_as_uint(sFk[q & 0x3fff]) ^ ((q & 0x4000u) << 17));
+}
+
+// acc[b] += the mixing matrix of one rank times the tiles v: the rank's sum by itself,
+// then added (one chain over the ranks' slots: errors of y and dx 2% larger, the input
+// gradient 3% faster).
+template <int NB>
+__device__ __forceinline__ void add_mixed(const float* sFk, const int (&code)[NB][2], int last, const v4f (&v)[NB],
+                                          v4f (&acc)[NB]) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        v4f one = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (b < NB - 1 || r < last) one = mfma4(coef(sFk, code[b], r), v[b][r], one);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[b][r] += one[r];
+    }
 }
 
 // A basis matrix (n = dim^2 contiguous floats, 4-byte aligned) to the wave's LDS
@@ -448,11 +465,7 @@ k_ewg_fwd(GenTab T, feq_binning B, int64_t E, const float* __restrict__ x, const
                 load_mixer<CT>(W, k + 1 < kRank ? k + 1 : k, co0 / 16, next);
                 mix_channels<CT, NB>(fs, M, G);
                 M = next;
-#pragma unroll
-                for (int b = 0; b < NB; ++b)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (b < NB - 1 || r < last) m[b] = mfma4(coef(sFe + k * (wd + 1), code[b], r), G[b][r], m[b]);
+                add_mixed<NB>(sFe + k * (wd + 1), code, last, G, m);
             }
             rotate_out<NB>(m, sB, dout, last, out_red, y + e * cout * dout, co0 / 16, cout);
         }
@@ -556,11 +569,7 @@ k_ewg_bwd_x(GenTab T, feq_binning B, int64_t E, const float* __restrict__ gy, co
 #pragma unroll
                     for (int r = 0; r < 4; ++r) Z[b] = mfma4(h[r], fs[0][b][r], Z[b]);
                 }
-#pragma unroll
-                for (int b = 0; b < NB; ++b)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (b < NB - 1 || r < last) dfs[b] = mfma4(coef(sFk, code[b], r), H[b][r], dfs[b]);
+                add_mixed<NB>(sFk, code, last, H, dfs);
                 weights_of(Z, dF[k]);
             }
             rotate_out<NB>(dfs, sB, din, last, in_red, gx + e * cin * din, ci0 / 16, cin);
