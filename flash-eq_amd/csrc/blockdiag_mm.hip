@@ -328,7 +328,7 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
         __syncthreads();
         stage_rows<true>(xo, noch, 16 * row, dout, sE, sPow, kPow + 1, dout_deg, n, st);
         __syncthreads();
-        float at = 0.0f, as = 0.0f;
+        float atr[4] = {}, asr[4] = {};     // four short chains of additions
 #pragma unroll
         for (int p = 0; p < MAXP; ++p) {
             if (wave + 4 * p >= PT.n) break;
@@ -339,11 +339,12 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
                 for (int r = 0; r < 4; ++r) {
                     const float q = st[(P.slot + z) * kSS + (4 * g + r) * 16 + c];
                     const v4f a = z ? A.a[p][1] : A.a[p][0], d = z ? A.d[p][1] : A.d[p][0], s = z ? A.s[p][1] : A.s[p][0];
-                    at += q * d[r];
-                    as += q * (l * (a[r] + (R.t - 0.5f) * d[r]) + s[r]);
+                    atr[r] += q * d[r];
+                    asr[r] += q * (l * (a[r] + (R.t - 0.5f) * d[r]) + s[r]);
                 }
             }
         }
+        const float at = (atr[0] + atr[1]) + (atr[2] + atr[3]), as = (asr[0] + asr[1]) + (asr[2] + asr[3]);
         float v = at * R.dtdr;
         if (L.has_lpos) v += as * (B.sh_scale / (R.r * (R.r + B.sh_scale)));
         sRed[threadIdx.x] = v;
