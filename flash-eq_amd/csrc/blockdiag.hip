@@ -271,13 +271,6 @@ int bin_csr(const feq_binning& b, int64_t E, const T* dist, Carver& cv, int32_t*
     return feq_csr_by_dst(lo, E, b.num_bins, *perm, *offsets, csr_ws, feq_csr_workspace(E, b.num_bins), stream);
 }
 
-// Whether the matrix-product form (float32) runs: its sizes and the workspace.
-template <class T>
-bool use_bdm(const feq_layout& L, const feq_binning& b, int64_t E, const void* ws, size_t ws_bytes) {
-    return std::is_same_v<T, float> && ws && bdm_supported(L, b, E) &&
-           ws_bytes >= bin_ws_bytes(b, E) + bdm_workspace(L, b, E);
-}
-
 template <class T>
 int blockdiag_fwd(const feq_layout* L, const feq_binning* b, int64_t E, const T* x, const T* table,
                   const T* dist, T* y, void* ws, size_t ws_bytes, feq_stream_t stream) {
@@ -290,7 +283,8 @@ int blockdiag_fwd(const feq_layout* L, const feq_binning* b, int64_t E, const T*
     const size_t lds = sizeof(T) * L->cin * L->din;
     if (lds > 64 * 1024) return fail(FEQ_ERR_UNSUPPORTED, "Cin*Din too large for this kernel");
     if constexpr (std::is_same_v<T, float>) {
-        if (use_bdm<T>(*L, *b, E, ws, ws_bytes)) {
+        const size_t need = feq_blockdiag_fwd_workspace(L, b, E);
+        if (need && ws && ws_bytes >= need) {
             Carver cv(ws);
             int32_t *perm, *offsets;
             if (int rc = bin_csr<T>(*b, E, dist, cv, &perm, &offsets, stream)) return rc;
@@ -336,7 +330,7 @@ int blockdiag_bwd(const feq_layout* L, const feq_binning* b, int64_t E, const T*
     if (int rc = bin_csr<T>(*b, E, dist, cv, &perm, &offsets, stream)) return rc;
     bool mm = false, dr_done = false;
     if constexpr (std::is_same_v<T, float>) {
-        mm = use_bdm<T>(*L, *b, E, ws, ws_bytes);
+        mm = bdm_bwd_supported(*L, *b, E) && ws_bytes >= feq_blockdiag_workspace(L, b, E);
         if (mm)
             if (int rc = bdm_bwd(*L, *b, E, gy, x, table, dist, perm, offsets, gx, gtable, gdist, &dr_done,
                                  static_cast<char*>(ws) + bin_ws_bytes(*b, E), s))
@@ -379,7 +373,16 @@ using namespace feq;
 
 extern "C" size_t feq_blockdiag_workspace(const feq_layout* L, const feq_binning* b, int64_t E) {
     if (!L || !b || E <= 0) return 0;
-    return bin_ws_bytes(*b, E) + (bdm_supported(*L, *b, E) ? bdm_workspace(*L, *b, E) : 0);
+    return bin_ws_bytes(*b, E) + (bdm_bwd_supported(*L, *b, E) ? bdm_bwd_workspace(*L, *b, E) : 0);
+}
+
+extern "C" size_t feq_blockdiag_workspace_f64(const feq_layout* L, const feq_binning* b, int64_t E) {
+    return L && b && E > 0 ? bin_ws_bytes(*b, E) : 0;
+}
+
+extern "C" size_t feq_blockdiag_fwd_workspace(const feq_layout* L, const feq_binning* b, int64_t E) {
+    if (!L || !b || E <= 0 || !bdm_fwd_supported(*L, *b, E)) return 0;
+    return bin_ws_bytes(*b, E) + bdm_fwd_workspace(*L, *b);
 }
 
 extern "C" int feq_blockdiag_fwd(const feq_layout* L, const feq_binning* b, int64_t E,

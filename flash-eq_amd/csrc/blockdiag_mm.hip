@@ -610,7 +610,7 @@ constexpr double kBdmMinWork = 2.5e7;
 // Where the products beat the per-edge kernels: their fixed cost (the sort by
 // bin and the packed table, about 80 us) against the per-edge kernels' 3 ps per
 // edge and table weight forward.
-bool bdm_supported(const feq_layout& L, const feq_binning& B, int64_t E) {
+static bool covers(const feq_layout& L, const feq_binning& B, int64_t E) {
     Pairs P;
     Units U;
     if (L.din > kMaxSlots || L.dout > kMaxSlots || L.wdim < 1 || B.num_bins < 1) return false;
@@ -623,6 +623,9 @@ bool bdm_supported(const feq_layout& L, const feq_binning& B, int64_t E) {
     if (!build_units(L, U)) return false;
     return static_cast<double>(E) * L.cin * L.cout * L.wdim >= kBdmMinWork;
 }
+
+bool bdm_bwd_supported(const feq_layout& L, const feq_binning& B, int64_t E) { return covers(L, B, E); }
+bool bdm_fwd_supported(const feq_layout& L, const feq_binning& B, int64_t E) { return covers(L, B, E); }
 
 namespace {
 size_t table_floats(const feq_layout& L, const feq_binning& B) {
@@ -639,11 +642,13 @@ int table_splits(const feq_layout& L, const feq_binning& B, int64_t E, int units
 }
 }  // namespace
 
-size_t bdm_workspace(const feq_layout& L, const feq_binning& B, int64_t E) {
+size_t bdm_fwd_workspace(const feq_layout& L, const feq_binning& B) { return sizeof(float) * frag_floats(L, B); }
+
+size_t bdm_bwd_workspace(const feq_layout& L, const feq_binning& B, int64_t E) {
     Units U;
     build_units(L, U);
     const int splits = table_splits(L, B, E, U.n);
-    return sizeof(float) * (frag_floats(L, B) + 64 + static_cast<size_t>(E) * tiles16(L.cin) + 64 +
+    return sizeof(float) * (align_up(frag_floats(L, B), 64) + align_up(static_cast<size_t>(E) * tiles16(L.cin), 64) +
                             (splits > 1 ? splits * table_floats(L, B) : 0));
 }
 

@@ -204,8 +204,10 @@ int ew0_bwd(const feq_layout& L, const feq_binning& B, int rank, int64_t E, cons
 // The generic block-diagonal op in float32 as matrix products over edges grouped
 // by bin (blockdiag_mm.hip); perm, offsets: the stable CSR by lower bin.
 // *dr_done: whether gdist was written.
-bool bdm_supported(const feq_layout& L, const feq_binning& B, int64_t E);
-size_t bdm_workspace(const feq_layout& L, const feq_binning& B, int64_t E);
+bool bdm_fwd_supported(const feq_layout& L, const feq_binning& B, int64_t E);
+bool bdm_bwd_supported(const feq_layout& L, const feq_binning& B, int64_t E);
+size_t bdm_fwd_workspace(const feq_layout& L, const feq_binning& B);
+size_t bdm_bwd_workspace(const feq_layout& L, const feq_binning& B, int64_t E);
 int bdm_fwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* x, const float* table, const float* dist,
             const int32_t* perm, float* y, void* ws, hipStream_t s);
 int bdm_bwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* gy, const float* x, const float* table,

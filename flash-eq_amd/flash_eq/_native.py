@@ -60,7 +60,9 @@ _SIGS = {
     "feq_profile_summary": ([ctypes.c_char_p, _SZ], ctypes.c_int),
     "feq_layout_init": ([_P, _P, _I32, _P, _I32, _I32, _I32], ctypes.c_int),
     "feq_bin_edges": ([_P, _I64, _P, _P, _P, _P], ctypes.c_int),
+    "feq_blockdiag_fwd_workspace": ([_P, _P, _I64], _SZ),
     "feq_blockdiag_workspace": ([_P, _P, _I64], _SZ),
+    "feq_blockdiag_workspace_f64": ([_P, _P, _I64], _SZ),
     "feq_blockdiag_fwd": ([_P, _P, _I64, _P, _P, _P, _P, _P, _SZ, _P], ctypes.c_int),
     "feq_blockdiag_bwd": ([_P, _P, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P], ctypes.c_int),
     "feq_blockdiag_fwd_f64": ([_P, _P, _I64, _P, _P, _P, _P, _P], ctypes.c_int),

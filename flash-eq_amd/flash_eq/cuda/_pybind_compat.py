@@ -68,8 +68,9 @@ def _library() -> ctypes.CDLL:
             lib = ctypes.CDLL(path)
             lib.feq_last_error.restype = ctypes.c_char_p
             lib.feq_layout_init.argtypes = [_P, _P, _I32, _P, _I32, _I32, _I32]
-            lib.feq_blockdiag_workspace.argtypes = [_P, _P, _I64]
-            lib.feq_blockdiag_workspace.restype = _SZ
+            for size in (lib.feq_blockdiag_workspace, lib.feq_blockdiag_workspace_f64):
+                size.argtypes = [_P, _P, _I64]
+                size.restype = _SZ
             lib.feq_blockdiag_fwd.argtypes = [_P, _P, _I64, _P, _P, _P, _P, _P, _SZ, _P]
             lib.feq_blockdiag_bwd.argtypes = [_P, _P, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]
             lib.feq_blockdiag_fwd_f64.argtypes = [_P, _P, _I64, _P, _P, _P, _P, _P]
@@ -165,9 +166,9 @@ def backward(grad_output, features, radial_table, distances, sh_scale, bin_param
     g, x, T, r = (t.to(cdt).contiguous() for t in (grad_output, features, radial_table, distances))
     gx, gt, gr = torch.zeros_like(x), torch.zeros_like(T), torch.zeros_like(r)
     lib = _library()
-    ws = torch.empty(max(int(lib.feq_blockdiag_workspace(ctypes.byref(L), ctypes.byref(b), E)), 1),
-                     dtype=torch.uint8, device=dev)
-    fn = lib.feq_blockdiag_bwd_f64 if cdt == torch.float64 else lib.feq_blockdiag_bwd
+    size, fn = ((lib.feq_blockdiag_workspace_f64, lib.feq_blockdiag_bwd_f64) if cdt == torch.float64 else
+                (lib.feq_blockdiag_workspace, lib.feq_blockdiag_bwd))
+    ws = torch.empty(max(int(size(ctypes.byref(L), ctypes.byref(b), E)), 1), dtype=torch.uint8, device=dev)
     with torch.cuda.device(dev):
         rc = fn(ctypes.byref(L), ctypes.byref(b), E, g.data_ptr() if E else None, x.data_ptr(),
                 T.data_ptr(), r.data_ptr(), gx.data_ptr(), gt.data_ptr(), gr.data_ptr(),

@@ -609,11 +609,11 @@ class BlockDiagonalFn(torch.autograd.Function):
                                                    N.ptr(xs), N.ptr(ts), N.ptr(rs), N.ptr(y),
                                                    N.stream_ptr(dev))
                 else:
-                    ws = N.workspace(lib.feq_blockdiag_workspace(N.ctypes.byref(layout),
-                                                                 N.ctypes.byref(binning), E), dev)
+                    n = lib.feq_blockdiag_fwd_workspace(N.ctypes.byref(layout), N.ctypes.byref(binning), E)
+                    ws = N.workspace(n, dev) if n else None
                     rc = lib.feq_blockdiag_fwd(N.ctypes.byref(layout), N.ctypes.byref(binning), E,
                                                N.ptr(xs), N.ptr(ts), N.ptr(rs), N.ptr(y), N.ptr(ws),
-                                               ws.numel(), N.stream_ptr(dev))
+                                               n, N.stream_ptr(dev))
             N.check(rc, "feq_blockdiag_fwd")
         ctx.save_for_backward(xs, ts, rs)
         ctx.meta = (layout, binning, features.dtype, table.dtype, dist.dtype)
@@ -630,9 +630,10 @@ class BlockDiagonalFn(torch.autograd.Function):
         gt = torch.empty_like(ts)
         gr = torch.empty_like(rs) if ctx.needs_input_grad[2] else None
         lib = N.lib()
-        ws = N.workspace(lib.feq_blockdiag_workspace(N.ctypes.byref(layout), N.ctypes.byref(binning),
-                                                     E), dev)
-        fn = lib.feq_blockdiag_bwd_f64 if xs.dtype == torch.float64 else lib.feq_blockdiag_bwd
+        f64 = xs.dtype == torch.float64
+        size = lib.feq_blockdiag_workspace_f64 if f64 else lib.feq_blockdiag_workspace
+        ws = N.workspace(size(N.ctypes.byref(layout), N.ctypes.byref(binning), E), dev)
+        fn = lib.feq_blockdiag_bwd_f64 if f64 else lib.feq_blockdiag_bwd
         with N.on_device(dev):
             rc = fn(N.ctypes.byref(layout), N.ctypes.byref(binning), E, N.ptr(g) if E else None,
                     N.ptr(xs), N.ptr(ts), N.ptr(rs), N.ptr(gx), N.ptr(gt), N.ptr(gr), N.ptr(ws),

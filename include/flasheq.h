@@ -118,12 +118,13 @@ int feq_bin_edges(const feq_binning* b, int64_t num_edges, const float* dist,
                   int32_t* lo, float* t, feq_stream_t stream);
 
 /* ---- generic block-diagonal op: table (num_bins+1, Cout, Cin, Wdim) ----------
- * The forward needs no workspace (NULL, 0); given feq_blockdiag_workspace bytes
- * it runs large calls as matrix products over edges grouped by bin.  The
- * backward needs feq_blockdiag_workspace bytes: it groups the edges by lower bin and sums the
- * table gradient per bin in a fixed order (no atomics: the same bits on every
- * run).  grad_dist may be NULL (not needed).  grad_x, grad_table and
- * grad_dist are overwritten. */
+ * The forward needs no workspace (NULL, 0); given feq_blockdiag_fwd_workspace
+ * bytes (0 where a call would not gain by it) it runs as matrix products over
+ * edges grouped by bin.  The backward needs feq_blockdiag_workspace bytes: it
+ * groups the edges by lower bin and sums the table gradient per bin in a fixed
+ * order (no atomics: the same bits on every run).  grad_dist may be NULL (not
+ * needed).  grad_x, grad_table and grad_dist are overwritten. */
+size_t feq_blockdiag_fwd_workspace(const feq_layout* L, const feq_binning* b, int64_t num_edges);
 size_t feq_blockdiag_workspace(const feq_layout* L, const feq_binning* b, int64_t num_edges);
 int feq_blockdiag_fwd(const feq_layout* L, const feq_binning* b, int64_t num_edges,
                       const float* x, const float* table, const float* dist, float* y,
@@ -134,7 +135,9 @@ int feq_blockdiag_bwd(const feq_layout* L, const feq_binning* b, int64_t num_edg
                       void* workspace, size_t ws_bytes, feq_stream_t stream);
 /* The same op in float64: the reference dispatches the kernels on float64 as well
  * (block_diagonal.cu:1332, 1605, AT_DISPATCH_FLOATING_TYPES_AND_HALF); bin
- * indices in float32, t and dt/dr in float64, as its InterpState<double>. */
+ * indices in float32, t and dt/dr in float64, as its InterpState<double>.  The
+ * backward needs feq_blockdiag_workspace_f64 bytes. */
+size_t feq_blockdiag_workspace_f64(const feq_layout* L, const feq_binning* b, int64_t num_edges);
 int feq_blockdiag_fwd_f64(const feq_layout* L, const feq_binning* b, int64_t num_edges,
                           const double* x, const double* table, const double* dist, double* y,
                           feq_stream_t stream);

@@ -202,3 +202,25 @@ def test_wigner_dimension_limit(suffix, lvals):
                    getattr(lib, "feq_wigner_basis_bwd" + suffix)(lv, len(lvals), one, one, E, one, one, one, None)):
             assert rc != 0 and "too large" in lib.feq_last_error().decode(), (E, rc, lib.feq_last_error())
     assert getattr(lib, "feq_wigner_basis" + suffix)(lv, len(lvals), one, one, 0, None, None, None) == 0
+
+
+@pytest.mark.parametrize("lin,lout,cin,cout,bins,E,fwd,bwd", [
+    ([0, 1, 2], [0, 1, 2], 32, 32, 64, 20000, True, True),
+    ([0, 1, 2], [0, 1, 2], 32, 32, 64, 1000, False, False),          # too little work
+    (list(range(7)), list(range(7)), 32, 32, 100, 131, True, True),
+])
+def test_blockdiag_products_and_their_workspaces(lin, lout, cin, cout, bins, E, fwd, bwd):
+    """The workspace of the block-diagonal op's products over bin-grouped edges: the sort's, the packed
+    table's and, backward only, the split sums'; none for the float32 forwards of the per-edge kernels, no more than the sort's for their backward and float64."""
+    lib = N.load_library()
+    L, b = N.make_layout(lin, lout, cin, cout), N.make_binning(0.0, 10.0, bins, False, 0.1)
+    args = (ctypes.byref(L), ctypes.byref(b), E)
+    up = lambda n: -(-n // 256) * 256
+    sort = up(8 * E) + up(4 * E) + up(4 * (bins + 1)) + up(lib.feq_csr_workspace(E, bins)) + 256
+    pad = lambda c: -(-c // 16) * 16
+    packed = 8 * bins * L.wdim * pad(cin) * pad(cout)
+    assert lib.feq_blockdiag_workspace_f64(*args) == sort
+    assert lib.feq_blockdiag_fwd_workspace(*args) == (sort + packed if fwd else 0)
+    most = sort + packed + 4 * pad(E) * pad(cin) // 16 + (256 << 20) + 1024
+    assert sort + packed < lib.feq_blockdiag_workspace(*args) <= most if bwd else \
+        lib.feq_blockdiag_workspace(*args) == sort
