@@ -137,7 +137,8 @@ constexpr int kPow = 32;        // powers of s kept per edge (+ 1: no bank confl
 // Operand order of the table: fragment (b, w, row tile, reduction tile) holds for
 // lane (c, g) the four values r of M, then of D: M[co, ci] with, forward, co = 16
 // row + c and ci = 16 red + 4 r + g, and transposed (TR) with ci = 16 row + c and
-// co = 16 red + 4 r + g.  A workgroup packs the 16 x 16 channels of one bin.
+// co = 16 red + 4 r + g.  A workgroup packs wchunk weights of the 16 x 16 channels of
+// one bin (all of them in turn left the chip idle: lvals 0..6 x 16, 64 bins, 155 us).
 template <bool TR>
 __global__ void __launch_bounds__(kThreads)
 k_bdm_pack(const float* __restrict__ table, int cout, int cin, int wd, int wchunk, float* __restrict__ frag) {
@@ -147,24 +148,21 @@ k_bdm_pack(const float* __restrict__ table, int cout, int cin, int wd, int wchun
     const int cot = blockIdx.y / nci, cit = blockIdx.y % nci;
     const int row = TR ? cit : cot, red = TR ? cot : cit, nrow = TR ? nci : nco, nred = TR ? nco : nci;
     const int64_t ts = static_cast<int64_t>(cout) * cin * wd;
-    for (int w0 = 0; w0 < wd; w0 += wchunk) {
-        const int nw = wd - w0 < wchunk ? wd - w0 : wchunk, ls = wchunk + 1;
-        __syncthreads();
-        for (int q = threadIdx.x; q < 256 * nw; q += kThreads) {
-            const int ch = q / nw, w = q - ch * nw, co = 16 * cot + ch / 16, ci = 16 * cit + ch % 16;
-            const bool ok = co < cout && ci < cin;
-            const int64_t at = ok ? b * ts + (static_cast<int64_t>(co) * cin + ci) * wd + w0 + w : 0;
-            const float lo = table[at], hi = table[ok ? at + ts : 0];
-            sm[ch * ls + w] = ok ? 0.5f * lo + 0.5f * hi : 0.0f;
-            sm[(256 + ch) * ls + w] = ok ? hi - lo : 0.0f;
-        }
-        __syncthreads();
-        for (int q = threadIdx.x; q < 512 * nw; q += kThreads) {
-            const int w = q / 512, k = q - w * 512, d = k >> 8, l = (k & 255) >> 2, r = k & 3;
-            const int a = l & 15, z = 4 * r + (l >> 4);       // row and reduction channel
-            const int ch = TR ? z * 16 + a : a * 16 + z;
-            frag[((((b * wd + w0 + w) * nrow + row) * nred + red) * 2 + d) * 256 + l * 4 + r] = sm[(256 * d + ch) * ls + w];
-        }
+    const int w0 = blockIdx.z * wchunk, nw = wd - w0 < wchunk ? wd - w0 : wchunk, ls = wchunk + 1;
+    for (int q = threadIdx.x; q < 256 * nw; q += kThreads) {
+        const int ch = q / nw, w = q - ch * nw, co = 16 * cot + ch / 16, ci = 16 * cit + ch % 16;
+        const bool ok = co < cout && ci < cin;
+        const int64_t at = ok ? b * ts + (static_cast<int64_t>(co) * cin + ci) * wd + w0 + w : 0;
+        const float lo = table[at], hi = table[ok ? at + ts : 0];
+        sm[ch * ls + w] = ok ? 0.5f * lo + 0.5f * hi : 0.0f;
+        sm[(256 + ch) * ls + w] = ok ? hi - lo : 0.0f;
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < 512 * nw; q += kThreads) {
+        const int w = q / 512, k = q - w * 512, d = k >> 8, l = (k & 255) >> 2, r = k & 3;
+        const int a = l & 15, z = 4 * r + (l >> 4);       // row and reduction channel
+        const int ch = TR ? z * 16 + a : a * 16 + z;
+        frag[((((b * wd + w0 + w) * nrow + row) * nred + red) * 2 + d) * 256 + l * 4 + r] = sm[(256 * d + ch) * ls + w];
     }
 }
 
@@ -583,11 +581,8 @@ bool build_units(const feq_layout& L, Units& T) {
 }
 
 int tiles16(int n) { return (n + 15) / 16; }
-constexpr int kPackLds = 48 * 1024;
-int pack_chunk(int wd) {
-    const int most = kPackLds / (512 * 4) - 1;
-    return wd < most ? wd : most;
-}
+// Weights per workgroup of the packing: up to 48 KB of LDS, or 16 where they are more.
+int pack_chunk(int wd) { return wd < 24 ? wd : 16; }
 size_t frag_floats(const feq_layout& L, const feq_binning& B) {
     return static_cast<size_t>(B.num_bins) * L.wdim * tiles16(L.cin) * tiles16(L.cout) * 512;
 }
@@ -597,19 +592,24 @@ template <bool TR>
 int pack(const feq_layout& L, const feq_binning& B, const float* table, float* frag, hipStream_t s) {
     auto k = k_bdm_pack<TR>;
     const int chunk = pack_chunk(L.wdim);
-    FEQ_LAUNCH("k_bdm_pack", k, dim3(B.num_bins, tiles16(L.cin) * tiles16(L.cout)), dim3(kThreads),
-               sizeof(float) * 512 * (chunk + 1), s, table, L.cout, L.cin, L.wdim, chunk, frag);
+    FEQ_LAUNCH("k_bdm_pack", k,
+               dim3(B.num_bins, tiles16(L.cin) * tiles16(L.cout), static_cast<unsigned>(ceil_div(L.wdim, chunk))),
+               dim3(kThreads), sizeof(float) * 512 * (chunk + 1), s, table, L.cout, L.cin, L.wdim, chunk, frag);
     return FEQ_OK;
 }
 
 }  // namespace
 
-// Work (edges times table weights) from which on the products run.
-constexpr double kBdmMinWork = 2.5e7;
+// Where the products run.  Their fixed cost is the sort by bin and two packings,
+// about 60 us, against 3 to 5 ps per edge and table weight in a per-edge kernel: from
+// kMinWork edges times weights on they are faster (measured around it, forward
+// and backward: lvals 0..2 x 16, 8000 edges 115 -> 60 and 943 -> 109 us; x 32, 1000 edges
+// 88 -> 57 and 380 -> 103; lvals 0..6 x 16, 440 edges 225 -> 164 and 767 -> 640; x 1,
+// 1 400 000 edges 1434 -> 1439 and 64.6 -> 5.2 ms).
+constexpr double kMinWork = 2.5e7;
+// The packed table takes no more memory than this.
+constexpr size_t kMaxFragBytes = size_t{4} << 30;
 
-// Where the products beat the per-edge kernels: their fixed cost (the sort by
-// bin and the packed table, about 80 us) against the per-edge kernels' 3 ps per
-// edge and table weight forward.
 static bool covers(const feq_layout& L, const feq_binning& B, int64_t E) {
     Pairs P;
     Units U;
@@ -621,11 +621,27 @@ static bool covers(const feq_layout& L, const feq_binning& B, int64_t E) {
     if (sizeof(float) * kSS * static_cast<size_t>(L.din + L.dout) > 128 * 1024) return false;
     if (!build_pairs(L, false, P) || P.n > 4 * kMaxP || !build_pairs(L, true, P) || P.n > 4 * kMaxP) return false;
     if (!build_units(L, U)) return false;
-    return static_cast<double>(E) * L.cin * L.cout * L.wdim >= kBdmMinWork;
+    return static_cast<double>(E) * L.cin * L.cout * L.wdim >= kMinWork &&
+           frag_floats(L, B) * sizeof(float) <= kMaxFragBytes;
 }
 
+// The backward takes them wherever they are covered: it sorts in any case, and its
+// per-edge distance and table gradients are slow enough that the packing of more bins
+// than edges pays too (lvals 0..2 x 32, 4096 bins, 2000 edges: 1403 -> 946 us).
 bool bdm_bwd_supported(const feq_layout& L, const feq_binning& B, int64_t E) { return covers(L, B, E); }
-bool bdm_fwd_supported(const feq_layout& L, const feq_binning& B, int64_t E) { return covers(L, B, E); }
+
+// The forward where the packing does not cost more than the per-edge kernel: 7 ps per
+// bin and packed weight (channels padded to 16) against 4 per edge and weight, or
+// against the 2.5 ns per weight that a few edges take together.  Lvals 0..2 x 32,
+// per-edge kernel and products: 1000 bins, 1400 edges 165 and 183 us, 2000 edges 231 and
+// 182; 4096 bins, 4096 edges 455 and 567, 8000 edges 857 and 584; lvals 0..6 x 32,
+// 100 bins, 131 edges 831 and 694.
+bool bdm_fwd_supported(const feq_layout& L, const feq_binning& B, int64_t E) {
+    if (!covers(L, B, E)) return false;
+    const double weights = static_cast<double>(L.cin) * L.cout * L.wdim;
+    const double packed = static_cast<double>(frag_floats(L, B)) / 2;     // bins times padded weights
+    return 7.0 * packed <= weights * (4.0 * static_cast<double>(E) > 2500.0 ? 4.0 * static_cast<double>(E) : 2500.0);
+}
 
 namespace {
 size_t table_floats(const feq_layout& L, const feq_binning& B) {
@@ -653,7 +669,7 @@ size_t bdm_bwd_workspace(const feq_layout& L, const feq_binning& B, int64_t E) {
 }
 
 static int bdm_lds(const void* fn, size_t bytes) {
-    if (bytes > 64 * 1024)
+    if (bytes > 48 * 1024)      // with the kernels' static LDS (up to 10 KB) beyond 64 KB
         FEQ_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
     return FEQ_OK;
 }

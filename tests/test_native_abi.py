@@ -207,11 +207,18 @@ def test_wigner_dimension_limit(suffix, lvals):
 @pytest.mark.parametrize("lin,lout,cin,cout,bins,E,fwd,bwd", [
     ([0, 1, 2], [0, 1, 2], 32, 32, 64, 20000, True, True),
     ([0, 1, 2], [0, 1, 2], 32, 32, 64, 1000, False, False),          # too little work
+    ([0, 1, 2], [0, 1, 2], 32, 32, 1000, 1400, False, True),         # the forward's packing costs more than it gives
+    ([0, 1, 2], [0, 1, 2], 32, 32, 1000, 2000, True, True),
+    ([0, 1, 2], [0, 1, 2], 32, 32, 4096, 4096, False, True),
+    ([0, 1, 2], [0, 1, 2], 1, 1, 4096, 1400000, False, True),        # packed at 256 times its size
     (list(range(7)), list(range(7)), 32, 32, 100, 131, True, True),
+    (list(range(7)), list(range(7)), 128, 128, 100, 7, True, True),  # few edges, 14 ms in a per-edge kernel
+    (list(range(7)), list(range(7)), 128, 128, 150, 20000, False, False),   # 4.5 GB packed
 ])
 def test_blockdiag_products_and_their_workspaces(lin, lout, cin, cout, bins, E, fwd, bwd):
-    """The workspace of the block-diagonal op's products over bin-grouped edges: the sort's, the packed
-    table's and, backward only, the split sums'; none for the float32 forwards of the per-edge kernels, no more than the sort's for their backward and float64."""
+    """Which calls of the block-diagonal op run as products over bin-grouped edges, and the workspace
+    they take: the sort's, the packed table's and, backward only, the split sums'; none for the
+    float32 forwards of the per-edge kernels, no more than the sort's for their backward and float64."""
     lib = N.load_library()
     L, b = N.make_layout(lin, lout, cin, cout), N.make_binning(0.0, 10.0, bins, False, 0.1)
     args = (ctypes.byref(L), ctypes.byref(b), E)
