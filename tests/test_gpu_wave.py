@@ -6,8 +6,11 @@ shape-generic kernels do, and is held to the same 1e-5 of the largest entry."""
 import pytest
 import torch
 
+import flash_eq as fe
 from flash_eq import _native as NAT
 from flash_eq.ops import edgewise_linear
+from helpers import rel_err
+from oracle import layer as OL
 from oracle import wigner as OW
 from test_gpu_edgewise import _run_parity, _select
 
@@ -96,3 +99,64 @@ def test_small_degrees_keep_their_precision(dev, monkeypatch, lv, c):
     _, gF1 = grads(x, F, torch.where(small, gy, 0.0))
     assert gF1[..., w_out].abs().max() > 0
     assert torch.equal(gF[..., w_out], gF1[..., w_out] * tiny)
+
+
+@pytest.mark.parametrize("same", [True, False])
+def test_widest_instance(dev, monkeypatch, same):
+    """Four blocks and 64 channels each way (the layer composes this layout, the entry points take
+    it), with P and Q one tensor and two."""
+    _select(monkeypatch, "split")
+    torch.manual_seed(9)
+    lv, c, E = list(range(7)), 64, 45
+    layer = fe.EquivariantEdgewiseLinear(fe.Repr(lv, c), fe.Repr(lv, c), num_bins=20)
+    g = torch.Generator().manual_seed(10)
+    x, gy = torch.randn(E, c, 49, generator=g), torch.randn(E, c, 49, generator=g)
+    r, P = torch.rand(E, generator=g) * 9 + 0.3, OW.basis(lv, torch.randn(E, 3, generator=g)).float()
+    layer, rw = layer.to(dev), layer.radial_weights
+    xg, rg, Pg = x.to(dev).requires_grad_(True), r.to(dev).requires_grad_(True), P.to(dev)
+    y = edgewise_linear(xg, Pg, Pg if same else Pg.clone(), rg, rw.channel_patterns, rw.radial_functions(),
+                        layer.layout(), layer.binning(), rw.rank)
+    y.backward(gy.to(dev))
+    params, cfg = OL.module_cfg(layer)
+    xd, rd = x.double().requires_grad_(True), r.double().requires_grad_(True)
+    yref = OL.edgewise_linear(xd, P.double(), P.double(), rd, params, cfg)
+    yref.backward(gy.double())
+    assert rel_err(y, yref) < 1e-5 and rel_err(xg.grad, xd.grad) < 1e-5 and rel_err(rg.grad, rd.grad) < 1e-4
+    for name, p in rw.named_parameters():
+        assert rel_err(p.grad, params[name].grad) < 1e-5, name
+
+
+@pytest.mark.parametrize("lin,lout,cin,cout,same", [
+    ([0, 1, 2, 3], [0, 1, 2, 3], 16, 16, True),             # one block, the next basis requested ahead
+    ([0, 1, 2, 3, 4], [0, 1, 2, 3], 17, 20, False),         # two, P and Q in turn in one copy
+    ([0, 1, 2, 3, 4, 5], [0, 1, 2, 3, 4, 5], 32, 32, False),
+    ([0, 1, 2, 3, 4, 5, 6], [0, 1, 2, 3, 4, 5, 6], 32, 32, True),
+])
+def test_waves_with_many_edges(dev, monkeypatch, lin, lout, cin, cout, same):
+    """Waves that take three and four edges each (2048 and 3072 waves) leave every edge's results as
+    calls of 1000 edges do, where a wave has one: the same bits, an edge's arithmetic being the same.
+    The sums over edges agree to the rounding of their order."""
+    _select(monkeypatch, "split")
+    E, nb = 7001, 30
+    L, B = NAT.make_layout(lin, lout, cin, cout), NAT.make_binning(0.0, nb / 10.0, nb, False, 0.1)
+    g = torch.Generator(device=dev).manual_seed(11)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    x, P, gy = rnd(E, cin, L.din), rnd(E, L.din, L.din), rnd(E, cout, L.dout)
+    Q = P if same else rnd(E, L.dout, L.dout)
+    r = torch.rand(E, generator=g, device=dev) * 9 + 0.3
+    C, F = rnd(4, cout, cin), rnd(nb + 1, 4, L.wdim)
+
+    def grads(s):
+        Ps = P[s].contiguous()
+        ins = [x[s].contiguous(), r[s].contiguous(), C.clone(), F.clone()]
+        for t in ins:
+            t.requires_grad_(True)
+        y = edgewise_linear(ins[0], Ps, Ps if same else Q[s].contiguous(), ins[1], ins[2], ins[3], L, B, 4)
+        return [y.detach(), *torch.autograd.grad(y, ins, gy[s].contiguous())]
+
+    y, gx, gr, gC, gF = grads(slice(0, E))
+    parts = [grads(slice(a, a + 1000)) for a in range(0, E, 1000)]
+    for k, whole in enumerate((y, gx, gr)):
+        assert torch.equal(whole, torch.cat([p[k] for p in parts])), ("y", "gx", "gr")[k]
+    assert rel_err(gC, sum(p[3].double() for p in parts)) < 1e-5
+    assert rel_err(gF, sum(p[4].double() for p in parts)) < 1e-5
