@@ -30,13 +30,12 @@
 // rows, one memory latency per 16 channels, bounds these.  (Tiles dealt to the
 // L2s in turn, so that each read every bin's fragments: 94 and 154 us.)
 #include "blockdiag_edge.h"
+#include "tile_math.h"
 
 #include <cfloat>
 
 namespace feq {
 namespace {
-
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
 constexpr int kSS = 257;        // floats from slot to slot of the staged rows
@@ -67,10 +66,6 @@ struct Units {
     Unit u[kMaxUnits];
 };
 
-__device__ __forceinline__ v4f mfma4(float a, float b, v4f c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
 // Edge of a sorted position, with its bin state.
 struct EdgeRow {
     int64_t e;
@@ -88,11 +83,6 @@ __device__ __forceinline__ EdgeRow edge_row(const feq_binning& B, const int32_t*
     R.dtdr = eb.dtdr;
     R.s = R.r / (R.r + B.sh_scale);
     return R;
-}
-
-// q / d for q < 2^15 and d < 2^10, inv = 1 / d.
-__device__ __forceinline__ int quotient(int q, float inv) {
-    return static_cast<int>((static_cast<float>(q) + 0.5f) * inv);
 }
 
 // Rows c0 .. c0 + 15 of (E, nch, dim) of the 16 edges at e[], times scale[edge][l]

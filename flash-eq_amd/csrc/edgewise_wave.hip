@@ -37,11 +37,10 @@
 // its results are not either, but an infinity may come out as NaN: the tiles multiply
 // positions that no weight joins by zeros.
 #include "feq_internal.h"
+#include "tile_math.h"
 
 namespace feq {
 namespace {
-
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int kMaxNB = 4;       // 16-slot blocks
 constexpr int kMaxCT = 4;       // 16-channel tiles
@@ -60,10 +59,6 @@ struct GenTab {
     int32_t cin, cout, din, dout, wd;
     int32_t last;                   // reduction steps that the last block needs
 };
-
-__device__ __forceinline__ v4f mfma4(float a, float b, v4f c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 // The lane's number, opaque to the compiler: what follows from it is computed
 // where it is used.  (Held in registers over the whole edge loop, the addresses

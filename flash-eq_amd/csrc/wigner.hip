@@ -14,6 +14,7 @@
 //
 // Plan layout per irrep (lvals order), n = 2l+1 doubles blocks:
 //   V (n*n, row-major) | z (n): signed m coupling of each row | partner (n)
+#include "tile_math.h"
 #include "wigner_math.h"
 
 namespace feq {
@@ -51,11 +52,6 @@ __device__ __forceinline__ void flat_table(const WignerArgs& A, const int32_t* _
         const int n = 2 * A.lvals[k] + 1, c = col - A.off[k];
         at[j] = static_cast<int16_t>(c >= 0 && c < n ? off + (r - A.off[k]) * n + c : -1);
     }
-}
-
-// q / d for q < 2^20 and d < 2^13, inv = 1 / d.
-__device__ __forceinline__ int quotient(int q, float inv) {
-    return static_cast<int>((static_cast<float>(q) + 0.5f) * inv);
 }
 
 template <int LMAX, class T, bool FLAT, int NW>
@@ -168,18 +164,18 @@ k_wigner_lane_bwd(WignerArgs A, int stride, const double* __restrict__ plan, con
         if (l == 0) continue;                         // D = 1 is constant
         const double* V = plan + A.plan_off[k];
         if constexpr (!FLAT) {
-        __syncthreads();                              // the previous block's reads (and sInv)
-        for (int q0 = 0; q0 < nn; q0 += 64) {         // a lane's element is the same in every edge
-            const int q = q0 + lane, r = q / n;
-            const bool ok = q < nn;
-            const T* src = gM + e0 * dd + (ok ? (base + r) * dim + sInv[base + q - r * n] : 0);
+            __syncthreads();                          // the previous block's reads (and sInv)
+            for (int q0 = 0; q0 < nn; q0 += 64) {     // a lane's element is the same in every edge
+                const int q = q0 + lane, r = q / n;
+                const bool ok = q < nn;
+                const T* src = gM + e0 * dd + (ok ? (base + r) * dim + sInv[base + q - r * n] : 0);
 #pragma unroll 4
-            for (int e = wave; e < ne; e += NW) {
-                const T v = src[static_cast<int64_t>(e) * dd];
-                if (ok) sB[e * nn + q] = v;
+                for (int e = wave; e < ne; e += NW) {
+                    const T v = src[static_cast<int64_t>(e) * dd];
+                    if (ok) sB[e * nn + q] = v;
+                }
             }
-        }
-        __syncthreads();
+            __syncthreads();
         }
         const int le = lane < ne ? lane : ne - 1;
         const T* b = sB + (FLAT ? le * stride + at : le * nn);
