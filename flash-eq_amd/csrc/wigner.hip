@@ -218,8 +218,9 @@ int with_lane_lmax(const WignerArgs& A, Fn&& f) {
 }
 // Values from edge to edge of the FLAT form, 0 where its LDS would exceed
 // kFlatLds or, backward, where it would read the zeros of degrees over 2 for
-// nothing (lvals 0..3, 40 000 edges: 83 us against 41).  With few edges the
-// columns' latency is what counts forward: all degrees at once, kFewLds.  And the LDS of the form that runs (else the widest block of the edges).
+// nothing (lvals 0..3, 40 000 edges: 83 us against 41).  With few edges the columns'
+// latency is what counts forward: all degrees at once, kFewLds.  *lds: that of the form
+// that runs (else the widest block of the edges).
 template <class T>
 int lane_shape(const WignerArgs& A, bool backward, bool few, size_t* lds) {
     size_t sum = 0;
@@ -231,9 +232,16 @@ int lane_shape(const WignerArgs& A, bool backward, bool few, size_t* lds) {
     *lds = use ? flat : sizeof(T) * kLaneEdges * n * n;
     return use ? static_cast<int>(sum) : 0;
 }
-// Fewer than two workgroups per CU: more waves share an edge's columns (16
-// forward, 8 backward, as the registers allow).
-bool few_edges(int64_t E) { return ceil_div(E, kLaneEdges) < 512; }
+// Few workgroups: more waves share an edge's columns (16 forward, 8 backward, as the
+// registers allow), up to one workgroup per CU, and up to two where the degrees give
+// the waves work.  24 000 edges (375 workgroups), with and without, forward: lvals 0..2 11.1
+// and 9.0 us, 0..3 18.3 and 15.8, 0..4 27.2 and 29.4, 0..6 69.5 and 71.7; backward: 0..3
+// 24.6 and 17.1, 0..6 144 and 119, in float64 0..5 95 and 73, 0..6 187 and 211.
+template <class T>
+bool few_edges(const WignerArgs& A, int64_t E, bool backward) {
+    const bool two = backward ? sizeof(T) == 8 && max_degree(A) == kLaneL : max_degree(A) > 3;
+    return ceil_div(E, kLaneEdges) <= (two ? 512 : 256);
+}
 int set_lds(const void* fn, size_t lds) {
     if (lds > 64 * 1024)
         FEQ_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
@@ -286,10 +294,10 @@ int wigner_fwd(const int32_t* lvals, int32_t n, const double* plan, const int32_
     if (!plan || !perm || !dirs || !out) return fail(FEQ_ERR_INVALID, "NULL pointer");
     if (int rc = check_dim<T>(A)) return rc;
     size_t lds;
-    if (lane_form(A, E))
+    if (lane_form<T>(A, E, false))
         return with_lane_lmax(A, [&](auto LL) -> int {
             constexpr int L = decltype(LL)::value;
-            const bool few = few_edges(E);
+            const bool few = few_edges<T>(A, E, false);
             const int stride = lane_shape<T>(A, false, few, &lds);
             auto kern = few ? (stride ? k_wigner_lane<L, T, true, 16> : k_wigner_lane<L, T, false, 16>)
                             : (stride ? k_wigner_lane<L, T, true, 4> : k_wigner_lane<L, T, false, 4>);
@@ -311,10 +319,10 @@ int wigner_bwd(const int32_t* lvals, int32_t n, const double* plan, const int32_
     if (!plan || !perm || !dirs || !grad_out || !grad_dirs) return fail(FEQ_ERR_INVALID, "NULL pointer");
     if (int rc = check_dim<T>(A)) return rc;
     size_t lds;
-    if (lane_form(A, E))
+    if (lane_form<T>(A, E, true))
         return with_lane_lmax(A, [&](auto LL) -> int {
             constexpr int L = decltype(LL)::value;
-            const bool few = few_edges(E);
+            const bool few = few_edges<T>(A, E, true);
             const int stride = lane_shape<T>(A, true, few, &lds);
             auto kern = few ? (stride ? k_wigner_lane_bwd<L, T, true, 8> : k_wigner_lane_bwd<L, T, false, 8>)
                             : (stride ? k_wigner_lane_bwd<L, T, true, 4> : k_wigner_lane_bwd<L, T, false, 4>);

@@ -1,5 +1,5 @@
-// Wigner-D bases with degrees over kLaneL, and of few edges: a thread per (edge,
-// column) (lane_form tells which calls come here).
+// Wigner-D bases with degrees over kLaneL, of few edges or of few columns: a thread
+// per (edge, column) (lane_form tells which calls come here).
 // Included by wigner_high.hip (float32) and wigner_high64.hip (float64): one
 // translation unit each, which compile for minutes.
 #pragma once
@@ -40,7 +40,7 @@ k_wigner(WignerArgs A, int epb, const double* __restrict__ plan, const int32_t* 
         const int l = A.lvals[k], base = A.off[k], c = c0 - base;
         const double* V = plan + A.plan_off[k];
         const EdgeFrame f = sFr[el];
-        const Trig tr = trig_of(f.phi, f.ang);
+        const Trig tr = l ? trig_of(f.phi, f.ang) : Trig{};
         T* dst = sM + el * dd + base * dim + sInv[c0];   // rows base.., column j
         switch (l) {
 #define FEQ_WCASE(LL) \
@@ -90,7 +90,7 @@ k_wigner_bwd(WignerArgs A, int epb, const double* __restrict__ plan, const int32
         const int l = A.lvals[k], base = A.off[k], c = c0 - base, n = 2 * l + 1;
         const double* V = plan + A.plan_off[k];
         const EdgeFrame f = sFr[el];
-        const Trig tr = trig_of(f.phi, f.ang);
+        const Trig tr = l ? trig_of(f.phi, f.ang) : Trig{};
         // column c of dL/dD is column sInv[c] of dL/dM; rows base.. of the block
         const T* gcol = sG + el * dd + base * dim + sInv[c0];
         const T* gpar = sG + el * dd + base * dim + sInv[base + n - 1 - c];
@@ -122,20 +122,11 @@ k_wigner_bwd(WignerArgs A, int epb, const double* __restrict__ plan, const int32
 
 template <class Fn>
 int with_lmax(const WignerArgs& A, Fn&& f) {
+    if (max_degree(A) <= 2) return f(std::integral_constant<int, 2>{});
+    if (max_degree(A) <= 4) return f(std::integral_constant<int, 4>{});
     if (max_degree(A) <= kLaneL) return f(std::integral_constant<int, kLaneL>{});
     if (max_degree(A) <= 10) return f(std::integral_constant<int, 10>{});
     return f(std::integral_constant<int, 16>{});
-}
-
-// Edges per workgroup: one thread per (edge, column), the edges' matrices
-// (dim x dim values of T, see check_dim) staged in at most 64 KB of LDS.
-template <class T>
-int wigner_epb(int dim, size_t* lds) {
-    const int e = 256 / dim;
-    const int cap = static_cast<int>(kMatrixBytes / (sizeof(T) * static_cast<size_t>(dim) * dim));
-    const int epb = e < cap ? e : cap;
-    *lds = sizeof(T) * static_cast<size_t>(epb) * dim * dim;
-    return epb;
 }
 
 }  // namespace
@@ -143,8 +134,8 @@ int wigner_epb(int dim, size_t* lds) {
 template <class T>
 int wigner_high_fwd(const WignerArgs& A, const double* plan, const int32_t* perm, int64_t E, const T* dirs, T* out,
                     hipStream_t s) {
-    size_t lds;
-    const int epb = wigner_epb<T>(A.dim, &lds);
+    const int epb = column_edges<T>(A);
+    const size_t lds = sizeof(T) * static_cast<size_t>(epb) * A.dim * A.dim;
     return with_lmax(A, [&](auto LL) -> int {
         auto kern = k_wigner<decltype(LL)::value, T>;
         FEQ_LAUNCH("k_wigner", kern, dim3(ceil_div(E, epb)), dim3(256), lds, s, A, epb, plan, perm, E, dirs, out);
@@ -155,8 +146,8 @@ int wigner_high_fwd(const WignerArgs& A, const double* plan, const int32_t* perm
 template <class T>
 int wigner_high_bwd(const WignerArgs& A, const double* plan, const int32_t* perm, int64_t E, const T* dirs,
                     const T* grad_out, T* grad_dirs, hipStream_t s) {
-    size_t lds;
-    const int epb = wigner_epb<T>(A.dim, &lds);
+    const int epb = column_edges<T>(A);
+    const size_t lds = sizeof(T) * static_cast<size_t>(epb) * A.dim * A.dim;
     return with_lmax(A, [&](auto LL) -> int {
         auto kern = k_wigner_bwd<decltype(LL)::value, T>;
         FEQ_LAUNCH("k_wigner_bwd", kern, dim3(ceil_div(E, epb)), dim3(256), lds, s, A, epb, plan, perm, E, dirs,

@@ -28,22 +28,6 @@ template <class T>
 int wigner_high_bwd(const WignerArgs& A, const double* plan, const int32_t* perm, int64_t E, const T* dirs,
                     const T* grad_out, T* grad_dirs, hipStream_t s);
 
-// The lane kernels take degrees up to kLaneL.  Degrees 5 and 6 on few edges are
-// bound by a column's latency (its unrolled code is fetched anew in each launch),
-// and a thread per column has all columns at once: lvals 0..6, forward and
-// backward, 523 edges 23 and 40 us against 33 and 66, 5000 edges 56 and 170
-// against 35 and 69.
-constexpr int64_t kColumnEdges = 1536;
-inline int max_degree(const WignerArgs& A) {
-    int lmax = 0;
-    for (int i = 0; i < A.nirr; ++i) lmax = A.lvals[i] > lmax ? A.lvals[i] : lmax;
-    return lmax;
-}
-inline bool lane_form(const WignerArgs& A, int64_t E) {
-    const int l = max_degree(A);
-    return l <= 4 || (l <= kLaneL && E > kColumnEdges);
-}
-
 // Representations whose matrix exceeds 64 KB are refused (dimensions over 128 in
 // float32, 90 in float64), whatever kernel the call would take: the column kernel
 // stages whole matrices, and every kernel holds perm in FEQ_MAX_SLOTS entries.
@@ -54,6 +38,40 @@ int check_dim(const WignerArgs& A) {
     if (sizeof(T) * static_cast<size_t>(A.dim) * A.dim > kMatrixBytes)
         return fail(FEQ_ERR_UNSUPPORTED, "representation dimension %d too large", A.dim);
     return FEQ_OK;
+}
+
+inline int max_degree(const WignerArgs& A) {
+    int lmax = 0;
+    for (int i = 0; i < A.nirr; ++i) lmax = A.lvals[i] > lmax ? A.lvals[i] : lmax;
+    return lmax;
+}
+// Edges per workgroup of the column kernels: one thread per (edge, column) of 256, the
+// edges' matrices (dim x dim values of T) staged in at most kMatrixBytes of LDS.
+template <class T>
+int column_edges(const WignerArgs& A) {
+    const int e = 256 / A.dim;
+    const int cap = static_cast<int>(kMatrixBytes / (sizeof(T) * static_cast<size_t>(A.dim) * A.dim));
+    return e < cap ? e : cap;
+}
+
+// The lane kernels take degrees up to kLaneL, where the column kernels' workgroups do
+// not all run at once: a thread per column has all columns of its edges at once, a
+// wave of the lane kernels one after the other (and degrees 5 and 6, whose unrolled code is
+// fetched anew in each launch, twice as many).  Float32, forward and backward in us,
+// column kernels and these: lvals 0..4, 2000 edges (200 workgroups) 11.5 and 13.7,
+// 13.5 and 21.3; 4500 edges (450) 15.4 and 24.9, 14.4 and 21.4; lvals 0..3, 3300 edges
+// (207) 8.6 and 10.5, 9.6 and 11.8; 4500 (282) 10.5 and 18.3, 9.7 and 11.8; lvals 0..6,
+// 2000 edges (400) 28.8 and 62.5, 34.2 and 62.3; 2600 (520) 40.7 and 87, 34.6 and 62.4.
+// In float64 the lines are the same, but forward at degrees 5 and 6: lvals 0..6, 2000
+// edges (667) 34 and 47, 3300 (1100) 50 and 47.  Matrices of up to 4 columns leave most of
+// a lane kernel's waves without one: degree 0, 640 000 edges 9.1 and 18.7, 32.4 and
+// 47.6; degrees 0 and 1 34.9 and 60.5, 37.2 and 63.2 (two of degree 1 51 and 100, 44 and 85).
+template <class T>
+bool lane_form(const WignerArgs& A, int64_t E, bool backward) {
+    const int lmax = max_degree(A);
+    if (lmax > kLaneL || A.dim <= 4) return false;
+    const int at_once = lmax <= 4 ? 256 : sizeof(T) == 8 && !backward ? 768 : 512;
+    return ceil_div(E, column_edges<T>(A)) > at_once;
 }
 
 namespace {
