@@ -160,3 +160,42 @@ def test_waves_with_many_edges(dev, monkeypatch, lin, lout, cin, cout, same):
         assert torch.equal(whole, torch.cat([p[k] for p in parts])), ("y", "gx", "gr")[k]
     assert rel_err(gC, sum(p[3].double() for p in parts)) < 1e-5
     assert rel_err(gF, sum(p[4].double() for p in parts)) < 1e-5
+
+
+@pytest.mark.parametrize("lin,lout,cin,cout", [([0, 1, 2, 3], [0, 1, 2, 3], 20, 16), ([0, 1, 2, 3, 4], [0, 2], 33, 24),
+                                               ([0, 1, 2, 3, 4, 5, 6], [0, 1, 2, 3, 4, 5, 6], 16, 16)])
+def test_infinities_and_nan_stay_where_the_generic_kernels_leave_them(dev, monkeypatch, lin, lout, cin, cout):
+    """Which results of the layer are finite is what the shape-generic kernels make it: infinite or NaN
+    features and gradients reach their own edge's results, the patterns' gradients of their
+    channel and the radial functions' gradients of their two bins, a radial function its bins' edges, a
+    pattern its channel; what else a call returns is unchanged."""
+    E, nb, inf, nan = 2600, 30, float("inf"), float("nan")
+    L, B = NAT.make_layout(lin, lout, cin, cout), NAT.make_binning(0.0, nb / 10.0, nb, False, 0.1)
+    g = torch.Generator().manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    x, gy, v = rnd(E, cin, L.din), rnd(E, cout, L.dout), rnd(E, 3)
+    P, Q = OW.basis(lin, v).float().to(dev), OW.basis(lout, v).float().to(dev)
+    r, C, F = torch.rand(E, generator=g) * 9 + 0.3, rnd(4, cout, cin), rnd(nb + 1, 4, L.wdim)
+
+    def grads(path, x, gy, C, F):
+        _select(monkeypatch, path)
+        ins = [t.to(dev).requires_grad_(True) for t in (x, r, C, F)]
+        y = edgewise_linear(ins[0], P, Q, ins[1], ins[2], ins[3], L, B, 4)
+        return [y.detach(), *torch.autograd.grad(y, ins, gy.to(dev))]
+
+    clean = grads("split", x, gy, C, F)
+    bad = {k: t.clone() for k, t in (("x", x), ("gy", gy), ("C", C), ("F", F))}
+    bad["x"][7, 3, 1], bad["x"][2599, 0, -1] = inf, nan
+    bad["gy"][1200, 2, 0] = -inf
+    bad["C"][1, 5, 4] = inf
+    bad["F"][11, 2, 0] = nan
+    for k in ("x", "gy", "C", "F"):
+        args = {"x": x, "gy": gy, "C": C, "F": F, k: bad[k]}
+        got, ref = grads("split", **args), grads("generic", **args)
+        for name, a, b, c in zip(("y", "gx", "gr", "gC", "gF"), got, ref, clean):
+            fin = torch.isfinite(b)
+            assert torch.equal(torch.isfinite(a), fin), (k, name)
+            if k in ("x", "gy") and name in ("y", "gx", "gr"):
+                same = torch.ones(E, dtype=torch.bool, device=dev)
+                same[[7, 2599] if k == "x" else [1200]] = False
+                assert torch.equal(a[same], c[same]), (k, name)
