@@ -6,16 +6,17 @@
 // them.  Here a workgroup takes 16 edges in the order of their bins (the stable
 // CSR by bin), one 16-channel tile of outputs, and reads each table row once for
 // the 16:
-//   forward   Y[co, e] (o)  += M_w[co, ci] X[ci, e] (i) + u_e D_w[co, ci] X[ci, e] (i)
-//   gradient  GX[ci, e] (i) += M_w[co, ci]^T G[co, e] (o) + u_e D_w^T G
+//   forward   Y[co, e] (o)  += W_w,e[co, ci] X[ci, e] (i)
+//   gradient  GX[ci, e] (i) += W_w,e[co, ci]^T G[co, e] (o)
 //   table     dT_w[co, ci]  += sum over e of G[co, e] (o) X[ci, e] (i)
-// with X = s^l x, G = s^l gy, M the mean of the bin's row and the next one, D the
-// next row's difference to it, u = t - 1/2.  M + u D keeps the per-edge kernels'
-// precision: inside a bin its two terms are no larger than they have to be (with the
-// row itself and t D, the errors of y and dx are 1.1 to 1.5 times theirs), and where
-// linear bins extrapolate (|t| >> 1) it stays well conditioned.  The table is first
-// packed into operand order (k_bdm_pack), M and D side by side, zero-padded to 16
-// channels.
+// with X = s^l x, G = s^l gy and W_e X = (1 - t_e) (T X) + t_e (T' X), T and T' the
+// bin's row and the next one: neither term is larger than it has to be, and at either
+// end of a bin its row alone counts.  Edges outside the bins, where the first and the
+// last one extrapolate (|t| >> 1), take T X + t D X with the rows' difference D, which is
+// well conditioned there as in the per-edge kernels; the distance gradient takes D X
+// everywhere.  (T + t D for every edge: errors of y and dx 1.1 to 1.5 times the per-edge
+// kernels'; the rows' mean and D: a small row beside a large one lost to it.)  The table
+// is first packed into operand order (k_bdm_pack), zero-padded to 16 channels.
 //
 // Lane l = (c = l % 16, g = l / 16); a reduction step r takes the indices
 // 4 r + g: the staged rows [slot][channel][edge] (257 floats from slot to slot)
@@ -24,8 +25,8 @@
 // products of one summed index and 16 channels by themselves, then added.
 //
 // Lvals 0..2 x 32, 20 000 edges, 65 table rows, the per-edge kernels and these:
-// forward 1163 us, now 82 + 18 (pack) + 35 (sort by bin); input and distance
-// gradients 816 + 1724, now 133 + 18 (pack); table gradient 2256, now 156 + 12.
+// forward 1163 us, now 86 + 13 (pack) + 35 (sort by bin); input and distance
+// gradients 816 + 1724, now 155 + 14 (pack); table gradient 2256, now 159 + 12.
 // The matrix steps alone would take 20 to 40 us each: the staging of 16 edges'
 // rows, one memory latency per 16 channels, bounds these.  (Tiles dealt to the
 // L2s in turn, so that each read every bin's fragments: 94 and 154 us.)
@@ -124,42 +125,70 @@ __device__ __forceinline__ bool finite(float v) { return fabsf(v) <= FLT_MAX; }
 
 constexpr int kPow = 32;        // powers of s kept per edge (+ 1: no bank conflicts)
 
-// Operand order of the table: fragment (b, w, row tile, reduction tile) holds for
-// lane (c, g) the four values r of M, then of D: M[co, ci] with, forward, co = 16
-// row + c and ci = 16 red + 4 r + g, and transposed (TR) with ci = 16 row + c and
-// co = 16 red + 4 r + g.  A workgroup packs wchunk weights of the 16 x 16 channels of
-// one bin (all of them in turn left the chip idle: lvals 0..6 x 16, 64 bins, 155 us).
-template <bool TR>
+// Operand order of the table: fragment (row b, w, row tile, reduction tile) holds for
+// lane (c, g) four values r: T[co, ci] with, forward, co = 16 row + c and ci = 16 red
+// + 4 r + g, and transposed (TR) with ci = 16 row + c and co = 16 red + 4 r + g.  The
+// num_bins + 1 rows, then the differences D of the bins that need them: all (ALLD) or the
+// first and the last.  A workgroup packs wchunk weights of the 16 x 16 channels of one
+// row (all weights in turn left the chip idle: lvals 0..6 x 16, 64 bins, 155 us).
+__host__ __device__ constexpr int diff_rows(int nb, bool alld) { return alld ? nb : nb < 2 ? nb : 2; }
+__device__ __forceinline__ int diff_row(int bin, int nb, bool alld) { return nb + 1 + (alld ? bin : bin ? 1 : 0); }
+
+__host__ __device__ constexpr int pack_floats(int wchunk) { return 256 * (wchunk | 1) + 16; }
+
+// Values that a thread requests before it uses the first (one at a time: 22 us a packing
+// at lvals 0..2 x 32 and 64 bins instead of 13).
+constexpr int kPackAhead = 5;
+
+template <bool TR, bool ALLD>
 __global__ void __launch_bounds__(kThreads)
-k_bdm_pack(const float* __restrict__ table, int cout, int cin, int wd, int wchunk, float* __restrict__ frag) {
-    extern __shared__ float sm[];   // [2][16 * 16][wchunk + 1]
-    const int64_t b = blockIdx.x;
+k_bdm_pack(const float* __restrict__ table, int nb, int cout, int cin, int wd, int wchunk, float* __restrict__ frag) {
+    // T, then D: [16][16][ls], an odd number of floats from channel to channel either way
+    extern __shared__ float sm[];
+    const int b = blockIdx.x;
     const int nci = (cin + 15) / 16, nco = (cout + 15) / 16;
     const int cot = blockIdx.y / nci, cit = blockIdx.y % nci;
     const int row = TR ? cit : cot, red = TR ? cot : cit, nrow = TR ? nci : nco, nred = TR ? nco : nci;
     const int64_t ts = static_cast<int64_t>(cout) * cin * wd;
-    const int w0 = blockIdx.z * wchunk, nw = wd - w0 < wchunk ? wd - w0 : wchunk, ls = wchunk + 1;
-    for (int q = threadIdx.x; q < 256 * nw; q += kThreads) {
-        const int ch = q / nw, w = q - ch * nw, co = 16 * cot + ch / 16, ci = 16 * cit + ch % 16;
-        const bool ok = co < cout && ci < cin;
-        const int64_t at = ok ? b * ts + (static_cast<int64_t>(co) * cin + ci) * wd + w0 + w : 0;
-        const float lo = table[at], hi = table[ok ? at + ts : 0];
-        sm[ch * ls + w] = ok ? 0.5f * lo + 0.5f * hi : 0.0f;
-        sm[(256 + ch) * ls + w] = ok ? hi - lo : 0.0f;
+    const int w0 = blockIdx.z * wchunk, nw = wd - w0 < wchunk ? wd - w0 : wchunk;
+    const int ls = wchunk | 1, half = pack_floats(wchunk);
+    const bool diff = b < nb && (ALLD || b == 0 || b == nb - 1);
+    const float inw = 1.0f / static_cast<float>(nw);
+    for (int w1 = 0; w1 < nw; w1 += kPackAhead) {       // kThreads values a step, kPackAhead steps in flight
+        float lo[kPackAhead], hi[kPackAhead];
+        int to[kPackAhead];
+#pragma unroll
+        for (int u = 0; u < kPackAhead; ++u) {
+            const int q = kThreads * (w1 + u < nw ? w1 + u : nw - 1) + threadIdx.x;
+            const int ch = quotient(q, inw), w = q - ch * nw, co = 16 * cot + ch / 16, ci = 16 * cit + ch % 16;
+            const bool ok = co < cout && ci < cin;
+            const int64_t at = ok ? b * ts + (static_cast<int64_t>(co) * cin + ci) * wd + w0 + w : 0;
+            lo[u] = table[at];
+            hi[u] = table[ok && diff ? at + ts : at];
+            lo[u] = ok ? lo[u] : 0.0f;
+            hi[u] = ok ? hi[u] : 0.0f;
+            to[u] = ch * ls + ch / 16 + w;
+        }
+#pragma unroll
+        for (int u = 0; u < kPackAhead; ++u) {
+            sm[to[u]] = lo[u];
+            if (diff) sm[half + to[u]] = hi[u] - lo[u];
+        }
     }
     __syncthreads();
-    for (int q = threadIdx.x; q < 512 * nw; q += kThreads) {
-        const int w = q / 512, k = q - w * 512, d = k >> 8, l = (k & 255) >> 2, r = k & 3;
+    for (int q = threadIdx.x; q < (diff ? 512 : 256) * nw; q += kThreads) {
+        const int d = q >= 256 * nw, w = q / 256 - d * nw, k = q & 255, l = k >> 2, r = k & 3;
         const int a = l & 15, z = 4 * r + (l >> 4);       // row and reduction channel
         const int ch = TR ? z * 16 + a : a * 16 + z;
-        frag[((((b * wd + w0 + w) * nrow + row) * nred + red) * 2 + d) * 256 + l * 4 + r] = sm[(256 * d + ch) * ls + w];
+        const int64_t fr = d ? diff_row(b, nb, ALLD) : b;
+        frag[(((fr * wd + w0 + w) * nrow + row) * nred + red) * 256 + k] = sm[half * d + ch * ls + ch / 16 + w];
     }
 }
 
 // ---------------------------------------------------------------------------
-// A tile's product for up to MAXP pairs per wave: acc[p] += M S + u (D S), or with
-// GD acc[p] += M S, accD[p] += D S, accS[p] += l (M S + u (D S)) (S: the staged
-// rows, l: the degree of the summed slot; the distance gradient's three sums).
+// A tile's product for up to MAXP pairs per wave: acc[p] += W S, and with GD accD[p] +=
+// D S, accS[p] += l (W S) (S: the staged rows, l: the degree of the summed slot; the
+// distance gradient's three sums).
 template <int MAXP, bool GD>
 struct TileAcc {
     v4f a[MAXP][2];
@@ -171,33 +200,39 @@ struct TileAcc {
 // (re += a re - b im, im += a im + b re).  in: whether the lane's column, an edge,
 // is of this bin.  The other columns' products are formed and not taken: multiplied
 // by zeros instead, a row of the table with an infinity or NaN would reach edges
-// that never read it.
+// that never read it.  outer: the columns outside the bins, else those inside.
 template <int MAXP, bool GD, int SIGN>
-__device__ __forceinline__ void tile_product(const Pairs& PT, int wave, const float* __restrict__ frag, int64_t bin, int wd,
-                                             int nrow, int row, int nred, int red, const float* st, bool in, float u,
-                                             const int* deg, TileAcc<MAXP, GD>& A) {
-    const int lane = threadIdx.x & 63;
-    const int64_t wstride = static_cast<int64_t>(nrow) * nred * 512;
-    const float* f0 = frag + ((bin * wd * nrow + row) * nred + red) * 512;
+__device__ __forceinline__ void tile_product(const Pairs& PT, int wave, const float* __restrict__ frag, int bin, int nb,
+                                             int wd, int nrow, int row, int nred, int red, const float* st, bool outer,
+                                             bool in, float t, const int* deg, TileAcc<MAXP, GD>& A) {
+    const unsigned lane = threadIdx.x & 63;
+    const int64_t wstride = static_cast<int64_t>(nrow) * nred * 256, bstride = wstride * wd;
+    const float* f0 = frag + (static_cast<int64_t>(row) * nred + red) * 256;
+    const float* fT = f0 + bin * bstride;
+    const float* fD = f0 + diff_row(bin, nb, GD) * bstride;
+    const float* fB = outer ? fD : fT + bstride;
+    const float ta = outer ? 1.0f : 1.0f - t;
     const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int p = 0; p < MAXP; ++p) {
         if (wave + 4 * p >= PT.n) break;
         const Pair P = PT.p[wave + 4 * p];
-        v4f Mn[2], Dn[2];       // the next summed index's fragments
+        v4f Tn[2], Bn[2], Dn[2];        // the next summed index's fragments
         auto fetch = [&](int k) {
-            const float* fa = f0 + (P.w + k * P.step) * wstride;
-            Mn[0] = *reinterpret_cast<const v4f*>(fa + 4 * lane);
-            Dn[0] = *reinterpret_cast<const v4f*>(fa + 256 + 4 * lane);
+            const int64_t at = (P.w + k * P.step) * wstride + 4 * lane;
+            Tn[0] = *reinterpret_cast<const v4f*>(fT + at);
+            Bn[0] = *reinterpret_cast<const v4f*>(fB + at);
+            if constexpr (GD) Dn[0] = *reinterpret_cast<const v4f*>(fD + at);
             if (P.z == 2) {
-                Mn[1] = *reinterpret_cast<const v4f*>(fa + wstride + 4 * lane);
-                Dn[1] = *reinterpret_cast<const v4f*>(fa + wstride + 256 + 4 * lane);
+                Tn[1] = *reinterpret_cast<const v4f*>(fT + at + wstride);
+                Bn[1] = *reinterpret_cast<const v4f*>(fB + at + wstride);
+                if constexpr (GD) Dn[1] = *reinterpret_cast<const v4f*>(fD + at + wstride);
             }
         };
         fetch(0);
         for (int k = 0; k < P.n; ++k) {
             const float* sr = st + (P.other + P.z * k) * kSS;
-            const v4f M[2] = {Mn[0], Mn[1]}, D[2] = {Dn[0], Dn[1]};
+            const v4f T[2] = {Tn[0], Tn[1]}, T1[2] = {Bn[0], Bn[1]}, D[2] = {Dn[0], Dn[1]};
             v4f S[2];
             if (k + 1 < P.n) fetch(k + 1);
 #pragma unroll
@@ -206,35 +241,34 @@ __device__ __forceinline__ void tile_product(const Pairs& PT, int wave, const fl
 #pragma unroll
                 for (int r = 0; r < 4; ++r) S[1][r] = sr[kSS + 64 * r + lane];
             }
-            // component c of the product of the (a, b) fragments Q and the rows S
-            auto product = [&](const v4f (&Q)[2], v4f (&acc)[2]) {
-                acc[0] = acc[1] = zero;
+            // components of the product of the (a, b) fragments Q and the rows S
+            auto product = [&](const v4f (&Q)[2], v4f (&out)[2]) {
+                out[0] = out[1] = zero;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) acc[0] = mfma4(Q[0][r], S[0][r], acc[0]);
+                for (int r = 0; r < 4; ++r) out[0] = mfma4(Q[0][r], S[0][r], out[0]);
                 if (P.z == 2) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        acc[1] = mfma4(Q[0][r], S[1][r], acc[1]);
-                        acc[0] = mfma4(Q[1][r], SIGN > 0 ? S[1][r] : -S[1][r], acc[0]);
-                        acc[1] = mfma4(Q[1][r], SIGN > 0 ? -S[0][r] : S[0][r], acc[1]);
+                        out[1] = mfma4(Q[0][r], S[1][r], out[1]);
+                        out[0] = mfma4(Q[1][r], SIGN > 0 ? S[1][r] : -S[1][r], out[0]);
+                        out[1] = mfma4(Q[1][r], SIGN > 0 ? -S[0][r] : S[0][r], out[1]);
                     }
                 }
             };
-            v4f ms[2], ds[2];
-            product(M, ms);
-            product(D, ds);
+            v4f ts[2], bs[2], ds[2];
+            product(T, ts);
+            product(T1, bs);
+            if constexpr (GD) product(D, ds);
             const float l = GD ? static_cast<float>(deg[P.other + P.z * k]) : 0.0f;
 #pragma unroll
             for (int z = 0; z < 2; ++z)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float both = fmaf(u, ds[z][r], ms[z][r]);
+                    const float v = in ? fmaf(t, bs[z][r], ta * ts[z][r]) : 0.0f;
+                    A.a[p][z][r] += v;
                     if constexpr (GD) {
-                        A.a[p][z][r] = in ? A.a[p][z][r] + ms[z][r] : A.a[p][z][r];
-                        A.d[p][z][r] = in ? A.d[p][z][r] + ds[z][r] : A.d[p][z][r];
-                        A.s[p][z][r] = in && l != 0.0f ? fmaf(l, both, A.s[p][z][r]) : A.s[p][z][r];
-                    } else {
-                        A.a[p][z][r] = in ? A.a[p][z][r] + both : A.a[p][z][r];
+                        A.d[p][z][r] += in ? ds[z][r] : 0.0f;
+                        A.s[p][z][r] = fmaf(l, v, A.s[p][z][r]);
                     }
                 }
         }
@@ -259,8 +293,8 @@ __device__ __forceinline__ void clear(TileAcc<MAXP, GD>& A) {
 // GD: the distance gradient's share of this channel tile to gpart[tile of
 // channels][position's edge], from xo, the features on the produced side.  Edges
 // whose results hold an infinity or NaN are formed again from the unpacked table,
-// as the per-edge kernels form them: M + u D of infinite terms is NaN where
-// the interpolated weight is not.
+// as the per-edge kernels form them: two infinite products are NaN where the
+// interpolated weight's is not.
 template <int MAXP, bool GD, int SIGN>
 __global__ void __launch_bounds__(kThreads, 2)
 k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __restrict__ perm,
@@ -270,7 +304,7 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
     extern __shared__ float st[];
     __shared__ float sPow[16 * (kPow + 1)];
     __shared__ int64_t sE[16];
-    __shared__ int sLo[16];
+    __shared__ int sKey[16];            // 2 bin, + 1 where the edge lies outside the bins
     __shared__ float sRed[4 * 64];
     __shared__ int sBad[16];
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
@@ -286,9 +320,10 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
     for (int q = threadIdx.x; q < din; q += kThreads) din_deg[q] = SIGN > 0 ? L.lslot_in[q] : L.lslot_out[q];
     for (int q = threadIdx.x; q < dout; q += kThreads) dout_deg[q] = SIGN > 0 ? L.lslot_out[q] : L.lslot_in[q];
     const EdgeRow R = edge_row(B, perm, dist, p0 + (c < n ? c : n - 1), E);
+    const int key = 2 * R.lo + ((R.lo == 0 && R.t < 0.0f) || (R.lo == B.num_bins - 1 && R.t > 1.0f));
     if (threadIdx.x < 16) {
         sE[c] = R.e;
-        sLo[c] = R.lo;
+        sKey[c] = key;
         sBad[c] = 0;
         float p = 1.0f;
         for (int l = 0; l < kPow; ++l) {
@@ -305,14 +340,19 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
         stage_rows<true>(x, nch, 16 * red, din, sE, sPow, kPow + 1, din_deg, n, st);
         __syncthreads();
         for (int p = 0; p < n;) {       // the tile's bins, in order
-            const int bin = sLo[p];
-            tile_product<MAXP, GD, SIGN>(PT, wave, frag, bin, wd, nrow, row, nred, red, st,
-                                         R.lo == bin, R.t - 0.5f, din_deg, A);
-            while (p < n && sLo[p] == bin) ++p;
+            const int bin = __builtin_amdgcn_readfirstlane(sKey[p] >> 1);
+            int kinds = 0;
+            while (p < n && sKey[p] >> 1 == bin) kinds |= 1 << (sKey[p++] & 1);
+            kinds = __builtin_amdgcn_readfirstlane(kinds);
+#pragma unroll 1
+            for (int outer = 0; outer < 2; ++outer)
+                if (kinds >> outer & 1)
+                    tile_product<MAXP, GD, SIGN>(PT, wave, frag, bin, B.num_bins, wd, nrow, row, nred, red, st, outer,
+                                                 key == 2 * bin + outer, R.t, din_deg, A);
         }
     }
     if constexpr (GD) {
-        // x on the produced side: sum of x accD, and of l x (acc + u accD) + x accS
+        // x on the produced side: sum of x accD, and of l x acc + x accS
         __syncthreads();
         stage_rows<true>(xo, noch, 16 * row, dout, sE, sPow, kPow + 1, dout_deg, n, st);
         __syncthreads();
@@ -328,7 +368,7 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
                     const float q = st[(P.slot + z) * kSS + (4 * g + r) * 16 + c];
                     const v4f a = z ? A.a[p][1] : A.a[p][0], d = z ? A.d[p][1] : A.d[p][0], s = z ? A.s[p][1] : A.s[p][0];
                     atr[r] += q * d[r];
-                    asr[r] += q * (l * (a[r] + (R.t - 0.5f) * d[r]) + s[r]);
+                    asr[r] += q * (l * a[r] + s[r]);
                 }
             }
         }
@@ -357,11 +397,7 @@ k_bdm_apply(feq_layout L, Pairs PT, feq_binning B, int64_t E, const int32_t* __r
         for (int z = 0; z < 2; ++z)
             if (z < P.z) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float v = A.a[p][z][r];
-                    if constexpr (GD) v += (R.t - 0.5f) * A.d[p][z][r];
-                    st[(P.slot + z) * kSS + (4 * g + r) * 16 + c] = v * sc;
-                }
+                for (int r = 0; r < 4; ++r) st[(P.slot + z) * kSS + (4 * g + r) * 16 + c] = A.a[p][z][r] * sc;
             }
     }
     __syncthreads();
@@ -571,20 +607,21 @@ bool build_units(const feq_layout& L, Units& T) {
 }
 
 int tiles16(int n) { return (n + 15) / 16; }
-// Weights per workgroup of the packing: up to 48 KB of LDS, or 16 where they are more.
+// Weights per workgroup of the packing: up to 47 KB of LDS, or 16 where they are more.
 int pack_chunk(int wd) { return wd < 24 ? wd : 16; }
-size_t frag_floats(const feq_layout& L, const feq_binning& B) {
-    return static_cast<size_t>(B.num_bins) * L.wdim * tiles16(L.cin) * tiles16(L.cout) * 512;
+// alld: the differences of every bin (the distance gradient rides along).
+size_t frag_floats(const feq_layout& L, const feq_binning& B, bool alld) {
+    return (static_cast<size_t>(B.num_bins) + 1 + diff_rows(B.num_bins, alld)) * L.wdim * tiles16(L.cin) * tiles16(L.cout) * 256;
 }
 constexpr int kMaxP = 8;        // pairs per wave; 4 with the distance gradient's sums
 
-template <bool TR>
+template <bool TR, bool ALLD>
 int pack(const feq_layout& L, const feq_binning& B, const float* table, float* frag, hipStream_t s) {
-    auto k = k_bdm_pack<TR>;
+    auto k = k_bdm_pack<TR, ALLD>;
     const int chunk = pack_chunk(L.wdim);
     FEQ_LAUNCH("k_bdm_pack", k,
-               dim3(B.num_bins, tiles16(L.cin) * tiles16(L.cout), static_cast<unsigned>(ceil_div(L.wdim, chunk))),
-               dim3(kThreads), sizeof(float) * 512 * (chunk + 1), s, table, L.cout, L.cin, L.wdim, chunk, frag);
+               dim3(B.num_bins + 1, tiles16(L.cin) * tiles16(L.cout), static_cast<unsigned>(ceil_div(L.wdim, chunk))),
+               dim3(kThreads), sizeof(float) * 2 * pack_floats(chunk), s, table, B.num_bins, L.cout, L.cin, L.wdim, chunk, frag);
     return FEQ_OK;
 }
 
@@ -592,10 +629,10 @@ int pack(const feq_layout& L, const feq_binning& B, const float* table, float* f
 
 // Where the products run.  Their fixed cost is the sort by bin and two packings,
 // about 60 us, against 3 to 5 ps per edge and table weight in a per-edge kernel: from
-// kMinWork edges times weights on they are faster (measured around it, forward
-// and backward: lvals 0..2 x 16, 8000 edges 115 -> 60 and 943 -> 109 us; x 32, 1000 edges
-// 88 -> 57 and 380 -> 103; lvals 0..6 x 16, 440 edges 225 -> 164 and 767 -> 640; x 1,
-// 1 400 000 edges 1434 -> 1439 and 64.6 -> 5.2 ms).
+// kMinWork edges times weights on they are faster.  Around it, forward and backward in us,
+// per-edge kernels and products: lvals 0..2 x 16, 8000 edges 112 and 937, 58 and 109; x 32,
+// 1300 edges 98 and 434, 60 and 110; lvals 0..6 x 16, 440 edges 226 and 785, 146 and 622;
+// x 8, 20 000 edges 83 and 1415, 80 and 165.
 constexpr double kMinWork = 2.5e7;
 // The packed table takes no more memory than this.
 constexpr size_t kMaxFragBytes = size_t{4} << 30;
@@ -612,25 +649,27 @@ static bool covers(const feq_layout& L, const feq_binning& B, int64_t E) {
     if (!build_pairs(L, false, P) || P.n > 4 * kMaxP || !build_pairs(L, true, P) || P.n > 4 * kMaxP) return false;
     if (!build_units(L, U)) return false;
     return static_cast<double>(E) * L.cin * L.cout * L.wdim >= kMinWork &&
-           frag_floats(L, B) * sizeof(float) <= kMaxFragBytes;
+           frag_floats(L, B, true) * sizeof(float) <= kMaxFragBytes;
 }
 
 // The backward takes them wherever they are covered: it sorts in any case, and its
 // per-edge distance and table gradients are slow enough that the packing of more bins
-// than edges pays too (lvals 0..2 x 32, 4096 bins, 2000 edges: 1403 -> 946 us).
+// than edges pays too (lvals 0..2 x 32, 4096 bins, 2000 edges: 1399 -> 837 us; x 1, padded
+// to 16, 4096 bins, 1 400 000 edges: 12.0 -> 5.0 ms).
 bool bdm_bwd_supported(const feq_layout& L, const feq_binning& B, int64_t E) { return covers(L, B, E); }
 
-// The forward where the packing does not cost more than the per-edge kernel: 7 ps per
-// bin and packed weight (channels padded to 16) against 4 per edge and weight, or
-// against the 2.5 ns per weight that a few edges take together.  Lvals 0..2 x 32,
-// per-edge kernel and products: 1000 bins, 1400 edges 165 and 183 us, 2000 edges 231 and
-// 182; 4096 bins, 4096 edges 455 and 567, 8000 edges 857 and 584; lvals 0..6 x 32,
-// 100 bins, 131 edges 831 and 694.
+// The forward where the packing does not cost more than the per-edge kernel: 4 ps per
+// packed weight (rows times weights of channels padded to 16) against 4 per edge and weight,
+// or against the 2.5 ns per weight that a few edges take together.  Lvals 0..2, per-edge
+// kernel and products: x 32, 4096 bins, 2000 edges 244 and 339 us, 4096 edges 456 and 361;
+// 1000 bins, 1400 edges 166 and 164; x 64, 1000 bins, 700 edges 355 and 438, 1000 edges
+// 453 and 440; x 16, 10 000 bins, 8000 edges 223 and 223; lvals 0..6 x 32, 100 bins, 131
+// edges 829 and 775; x 128, 7 edges 8.4 and 3.1 ms.
 bool bdm_fwd_supported(const feq_layout& L, const feq_binning& B, int64_t E) {
     if (!covers(L, B, E)) return false;
     const double weights = static_cast<double>(L.cin) * L.cout * L.wdim;
-    const double packed = static_cast<double>(frag_floats(L, B)) / 2;     // bins times padded weights
-    return 7.0 * packed <= weights * (4.0 * static_cast<double>(E) > 2500.0 ? 4.0 * static_cast<double>(E) : 2500.0);
+    const double packed = static_cast<double>(frag_floats(L, B, false));     // rows times padded weights
+    return 4.0 * packed <= weights * (4.0 * static_cast<double>(E) > 2500.0 ? 4.0 * static_cast<double>(E) : 2500.0);
 }
 
 namespace {
@@ -648,13 +687,13 @@ int table_splits(const feq_layout& L, const feq_binning& B, int64_t E, int units
 }
 }  // namespace
 
-size_t bdm_fwd_workspace(const feq_layout& L, const feq_binning& B) { return sizeof(float) * frag_floats(L, B); }
+size_t bdm_fwd_workspace(const feq_layout& L, const feq_binning& B) { return sizeof(float) * frag_floats(L, B, false); }
 
 size_t bdm_bwd_workspace(const feq_layout& L, const feq_binning& B, int64_t E) {
     Units U;
     build_units(L, U);
     const int splits = table_splits(L, B, E, U.n);
-    return sizeof(float) * (align_up(frag_floats(L, B), 64) + align_up(static_cast<size_t>(E) * tiles16(L.cin), 64) +
+    return sizeof(float) * (align_up(frag_floats(L, B, true), 64) + align_up(static_cast<size_t>(E) * tiles16(L.cin), 64) +
                             (splits > 1 ? splits * table_floats(L, B) : 0));
 }
 
@@ -669,7 +708,7 @@ int bdm_fwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* x
     Pairs P;
     build_pairs(L, false, P);
     float* frag = static_cast<float*>(ws);
-    if (int rc = pack<false>(L, B, table, frag, s)) return rc;
+    if (int rc = pack<false, false>(L, B, table, frag, s)) return rc;
     auto k = P.n <= 16 ? k_bdm_apply<4, false, 1> : k_bdm_apply<kMaxP, false, 1>;
     const size_t lds = sizeof(float) * kSS * (L.din > L.dout ? L.din : L.dout);
     if (int rc = bdm_lds(reinterpret_cast<const void*>(k), lds)) return rc;
@@ -687,10 +726,10 @@ int bdm_bwd(const feq_layout& L, const feq_binning& B, int64_t E, const float* g
     build_pairs(L, true, P);
     build_units(L, U);
     float* frag = static_cast<float*>(ws);
-    float* gpart = frag + align_up(frag_floats(L, B), 64);
-    if (int rc = pack<true>(L, B, table, frag, s)) return rc;
+    float* gpart = frag + align_up(frag_floats(L, B, true), 64);
     // the distance gradient rides along where its sums fit the registers
     const bool gd = gdist && P.n <= 16;
+    if (int rc = gd ? pack<true, true>(L, B, table, frag, s) : pack<true, false>(L, B, table, frag, s)) return rc;
     auto k = gd ? k_bdm_apply<4, true, -1> : P.n <= 16 ? k_bdm_apply<4, false, -1> : k_bdm_apply<kMaxP, false, -1>;
     const size_t lds = sizeof(float) * kSS * (L.din > L.dout ? L.din : L.dout);
     if (int rc = bdm_lds(reinterpret_cast<const void*>(k), lds)) return rc;

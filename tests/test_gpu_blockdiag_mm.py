@@ -117,3 +117,26 @@ def test_errors_no_larger_than_the_per_edge_kernels(dev, lin, lout, cin, cout, n
     print(err)
     for name, a, c in zip(("y", "gx", "gT", "gr"), *err):
         assert a < c * (1.2 if name == "gr" else 1.05), (name, a, c)
+
+
+@pytest.mark.parametrize("lin,lout,c", [([0, 1, 2], [0, 1, 2], 32), ([0, 1, 2, 3, 4, 5, 6], [0, 1, 2, 3], 16)])
+def test_small_rows_beside_large_ones(dev, lin, lout, c):
+    """Rows of magnitude 2^-30 and 1 in turn, at distances on the lower edge of each bin (exact in
+    float32: t = 0): the small rows' results are as exact as the large ones', 32 c terms' float32
+    rounding, 1e-5 of each edge's largest entry.  A third of the way into a bin the two rows count."""
+    nb, E = 64, 3000
+    b = BD.Binning.linear(nb, 0.0, 8.0)
+    g = torch.Generator().manual_seed(21)
+    L = NAT.make_layout(lin, lout, c, c)
+    x, gy = torch.randn(E, c, L.din, generator=g), torch.randn(E, c, L.dout, generator=g)
+    T = torch.randn(nb + 1, c, c, L.wdim, generator=g)
+    T[::2] *= 2.0 ** -30
+    bins = torch.randint(1, nb, (E,), generator=g).float()
+    for part in (0.0, 0.375):
+        r = (bins + part) * 0.125
+        y, gx, _, _ = _raw(dev, lin, lout, b, nb, False, *(t.to(dev) for t in (x, T, r, gy)), True)
+        ey = BD.forward(x.double(), T.double(), r.double(), lin, lout, b)
+        ex = BD.backward(gy.double(), x.double(), T.double(), r.double(), lin, lout, b)[0]
+        for a, e in ((y, ey), (gx, ex)):
+            off = (a.cpu().double() - e).abs().amax((1, 2)) / e.abs().amax((1, 2))
+            assert off.max() < 1e-5, (part, off.max())

@@ -207,10 +207,10 @@ def test_wigner_dimension_limit(suffix, lvals):
 @pytest.mark.parametrize("lin,lout,cin,cout,bins,E,fwd,bwd", [
     ([0, 1, 2], [0, 1, 2], 32, 32, 64, 20000, True, True),
     ([0, 1, 2], [0, 1, 2], 32, 32, 64, 1000, False, False),          # too little work
-    ([0, 1, 2], [0, 1, 2], 32, 32, 1000, 1400, False, True),         # the forward's packing costs more than it gives
-    ([0, 1, 2], [0, 1, 2], 32, 32, 1000, 2000, True, True),
-    ([0, 1, 2], [0, 1, 2], 32, 32, 4096, 4096, False, True),
-    ([0, 1, 2], [0, 1, 2], 1, 1, 4096, 1400000, False, True),        # packed at 256 times its size
+    ([0, 1, 2], [0, 1, 2], 32, 32, 4096, 2000, False, True),         # the forward's packing costs more than it gives
+    ([0, 1, 2], [0, 1, 2], 32, 32, 4096, 4200, True, True),
+    ([0, 1, 2], [0, 1, 2], 1, 1, 4096, 1400000, True, True),
+    ([0, 1, 2], [0, 1, 2], 1, 1, 8000, 1400000, False, True),        # packed at 256 times its size
     (list(range(7)), list(range(7)), 32, 32, 100, 131, True, True),
     (list(range(7)), list(range(7)), 128, 128, 100, 7, True, True),  # few edges, 14 ms in a per-edge kernel
     (list(range(7)), list(range(7)), 128, 128, 150, 20000, False, False),   # 4.5 GB packed
@@ -225,9 +225,11 @@ def test_blockdiag_products_and_their_workspaces(lin, lout, cin, cout, bins, E, 
     up = lambda n: -(-n // 256) * 256
     sort = up(8 * E) + up(4 * E) + up(4 * (bins + 1)) + up(lib.feq_csr_workspace(E, bins)) + 256
     pad = lambda c: -(-c // 16) * 16
-    packed = 8 * bins * L.wdim * pad(cin) * pad(cout)
+    row = 4 * L.wdim * pad(cin) * pad(cout)
     assert lib.feq_blockdiag_workspace_f64(*args) == sort
-    assert lib.feq_blockdiag_fwd_workspace(*args) == (sort + packed if fwd else 0)
+    # the rows, and the differences at the first and last bin or, backward, everywhere
+    assert lib.feq_blockdiag_fwd_workspace(*args) == (sort + (bins + 3) * row if fwd else 0)
+    packed = (2 * bins + 1) * row
     most = sort + packed + 4 * pad(E) * pad(cin) // 16 + (256 << 20) + 1024
     assert sort + packed < lib.feq_blockdiag_workspace(*args) <= most if bwd else \
         lib.feq_blockdiag_workspace(*args) == sort
